@@ -958,20 +958,22 @@ int configure_bricks(rdy_engine *e, double lam, const int32_t *dims) {
     return RDY_OK;
 }
 
-// launches the bonded-term kernels on the current buffer
-void launch_bonded(rdy_engine *e) {
-    BondTerm *t;
-    uint32_t n;
-    Grid g = e->grid(e->cur);
-    if ((n = (uint32_t)e->terms_h[0].size()) && (t = e->d_terms[0]))
-        hipLaunchKernelGGL(k_bonds, dim3(blocks_for(n, 256)), dim3(256), 0, e->stream, g, e->reps, e->topo(), t, n,
-                           e->e_bonded);
-    if ((n = (uint32_t)e->terms_h[1].size()) && (t = e->d_terms[1]))
-        hipLaunchKernelGGL(k_angles, dim3(blocks_for(n, 256)), dim3(256), 0, e->stream, g, e->reps, e->topo(), t, n,
-                           e->e_bonded);
-    if ((n = (uint32_t)e->terms_h[2].size()) && (t = e->d_terms[2]))
-        hipLaunchKernelGGL(k_dihedrals, dim3(blocks_for(n, 256)), dim3(256), 0, e->stream, g, e->reps, e->topo(), t, n,
-                           e->e_bonded);
+// launches the bonded terms on the current buffer; energy: form the bonded energies too (a fused step needs
+// the forces only)
+void launch_bonded(rdy_engine *e, bool energy) {
+    const BondTerm *t[3];
+    uint32_t n[3], nb[3];
+    for (int k = 0; k < 3; ++k) {
+        t[k] = e->d_terms[k];
+        n[k] = t[k] ? (uint32_t)e->terms_h[k].size() : 0u;
+        nb[k] = (n[k] + BONDED_THREADS - 1) / BONDED_THREADS;
+    }
+    const uint32_t blocks = nb[0] + nb[1] + nb[2];
+    if (blocks == 0) return;
+    const auto kernel = energy ? k_bonded<true> : k_bonded<false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(BONDED_THREADS), 0, e->stream, e->grid(e->cur),
+                       (const ReplicaDev *)e->reps, e->topo(), t[0], n[0], t[1], n[1], t[2], n[2], nb[0], nb[1],
+                       e->e_bonded);
 }
 
 uint32_t wl_blocks(const rdy_engine *e) { return blocks_for(e->max_particles, e->block); }
@@ -1033,7 +1035,7 @@ void launch_walk(rdy_engine *e, int prologue, int handler, double dt, bool slow_
 
 // the first walk of a run: the forces of the current state and step 1's move (bonded terms first)
 void launch_prologue(rdy_engine *e, double dt) {
-    launch_bonded(e);
+    launch_bonded(e, false);
     launch_walk(e, 1, (int)RDY_HANDLER_NONE, dt);
     e->wl_valid[1 - e->cur] = false;
     e->cur = 1 - e->cur;
@@ -1060,7 +1062,7 @@ void launch_step(rdy_engine *e, int handler, double dt, int last) {
     hipLaunchKernelGGL(k_step_begin, dim3(blocks_for(nthreads, 256)), dim3(256), 0, e->stream, e->reps, nr, last,
                        e->grid(n), (uint32_t)nc, e->fb, (uint32_t)nfb, e->edit_count, e->e_bonded,
                        (const uint32_t *)e->loc, e->loc_cur, (uint32_t)nloc);
-    launch_bonded(e);
+    launch_bonded(e, false);
     const int h = (handler != RDY_HANDLER_NONE && e->n_rx > 0) ? handler : RDY_HANDLER_NONE;
     launch_walk(e, 0, h, dt, h != RDY_HANDLER_NONE);
     const bool topo_rx = topo_reactions_on(e);
@@ -1093,7 +1095,7 @@ void launch_forces(rdy_engine *e, double *force_out) {
     unsigned long long *vir = e->record_virial ? e->virial : nullptr;
     hipLaunchKernelGGL(k_advance, dim3(blocks_for(nr, 64)), dim3(64), 0, e->stream, e->reps, nr, 0, e->e_bonded,
                        (uint32_t *)nullptr, vir);
-    launch_bonded(e);
+    launch_bonded(e, true);
     const int c = e->cur;
     for_brick_groups(e, [&](auto ah, uint32_t nb, uint32_t b0) {
         hipLaunchKernelGGL((k_brick<MODE_FORCES, decltype(ah)::value>), dim3(nb), dim3(BRICK_THREADS), e->brick_smem,

@@ -393,6 +393,8 @@ __global__ __launch_bounds__(256) void k_integrate(Grid cur, ReplicaDev *reps, T
 // bonded terms (CPUTopologyActions.cpp:55-123): FP64, fixed-point atomics into the per-particle
 // bonded force; energies into e_bonded[replica] (fixed point 2^-24)
 // -------------------------------------------------------------------------------------------------
+constexpr uint32_t BONDED_THREADS = 256;
+
 struct BondTerm {
     uint32_t r, h[4];
     uint32_t mult;
@@ -428,13 +430,11 @@ __device__ __forceinline__ void add_fb(const Topo &topo, const ReplicaDev &R, ui
     for (int d = 0; d < 3; ++d) atomicAdd((unsigned long long *)&fb[d], (unsigned long long)to_fixed_d(f[d], FORCE_SCALE));
 }
 
-__global__ void k_bonds(Grid cur, ReplicaDev *reps, Topo topo, const BondTerm *terms, uint32_t n,
-                        unsigned long long *e_bonded) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const BondTerm t = terms[i];
-    const ReplicaDev &R = reps[t.r];
-    if (!R.in_use || t.k == 0) return;
+// One term of each kind adds its forces to the bonded force accumulators and returns its energy
+// (ENERGY false: zero, and what only the energy needs is not formed).
+template <bool ENERGY>
+__device__ __forceinline__ long long bond_term(const Grid &cur, const ReplicaDev &R, const Topo &topo,
+                                               const BondTerm &t) {
     double a[3], b[3], x[3];
     pos_of(cur, topo, R, t.h[0], a);
     pos_of(cur, topo, R, t.h[1], b);
@@ -444,8 +444,185 @@ __global__ void k_bonds(Grid cur, ReplicaDev *reps, Topo topo, const BondTerm *t
     double fi[3] = {c * x[0], c * x[1], c * x[2]}, fj[3] = {-fi[0], -fi[1], -fi[2]};
     add_fb(topo, R, t.h[0], fi);
     add_fb(topo, R, t.h[1], fj);
-    double e = t.k * (norm - t.p0) * (norm - t.p0);
-    atomicAdd(&e_bonded[t.r], (unsigned long long)to_fixed_d(e, ENERGY_SCALE));
+    return ENERGY ? to_fixed_d(t.k * (norm - t.p0) * (norm - t.p0), ENERGY_SCALE) : 0;
+}
+
+template <bool ENERGY>
+__device__ __forceinline__ long long angle_term(const Grid &cur, const ReplicaDev &R, const Topo &topo,
+                                                const BondTerm &t) {
+    const double SMALL = 1e-10;  // AnglePotential.cpp:49
+    double pi_[3], pj[3], pk[3], xji[3], xjk[3];
+    pos_of(cur, topo, R, t.h[0], pi_);
+    pos_of(cur, topo, R, t.h[1], pj);
+    pos_of(cur, topo, R, t.h[2], pk);
+    sdiff(pj, pi_, R, xji);
+    sdiff(pj, pk, R, xjk);
+    double sp = dot(xji, xjk);
+    double nji2 = dot(xji, xji);
+    if (nji2 < SMALL) nji2 = SMALL;
+    double njk2 = dot(xjk, xjk);
+    if (njk2 < SMALL) njk2 = SMALL;
+    double nprod = sqrt(nji2) * sqrt(njk2);
+    if (nprod < SMALL) nprod = SMALL;
+    double inv = 1. / nprod;
+    double ct = fmin(fmax(inv * sp, -1.), 1.);
+    double si = sqrt(1. - ct * ct);
+    if (si < SMALL) si = SMALL;
+    si = 1. / si;
+    double c = 2. * t.k * (acos(ct) - t.p0) * si;
+    double f_i[3], f_j[3], f_k[3];
+    for (int d = 0; d < 3; ++d) {
+        double force_i = c * ct * (1. / nji2) * xji[d] - c * inv * xjk[d];
+        double force_k = -c * inv * xji[d] + c * ct * (1. / njk2) * xjk[d];
+        f_i[d] = -force_i;
+        f_j[d] = force_i + force_k;
+        f_k[d] = -force_k;
+    }
+    add_fb(topo, R, t.h[0], f_i);
+    add_fb(topo, R, t.h[1], f_j);
+    add_fb(topo, R, t.h[2], f_k);
+    if constexpr (!ENERGY) return 0;
+    const double dth = acos(sp / (sqrt(dot(xji, xji)) * sqrt(dot(xjk, xjk)))) - t.p0;
+    return to_fixed_d(t.k * dth * dth, ENERGY_SCALE);
+}
+
+// cosine dihedral: energy as TorsionPotential.cpp:53-70; force = analytic gradient of the same
+// angle (closed form of the IUPAC dihedral gradient, phi_ref = -psi - pi), zero when |cos phi| < 1e-4
+template <bool ENERGY>
+__device__ __forceinline__ long long dihedral_term(const Grid &cur, const ReplicaDev &R, const Topo &topo,
+                                                   const BondTerm &t) {
+    const double SMALL = 1e-4;
+    double pi_[3], pj[3], pk[3], pl[3], xji[3], xkj[3], xkl[3], xjk[3];
+    pos_of(cur, topo, R, t.h[0], pi_);
+    pos_of(cur, topo, R, t.h[1], pj);
+    pos_of(cur, topo, R, t.h[2], pk);
+    pos_of(cur, topo, R, t.h[3], pl);
+    sdiff(pj, pi_, R, xji);
+    sdiff(pk, pj, R, xkj);
+    sdiff(pk, pl, R, xkl);
+    for (int d = 0; d < 3; ++d) xjk[d] = -1. * xkj[d];
+    double m[3], nn[3], mxn[3];
+    cross(xji, xkj, m);
+    cross(xkl, xjk, nn);
+    cross(m, nn, mxn);
+    double jkn = sqrt(dot(xjk, xjk));
+    if (jkn < SMALL) jkn = SMALL;
+    double mnn = sqrt(dot(m, m)) * sqrt(dot(nn, nn));
+    if (mnn < SMALL) mnn = SMALL;
+    long long e = 0;
+    if constexpr (ENERGY) {
+        double phi_e = -atan2(dot(mxn, xjk) / (mnn * jkn), dot(m, nn) / mnn);
+        e = to_fixed_d(t.k * (1 + cos((double)t.mult * phi_e - t.p0)), ENERGY_SCALE);
+    }
+
+    double x2 = dot(xjk, xjk);
+    if (x2 < SMALL) x2 = SMALL;
+    double m2 = dot(m, m);
+    if (m2 < SMALL) m2 = SMALL;
+    double n2 = dot(nn, nn);
+    if (n2 < SMALL) n2 = SMALL;
+    double mn = sqrt(m2) * sqrt(n2);
+    if (mn < SMALL) mn = SMALL;
+    double cos_phi = dot(nn, m) / mn;
+    if (fabs(cos_phi) < SMALL) return e;
+    double sin_phi = dot(mxn, xjk) / (mn * sqrt(x2));
+    double phi = -atan2(sin_phi, cos_phi);
+    double dV = -t.k * (double)t.mult * sin((double)t.mult * phi - t.p0);
+    double b1[3], b2[3], b3[3], A[3], B[3];
+    for (int d = 0; d < 3; ++d) {
+        b1[d] = -xji[d];
+        b2[d] = xjk[d];
+        b3[d] = xkl[d];
+    }
+    cross(b1, b2, A);
+    cross(b2, b3, B);
+    double A2 = dot(A, A), B2 = dot(B, B);
+    if (A2 < SMALL) A2 = SMALL;
+    if (B2 < SMALL) B2 = SMALL;
+    double b2n = sqrt(x2);
+    double p12 = dot(b1, b2) / x2, p32 = dot(b3, b2) / x2;
+    double fi[3], fj[3], fk[3], fl[3];
+    for (int d = 0; d < 3; ++d) {
+        double gi = -b2n * A[d] / A2, gl = b2n * B[d] / B2;
+        fi[d] = dV * gi;
+        fj[d] = dV * (-(1.0 + p12) * gi + p32 * gl);
+        fk[d] = dV * (p12 * gi - (1.0 + p32) * gl);
+        fl[d] = dV * gl;
+    }
+    add_fb(topo, R, t.h[0], fi);
+    add_fb(topo, R, t.h[1], fj);
+    add_fb(topo, R, t.h[2], fk);
+    add_fb(topo, R, t.h[3], fl);
+    return e;
+}
+
+// block-wide sums of the bonded energies, one atomic per run of waves of one replica (the terms are listed
+// replica after replica, so a wave that holds two replicas' terms is rare and adds lane by lane)
+__device__ __forceinline__ void block_add_bonded(unsigned long long *e_bonded, bool valid, uint32_t r, long long e) {
+    __shared__ long long s_e[BONDED_THREADS / 64];
+    __shared__ uint32_t s_r[BONDED_THREADS / 64];
+    const unsigned long long vm = __ballot(valid);
+    const uint32_t w = threadIdx.x / 64, lead = vm ? (uint32_t)__ffsll((long long)vm) - 1u : 0u;
+    const uint32_t r0 = __shfl(r, (int)lead);
+    long long v = valid ? e : 0;
+    if (!__all(!valid || r == r0)) {
+        if (valid && v != 0) atomicAdd(&e_bonded[r], (unsigned long long)v);
+        v = 0;
+    }
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if (__lane_id() == 0) {
+        s_e[w] = v;
+        s_r[w] = r0;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        long long run = s_e[0];
+        for (uint32_t k = 1; k <= BONDED_THREADS / 64; ++k) {
+            if (k < BONDED_THREADS / 64 && s_r[k] == s_r[k - 1]) {
+                run += s_e[k];
+                continue;
+            }
+            if (run != 0) atomicAdd(&e_bonded[s_r[k - 1]], (unsigned long long)run);
+            if (k < BONDED_THREADS / 64) run = s_e[k];
+        }
+    }
+}
+
+// All bonded terms in one launch: the first nb0 blocks take the bonds, the next nb1 the angles, the rest the
+// dihedrals (a block holds one kind, so its waves do not diverge).  With ENERGY the terms' energies go to
+// e_bonded through one atomic per block: an atomic per term on the replica's one word serialised the terms, and
+// the three kinds took 1.18 + 1.16 + 1.14 ms at 100,000 beads in chains of 50 (82 us at 2,000 beads).  The fused
+// step reads no energies (an export evaluates the forces again), so its launches form none: 50 us at 100,000
+// beads, 6.4 us at 2,000.  What is left there is the 64-bit force atomics, 27 a bead, and the FP64 angles.
+template <bool ENERGY>
+__global__ __launch_bounds__(BONDED_THREADS) void k_bonded(Grid cur, const ReplicaDev *reps, Topo topo,
+                                                           const BondTerm *bonds, uint32_t n_bonds,
+                                                           const BondTerm *angles, uint32_t n_angles,
+                                                           const BondTerm *dihedrals, uint32_t n_dihedrals,
+                                                           uint32_t nb0, uint32_t nb1, unsigned long long *e_bonded) {
+    uint32_t b = blockIdx.x, kind = 0, n = n_bonds;
+    const BondTerm *terms = bonds;
+    if (b >= nb0 + nb1) {
+        b -= nb0 + nb1, kind = 2, n = n_dihedrals, terms = dihedrals;
+    } else if (b >= nb0) {
+        b -= nb0, kind = 1, n = n_angles, terms = angles;
+    }
+    const uint32_t i = b * BONDED_THREADS + threadIdx.x;
+    long long e = 0;
+    uint32_t r = 0;
+    bool valid = i < n;
+    if (valid) {
+        const BondTerm t = terms[i];
+        r = t.r;
+        const ReplicaDev &R = reps[r];
+        valid = R.in_use && !(kind == 0 && t.k == 0);
+        if (valid) {
+            if (kind == 0) e = bond_term<ENERGY>(cur, R, topo, t);
+            else if (kind == 1) e = angle_term<ENERGY>(cur, R, topo, t);
+            else e = dihedral_term<ENERGY>(cur, R, topo, t);
+        }
+    }
+    if constexpr (ENERGY) block_add_bonded(e_bonded, valid, r, e);
 }
 
 // BreakBonds (Actions.h:235-290): one thread per bond term.  The first term of each run of terms on
@@ -488,120 +665,6 @@ __global__ void k_break_bonds(Grid cur, const ReplicaDev *reps, Topo topo, const
         out[3ull * p + 1] = t.h[0];
         out[3ull * p + 2] = t.h[1];
     }
-}
-
-__global__ void k_angles(Grid cur, ReplicaDev *reps, Topo topo, const BondTerm *terms, uint32_t n,
-                         unsigned long long *e_bonded) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const BondTerm t = terms[i];
-    const ReplicaDev &R = reps[t.r];
-    if (!R.in_use) return;
-    const double SMALL = 1e-10;  // AnglePotential.cpp:49
-    double pi_[3], pj[3], pk[3], xji[3], xjk[3];
-    pos_of(cur, topo, R, t.h[0], pi_);
-    pos_of(cur, topo, R, t.h[1], pj);
-    pos_of(cur, topo, R, t.h[2], pk);
-    sdiff(pj, pi_, R, xji);
-    sdiff(pj, pk, R, xjk);
-    double sp = dot(xji, xjk);
-    double e = t.k * (acos(sp / (sqrt(dot(xji, xji)) * sqrt(dot(xjk, xjk)))) - t.p0) *
-               (acos(sp / (sqrt(dot(xji, xji)) * sqrt(dot(xjk, xjk)))) - t.p0);
-    double nji2 = dot(xji, xji);
-    if (nji2 < SMALL) nji2 = SMALL;
-    double njk2 = dot(xjk, xjk);
-    if (njk2 < SMALL) njk2 = SMALL;
-    double nprod = sqrt(nji2) * sqrt(njk2);
-    if (nprod < SMALL) nprod = SMALL;
-    double inv = 1. / nprod;
-    double ct = fmin(fmax(inv * sp, -1.), 1.);
-    double si = sqrt(1. - ct * ct);
-    if (si < SMALL) si = SMALL;
-    si = 1. / si;
-    double c = 2. * t.k * (acos(ct) - t.p0) * si;
-    double f_i[3], f_j[3], f_k[3];
-    for (int d = 0; d < 3; ++d) {
-        double force_i = c * ct * (1. / nji2) * xji[d] - c * inv * xjk[d];
-        double force_k = -c * inv * xji[d] + c * ct * (1. / njk2) * xjk[d];
-        f_i[d] = -force_i;
-        f_j[d] = force_i + force_k;
-        f_k[d] = -force_k;
-    }
-    add_fb(topo, R, t.h[0], f_i);
-    add_fb(topo, R, t.h[1], f_j);
-    add_fb(topo, R, t.h[2], f_k);
-    atomicAdd(&e_bonded[t.r], (unsigned long long)to_fixed_d(e, ENERGY_SCALE));
-}
-
-// cosine dihedral: energy as TorsionPotential.cpp:53-70; force = analytic gradient of the same
-// angle (closed form of the IUPAC dihedral gradient, phi_ref = -psi - pi), zero when |cos phi| < 1e-4
-__global__ void k_dihedrals(Grid cur, ReplicaDev *reps, Topo topo, const BondTerm *terms, uint32_t n,
-                            unsigned long long *e_bonded) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const BondTerm t = terms[i];
-    const ReplicaDev &R = reps[t.r];
-    if (!R.in_use) return;
-    const double SMALL = 1e-4;
-    double pi_[3], pj[3], pk[3], pl[3], xji[3], xkj[3], xkl[3], xjk[3];
-    pos_of(cur, topo, R, t.h[0], pi_);
-    pos_of(cur, topo, R, t.h[1], pj);
-    pos_of(cur, topo, R, t.h[2], pk);
-    pos_of(cur, topo, R, t.h[3], pl);
-    sdiff(pj, pi_, R, xji);
-    sdiff(pk, pj, R, xkj);
-    sdiff(pk, pl, R, xkl);
-    for (int d = 0; d < 3; ++d) xjk[d] = -1. * xkj[d];
-    double m[3], nn[3], mxn[3];
-    cross(xji, xkj, m);
-    cross(xkl, xjk, nn);
-    cross(m, nn, mxn);
-    double jkn = sqrt(dot(xjk, xjk));
-    if (jkn < SMALL) jkn = SMALL;
-    double mnn = sqrt(dot(m, m)) * sqrt(dot(nn, nn));
-    if (mnn < SMALL) mnn = SMALL;
-    double phi_e = -atan2(dot(mxn, xjk) / (mnn * jkn), dot(m, nn) / mnn);
-    double e = t.k * (1 + cos((double)t.mult * phi_e - t.p0));
-    atomicAdd(&e_bonded[t.r], (unsigned long long)to_fixed_d(e, ENERGY_SCALE));
-
-    double x2 = dot(xjk, xjk);
-    if (x2 < SMALL) x2 = SMALL;
-    double m2 = dot(m, m);
-    if (m2 < SMALL) m2 = SMALL;
-    double n2 = dot(nn, nn);
-    if (n2 < SMALL) n2 = SMALL;
-    double mn = sqrt(m2) * sqrt(n2);
-    if (mn < SMALL) mn = SMALL;
-    double cos_phi = dot(nn, m) / mn;
-    if (fabs(cos_phi) < SMALL) return;
-    double sin_phi = dot(mxn, xjk) / (mn * sqrt(x2));
-    double phi = -atan2(sin_phi, cos_phi);
-    double dV = -t.k * (double)t.mult * sin((double)t.mult * phi - t.p0);
-    double b1[3], b2[3], b3[3], A[3], B[3];
-    for (int d = 0; d < 3; ++d) {
-        b1[d] = -xji[d];
-        b2[d] = xjk[d];
-        b3[d] = xkl[d];
-    }
-    cross(b1, b2, A);
-    cross(b2, b3, B);
-    double A2 = dot(A, A), B2 = dot(B, B);
-    if (A2 < SMALL) A2 = SMALL;
-    if (B2 < SMALL) B2 = SMALL;
-    double b2n = sqrt(x2);
-    double p12 = dot(b1, b2) / x2, p32 = dot(b3, b2) / x2;
-    double fi[3], fj[3], fk[3], fl[3];
-    for (int d = 0; d < 3; ++d) {
-        double gi = -b2n * A[d] / A2, gl = b2n * B[d] / B2;
-        fi[d] = dV * gi;
-        fj[d] = dV * (-(1.0 + p12) * gi + p32 * gl);
-        fk[d] = dV * (p12 * gi - (1.0 + p32) * gl);
-        fl[d] = dV * gl;
-    }
-    add_fb(topo, R, t.h[0], fi);
-    add_fb(topo, R, t.h[1], fj);
-    add_fb(topo, R, t.h[2], fk);
-    add_fb(topo, R, t.h[3], fl);
 }
 
 // -------------------------------------------------------------------------------------------------
