@@ -2201,9 +2201,9 @@ int rdy_count_types(rdy_engine *e, uint64_t *counts, uint32_t n_reps) {
     if (rc) return rc;
     unsigned long long *d = (unsigned long long *)e->scratch;
     HIP_TRY(hipMemsetAsync(d, 0, words * 8, e->stream));
-    ensure_wl(e);
-    hipLaunchKernelGGL(k_count_types, dim3(wl_blocks(e)), dim3(e->block), 0, e->stream, e->grid(e->cur), e->n_types, d,
-                       n_reps, (uint32_t)e->max_particles);
+    const uint32_t nc = (uint32_t)std::max<uint64_t>(e->cells_hwm, 1);
+    hipLaunchKernelGGL(k_count_types, dim3(blocks_for(nc, COUNT_CELLS)), dim3(256), 0, e->stream, e->grid(e->cur), e->cap,
+                       nc, e->n_types, d, n_reps);
     HIP_TRY(hipMemcpyAsync(counts, d, words * 8, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     return RDY_OK;
