@@ -171,6 +171,10 @@ class Engine:
         pos = np.ascontiguousarray(pos, dtype=np.float64).reshape(-1, 3)
         types = np.ascontiguousarray(types, dtype=np.uint32)
         assert len(pos) == len(types)
+        # handles the replica's topology particles can take: the upload's, then the reserve
+        flavored = int((self._flavor[types[types < self.n_types]] != 0).sum()) if self._flavor is not None else 0
+        self._topo_handles = getattr(self, "_topo_handles", {})
+        self._topo_handles[r] = flavored + getattr(self, "_topo_reserve", {}).get(r, 0)
         L.check(self._lib.rdy_set_particles(self._h, r, len(types), _ptr(pos, _dp), _ptr(types, _u32p)))
 
     def n_particles(self, r=0):
@@ -328,6 +332,10 @@ class Engine:
         """topology_types[k]: type of topology k; topology_of[h]: topology of topology particle h"""
         tt = np.ascontiguousarray(topology_types, dtype=np.uint32)
         to = np.ascontiguousarray(topology_of, dtype=np.uint32)
+        # the engine reads one entry per topology particle: a list too short ends in an index that it refuses
+        missing = getattr(self, "_topo_handles", {}).get(r, 0) - len(to)
+        if missing > 0:
+            to = np.concatenate([to, np.full(missing, 0xFFFFFFFE, dtype=np.uint32)])
         L.check(self._lib.rdy_set_topologies(self._h, r, len(tt), _ptr(tt, _u32p), _ptr(to, _u32p)))
 
     def topology_types(self, r=0):
@@ -340,6 +348,8 @@ class Engine:
     def reserve_topology_particles(self, r, n):
         """handles for particles that join topologies by fusion; takes effect with the next set_particles"""
         L.check(self._lib.rdy_reserve_topology_particles(self._h, r, int(n)))
+        self._topo_reserve = getattr(self, "_topo_reserve", {})
+        self._topo_reserve[r] = int(n)
 
     def topology_fusions(self, r=0):
         """rows (topology, topology particle handle, joining particle's old handle, its new handle) of the last
