@@ -125,7 +125,7 @@ int rdy_replica_footprint(const rdy_engine *e, const rdy_replica_desc *desc, uin
  * get fresh handles from the replica's counter (Particle::nextId, Particle.h:112-114). */
 int rdy_set_particles(rdy_engine *e, uint32_t replica, uint64_t n, const double *pos, const uint32_t *types);
 uint64_t rdy_particle_count(rdy_engine *e, uint32_t replica);
-/* copies up to cap live particles (order unspecified); returns the count via *n */
+/* copies the first cap live particles in ascending handle order; returns their number via *n */
 int rdy_get_particles(rdy_engine *e, uint32_t replica, uint64_t cap, double *pos, uint32_t *types,
                       uint32_t *handles, uint64_t *n);
 /* forces of the last force evaluation, aligned with rdy_get_particles' order of the same state */

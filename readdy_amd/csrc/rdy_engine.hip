@@ -32,6 +32,9 @@ int set_err(int code, const std::string &msg) {
         if (e_ != hipSuccess) return set_err(RDY_ERR_HIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+constexpr size_t STAGING_SMALL = 256u << 10;  // pinned bytes a small readback uses
+constexpr size_t STAGING_HALF = 4u << 20;     // one half of the pinned area a large one streams through
+
 struct HostReplica {
     bool in_use = false;
     uint64_t cell_base = 0, n_cells = 0;
@@ -40,6 +43,7 @@ struct HostReplica {
     uint32_t topo_reserve = 0;  // handles reserved for topology-particle fusions (rdy_reserve_topology_particles)
     uint32_t tt_base = 0, n_tt = 0;  // topologies (their types) for spatial topology reactions
     bool has_particles = false;  // particles were uploaded since the replica was added
+    uint64_t handle_guess = 0;   // handles a readback makes room for (the last one read and some growth)
     ReplicaDev dev{};
 };
 
@@ -208,6 +212,9 @@ struct rdy_engine {
     // scratch
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    char *staging = nullptr;  // pinned (gather, copy_out)
+    size_t staging_bytes = 0;
+    hipEvent_t staging_ev[2] = {nullptr, nullptr};
     double *d_noise = nullptr;
     size_t noise_cap = 0;
     int cur = 0;
@@ -1265,6 +1272,9 @@ int rdy_engine_destroy(rdy_engine *e) {
         (void)hipEventDestroy(pe.first);
         (void)hipEventDestroy(pe.second);
     }
+    if (e->staging) (void)hipHostFree(e->staging);
+    for (hipEvent_t ev : e->staging_ev)
+        if (ev) (void)hipEventDestroy(ev);
     (void)hipStreamDestroy(e->stream);
     delete e;
     return RDY_OK;
@@ -1481,6 +1491,7 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
                            (uint32_t)n, n_topo, spare, dpos, dty, (const uint8_t *)e->d_flavor, e->topo(), e->cap,
                            (uint32_t)e->max_particles, e->err);
     }
+    H.handle_guess = hn + (uint64_t)hn / 2 + 4096;
     e->wl_valid[e->cur] = false;
     e->version++;
     return check_errors(e);
@@ -1492,36 +1503,127 @@ uint64_t rdy_particle_count(rdy_engine *e, uint32_t r) {
     return n;
 }
 
+// the engine's pinned staging area, grown to `bytes` (no copy is in flight between calls)
+static int ensure_staging(rdy_engine *e, size_t bytes) {
+    if (bytes <= e->staging_bytes) return RDY_OK;
+    if (e->staging) HIP_TRY(hipHostFree(e->staging));
+    e->staging = nullptr;
+    e->staging_bytes = 0;
+    HIP_TRY(hipHostMalloc((void **)&e->staging, bytes, hipHostMallocDefault));
+    e->staging_bytes = bytes;
+    return RDY_OK;
+}
+
+// Device arrays to host memory through the pinned staging area, in chunks: while one half is on its way from
+// the device, the other is copied out (a copy straight into pageable memory is staged page by page).
+struct HostCopy {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+
+static int copy_out(rdy_engine *e, const HostCopy (&c)[4]) {
+    if (int rc = ensure_staging(e, 2 * STAGING_HALF)) return rc;
+    for (hipEvent_t &ev : e->staging_ev)
+        if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    HostCopy flying[2][4];  // pieces of each half on their way (an array never has two pieces in one half)
+    int n_flying[2] = {0, 0}, half = 0;
+    auto drain = [&](int h) -> int {
+        if (n_flying[h] == 0) return RDY_OK;
+        HIP_TRY(hipEventSynchronize(e->staging_ev[h]));
+        for (int q = 0; q < n_flying[h]; ++q) std::memcpy(flying[h][q].dst, flying[h][q].src, flying[h][q].bytes);
+        n_flying[h] = 0;
+        return RDY_OK;
+    };
+    size_t k = 0, off = 0;
+    while (k < 4) {
+        char *base = e->staging + (size_t)half * STAGING_HALF;
+        size_t used = 0;
+        while (k < 4 && used < STAGING_HALF) {
+            const size_t m = std::min(c[k].bytes - off, STAGING_HALF - used);
+            if (m) {
+                HIP_TRY(hipMemcpyAsync(base + used, (const char *)c[k].src + off, m, hipMemcpyDeviceToHost, e->stream));
+                flying[half][n_flying[half]++] = {(char *)c[k].dst + off, base + used, m};
+            }
+            used += m;
+            off += m;
+            if (off == c[k].bytes) {
+                ++k;
+                off = 0;
+            }
+        }
+        HIP_TRY(hipEventRecord(e->staging_ev[half], e->stream));
+        half ^= 1;
+        if (int rc = drain(half)) return rc;  // the half to be filled next
+    }
+    if (int rc = drain(half)) return rc;
+    return drain(half ^ 1);
+}
+
+// the live particles of replica r in ascending handle order (cap 0: their number only)
 static int gather(rdy_engine *e, uint32_t r, uint64_t cap, double *pos, uint32_t *types, uint32_t *handles,
                   double *forces, uint64_t *n) {
     int rc = check_replica(e, r);
     if (rc) return rc;
-    const uint64_t ncap = e->max_particles;
-    size_t bytes = 64 + ncap * (6 * sizeof(double) + 2 * sizeof(uint32_t));
-    if ((rc = ensure_scratch(e, bytes))) return rc;
-    uint32_t *cnt = (uint32_t *)e->scratch;
-    double *dpos = (double *)((char *)e->scratch + 64);
-    double *dfor = dpos + 3 * ncap;
-    uint32_t *dty = (uint32_t *)(dfor + 3 * ncap);
-    uint32_t *dh = dty + ncap;
-    HIP_TRY(hipMemsetAsync(cnt, 0, 4, e->stream));
-    ensure_wl(e);
-    hipLaunchKernelGGL(k_gather, dim3(wl_blocks(e)), dim3(e->block), 0, e->stream, e->grid(e->cur), r, cnt,
-                       (uint32_t)ncap, dpos, dty, dh, (const double *)e->force_out, forces ? dfor : (double *)nullptr,
-                       (uint32_t)e->max_particles);
-    uint32_t hc = 0;
-    HIP_TRY(hipMemcpyAsync(&hc, cnt, 4, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    *n = hc;
-    uint64_t m = std::min<uint64_t>(hc, cap);
-    if (m) {
-        if (pos) HIP_TRY(hipMemcpyAsync(pos, dpos, m * 3 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        if (forces) HIP_TRY(hipMemcpyAsync(forces, dfor, m * 3 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        if (types) HIP_TRY(hipMemcpyAsync(types, dty, m * sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
-        if (handles) HIP_TRY(hipMemcpyAsync(handles, dh, m * sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
+    HostReplica &H = e->reps_h[r];
+    const uint64_t ncap = std::min<uint64_t>(cap, e->max_particles);
+    const Grid g = e->grid(e->cur);
+    const uint32_t blocks = blocks_for(H.n_cells, 256);
+    for (int attempt = 0;; ++attempt) {
+        // the bitmap covers the handles of the last read and half as many again; a replica that has grown
+        // past it says how many it has, and the readback is repeated
+        const uint64_t hmax = std::min<uint64_t>(H.handle_guess, 1ull << 32), per = 32ull * RANK_GROUP_WORDS;
+        const uint32_t groups = ncap ? (uint32_t)((hmax + per - 1) / per) : 0u;
+        const uint32_t tiles = (groups + RANK_TILE - 1) / RANK_TILE, words = groups * RANK_GROUP_WORDS;
+        const size_t off_sum = 4ull * groups, off_bits = (off_sum + 4ull * tiles + 63) & ~(size_t)63;
+        const size_t off_info = off_bits + 4ull * words, off_pos = off_info + 64;
+        const size_t off_for = off_pos + (pos ? 24 * ncap : 0), off_ty = off_for + (forces ? 24 * ncap : 0);
+        const size_t off_h = off_ty + (types ? 4 * ncap : 0), end = off_h + (handles ? 4 * ncap : 0);
+        if ((rc = ensure_scratch(e, end))) return rc;
+        char *base = (char *)e->scratch;
+        uint32_t *pre = (uint32_t *)base, *sums = (uint32_t *)(base + off_sum), *bits = (uint32_t *)(base + off_bits);
+        HIP_TRY(hipMemsetAsync(base + off_bits, 0, off_pos - off_bits, e->stream));
+        hipLaunchKernelGGL(k_rank_mark, dim3(blocks), dim3(256), 0, e->stream, g, (const ReplicaDev *)e->reps, r, e->cap,
+                           (uint32_t)H.cell_base, (uint32_t)H.n_cells, bits, words, (RankInfo *)(base + off_info));
+        if (ncap) {
+            if (tiles > 1)
+                hipLaunchKernelGGL(k_rank_sums, dim3(tiles), dim3(SCAN_THREADS), 0, e->stream, (const uint32_t *)bits,
+                                   groups, sums);
+            hipLaunchKernelGGL(k_rank_prefix, dim3(tiles), dim3(SCAN_THREADS), 0, e->stream, (const uint32_t *)bits,
+                               groups, (const uint32_t *)sums, pre);
+            hipLaunchKernelGGL(k_rank_write, dim3(blocks), dim3(256), 0, e->stream, g, r, e->cap, (uint32_t)H.cell_base,
+                               (uint32_t)H.n_cells, (const uint32_t *)bits, words, (const uint32_t *)pre, (uint32_t)ncap,
+                               pos ? (double *)(base + off_pos) : nullptr, types ? (uint32_t *)(base + off_ty) : nullptr,
+                               handles ? (uint32_t *)(base + off_h) : nullptr, (const double *)e->force_out,
+                               forces ? (double *)(base + off_for) : nullptr);
+        }
+        // a small answer comes back whole with the count, in one copy and one wait
+        const bool small = end - off_info <= STAGING_SMALL;
+        const size_t first = small ? end - off_info : sizeof(RankInfo);
+        if ((rc = ensure_staging(e, STAGING_SMALL))) return rc;
+        HIP_TRY(hipMemcpyAsync(e->staging, base + off_info, first, hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
+        RankInfo info;
+        std::memcpy(&info, e->staging, sizeof info);
+        H.handle_guess = info.handle_next + (uint64_t)info.handle_next / 2 + 4096;
+        if (info.beyond && attempt == 0) continue;
+        *n = info.live;
+        const uint64_t m = std::min<uint64_t>(info.live, ncap);
+        if (m == 0) return RDY_OK;
+        if (small) {
+            const char *w = e->staging;
+            if (pos) std::memcpy(pos, w + (off_pos - off_info), 24 * m);
+            if (forces) std::memcpy(forces, w + (off_for - off_info), 24 * m);
+            if (types) std::memcpy(types, w + (off_ty - off_info), 4 * m);
+            if (handles) std::memcpy(handles, w + (off_h - off_info), 4 * m);
+            return RDY_OK;
+        }
+        const HostCopy all[4] = {{pos, base + off_pos, pos ? 24 * m : 0},
+                                 {forces, base + off_for, forces ? 24 * m : 0},
+                                 {types, base + off_ty, types ? 4 * m : 0},
+                                 {handles, base + off_h, handles ? 4 * m : 0}};
+        return copy_out(e, all);
     }
-    return RDY_OK;
 }
 
 int rdy_get_particles(rdy_engine *e, uint32_t r, uint64_t cap, double *pos, uint32_t *types, uint32_t *handles,

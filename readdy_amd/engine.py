@@ -185,24 +185,22 @@ class Engine:
     def get_particles(self, r=0):
         """(positions, types, handles) of live particles, sorted by handle."""
         n = self.n_particles(r)
-        pos = np.zeros((n, 3))
-        types = np.zeros(n, dtype=np.uint32)
-        hs = np.zeros(n, dtype=np.uint32)
+        pos = np.empty((n, 3))
+        types = np.empty(n, dtype=np.uint32)
+        hs = np.empty(n, dtype=np.uint32)
         m = ctypes.c_uint64()
         L.check(self._lib.rdy_get_particles(self._h, r, n, _ptr(pos, _dp), _ptr(types, _u32p), _ptr(hs, _u32p),
                                             ctypes.byref(m)))
-        o = np.argsort(hs, kind="stable")
-        return pos[o], types[o], hs[o]
+        return pos, types, hs
 
     def get_forces(self, r=0):
         """(forces, handles) of the last force evaluation, sorted by handle."""
         n = self.n_particles(r)
-        f = np.zeros((n, 3))
-        hs = np.zeros(n, dtype=np.uint32)
+        f = np.empty((n, 3))
+        hs = np.empty(n, dtype=np.uint32)
         m = ctypes.c_uint64()
         L.check(self._lib.rdy_get_forces(self._h, r, n, _ptr(f, _dp), _ptr(hs, _u32p), ctypes.byref(m)))
-        o = np.argsort(hs, kind="stable")
-        return f[o], hs[o]
+        return f, hs
 
     def set_bonds(self, r, idx, k, length):
         idx = np.ascontiguousarray(idx, dtype=np.uint32).reshape(-1, 2)

@@ -42,3 +42,44 @@ def test_counts_per_replica_and_type(sizes, kw):
         assert got[0].sum() == 0
         assert np.array_equal(e.count_types(2), got[:2])
     e.close()
+
+
+@pytest.mark.parametrize("n,kw", [(0, {}), (1, {}), (255, {}), (256, {}), (5000, {}), (3000, dict(bin_capacity=2)),
+                                  (40000, {}),      # larger than the area a small answer comes back through
+                                  (400001, {})])    # several halves of the streamed area, a remainder in each
+def test_particles_come_back_in_handle_order(n, kw):
+    """Handles are the upload order, so the arrays come back as they went up; a second replica's stay apart."""
+    box = 12.0 if n < 6000 else 60.0
+    e, data = _engine((n, 77), box=box, **kw)
+    for r, pos, types in data:
+        p, t, h = e.get_particles(r)
+        assert np.array_equal(h, np.arange(len(types)))
+        assert np.array_equal(t, types)
+        assert np.array_equal(p, pos)
+        assert e.n_particles(r) == len(types)
+    e.close()
+
+
+def test_handles_past_the_expected_range_and_forces_in_step():
+    """Decays and conversions leave gaps and reach handles beyond the last read (a conversion renames: 900 x 40 steps
+    pass the first estimate): the particles still come back ordered, and the forces in the same order."""
+    rng = np.random.default_rng(5)
+    e = Engine(2, [1.0, 1.0], potentials=[(L.POT_HARMONIC_REPULSION, a, b, [10.0, 1.0]) for a, b in ((0, 0), (0, 1), (1, 1))],
+               reactions=[dict(kind=L.RX_CONVERSION, educts=[0], products=[1], rate=80.0),
+                          dict(kind=L.RX_CONVERSION, educts=[1], products=[0], rate=80.0),
+                          dict(kind=L.RX_DECAY, educts=[0], products=[], rate=0.5)])
+    r = e.add_replica([10.0] * 3, seed=9, max_particles=1000)
+    e.set_particles(r, (rng.random((900, 3)) - 0.5) * 10.0, np.zeros(900, np.uint32))
+    e.run(L.HANDLER_UA, 0.01, 40)
+    p, t, h = e.get_particles(r)
+    assert h.max() > 4096 + 1350 and len(h) == e.n_particles(r) < 900
+    assert np.all(np.diff(h.astype(np.int64)) > 0)
+    assert np.array_equal(e.count_types(1)[0], np.bincount(t, minlength=2))
+    f, hf = e.get_forces(r)
+    assert np.array_equal(hf, h)
+    d = p[None] - p[:, None]  # neighbour - particle
+    d -= 10.0 * np.round(d / 10.0)
+    dist = np.sqrt((d * d).sum(2)) + 10.0 * np.eye(len(p))
+    ref = (np.where(dist < 1.0, 10.0 * (dist - 1.0) / dist, 0.0)[:, :, None] * d).sum(1)
+    assert np.linalg.norm(f - ref) < 1e-5 * np.linalg.norm(ref)
+    e.close()
