@@ -16,11 +16,11 @@
 // A brick whose halo holds more particles than the LDS budget takes a slow path that reads
 // neighbours straight from the bins.
 //
-// Per axis a brick is either in halo mode (extent e, halo r on both sides; the host guarantees
-// e + 2r <= dims on periodic axes, so halo cells are distinct and the local displacement is the
-// minimum image) or in whole-axis mode (the brick spans the axis, no halo; neighbour coordinates
-// wrap inside the brick), which also reproduces the de-duplicated adjacency of small grids
-// (CellLinkedList.cpp:74-137).
+// Per axis a brick is either in halo mode (extent e, halo r on both sides; the axis has at least 2r + 1
+// cells when it is periodic, so the cells of a stencil are distinct; when e + 2r exceeds the axis, halo
+// cells repeat cells of the brick at another image) or in whole-axis mode (a periodic axis of at most
+// 2r cells: the brick spans it, no halo; neighbour coordinates wrap inside the brick), which also
+// reproduces the de-duplicated adjacency of small grids (CellLinkedList.cpp:74-137).
 #pragma once
 
 #include "rdy_kernels.hip"

@@ -736,14 +736,17 @@ int check_replica(rdy_engine *e, uint32_t r) {
     return RDY_OK;
 }
 
-// splits replica r's grid into bricks (halo mode where the axis is long enough, whole-axis otherwise)
+// Splits replica r's grid into bricks.  An axis is in halo mode, also when one brick spans it (its halo then holds
+// images of its own far cells), unless it is periodic and shorter than a stencil: the 2r + 1 cells of a stencil
+// have to be distinct, so that every neighbour is staged at one image only (a pair closer than the cutoff is
+// adjacent through that image, since the cells between the other way are at least a cutoff wide).
 void make_bricks(rdy_engine *e, uint32_t r, std::vector<BrickDev> &out) {
     const ReplicaDev &R = e->reps_h[r].dev;
     std::vector<std::pair<int32_t, int32_t>> seg[3];
     uint32_t whole = 0, halo[3];
     for (int a = 0; a < 3; ++a) {
         const int32_t D = R.dims[a], B = (int32_t)e->brick[a], h = e->radius;
-        const bool w = D <= B || (R.pbc[a] && D < B + 2 * h);
+        const bool w = R.pbc[a] && D < 2 * h + 1;
         if (w) {
             whole |= 1u << a;
             seg[a].push_back({0, D});
@@ -901,7 +904,7 @@ void choose_brick(double lam, const int32_t *dims, int radius, uint32_t out[3]) 
                 const uint32_t ee[3] = {ex, ey, ez};
                 for (int a = 0; a < 3; ++a) {
                     const double D = (double)dims[a];
-                    if ((double)ee[a] + 2.0 * radius > D) {
+                    if (D < 2.0 * radius + 1.0) {
                         staged *= D;  // whole-axis brick: no halo
                     } else {
                         const double n = std::ceil(D / ee[a]);
