@@ -791,17 +791,21 @@ __device__ __forceinline__ void finish_particle(const Grid &nxt, const ReplicaDe
     if (slot != 0xFFFFFFFFu && (me.tw & TW_TOPO) && topo.loc) topo.loc[R.topo_base + me.h] = slot;
 }
 
-// visits the records of the brick's own cells straight from the bins: fn(slot, state)
+// fn(cell) for the brick's own cells, spread over the block's threads
 template <class Fn>
-__device__ __forceinline__ void for_each_own_record(const Grid &cur, const BrickDev &B, const RepGeom &geo,
-                                                    uint32_t cap, Fn &&fn) {
+__device__ __forceinline__ void for_each_own_cell(const BrickDev &B, Fn &&fn) {
     const uint32_t ncell = (uint32_t)(B.e[0] * B.e[1] * B.e[2]);
     for (uint32_t ci = threadIdx.x; ci < ncell; ci += BRICK_THREADS) {
         const uint32_t lz = ci % B.e[2], ly = (ci / B.e[2]) % B.e[1], lx = ci / (B.e[2] * B.e[1]);
-        const uint32_t cell = geo.cell_base +
-                              ((uint32_t)(B.o[0] + lx) * (uint32_t)geo.dims[1] + (uint32_t)(B.o[1] + ly)) *
-                                  (uint32_t)geo.dims[2] +
-                              (uint32_t)(B.o[2] + lz);
+        fn(B.cell_base + ((uint32_t)(B.o[0] + lx) * (uint32_t)B.dims[1] + (uint32_t)(B.o[1] + ly)) * (uint32_t)B.dims[2] +
+           (uint32_t)(B.o[2] + lz));
+    }
+}
+
+// visits the records of the brick's own cells straight from the bins: fn(slot, state)
+template <class Fn>
+__device__ __forceinline__ void for_each_own_record(const Grid &cur, const BrickDev &B, uint32_t cap, Fn &&fn) {
+    for_each_own_cell(B, [&](uint32_t cell) {
         const uint32_t n = cur.counts[cell];
         const uint32_t m = n < cap ? n : cap;
         for (uint32_t k = 0; k < m; ++k) fn(cell * cap + k, cur.bins[cell * cap + k]);
@@ -815,7 +819,7 @@ __device__ __forceinline__ void for_each_own_record(const Grid &cur, const Brick
                     fn(cur.nbin + o, cur.bins[cur.nbin + o]);
                 }
         }
-    }
+    });
 }
 
 struct ForceWave {  // per-wave LDS of k_brick
@@ -852,7 +856,7 @@ __device__ __forceinline__ void release_slow_list(uint32_t *list) {
 // forces (+ Euler-Maruyama + re-bin) of every particle of one brick; MODE as in k_fused.
 // AH: the launch covers bricks brick0.. that are in halo mode on every axis (else: none is).
 template <int MODE, bool AH>
-__global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, ReplicaDev *reps, Tables T, Topo topo,
+__global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Grid clear, ReplicaDev *reps, Tables T, Topo topo,
                                                          const BrickDev *bricks, uint32_t brick0, uint32_t cap,
                                                          int radius, double dt,
                                                          const double *noise, double *force_out, uint32_t max_states,
@@ -863,6 +867,13 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Rep
     const uint32_t bidx = brick0 + xcd_block(blockIdx.x, gridDim.x);
     const BrickDev B = bricks[bidx];
     const ReplicaDev &R = reps[B.r];
+    if (MODE == MODE_REBIN) {  // the buffer after the target is cleared for the re-binning (or walk) that follows
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            *nxt.wl_count = 0u;
+            *clear.ovf_count = 0u;
+        }
+        for_each_own_cell(B, [&](uint32_t cell) { clear.counts[cell] = 0u; });
+    }
     if (!R.in_use) return;
     if (MODE != MODE_FORCES) virial = nullptr;
     long long vir[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -870,7 +881,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Rep
     const bool forces_on = MODE == MODE_FORCES || (MODE == MODE_STEP && R.active);
     if (!forces_on) {
         // re-bin only (neighbour-list update, or a replica whose step budget is spent): no staging
-        for_each_own_record(cur, B, geo, cap, [&](uint32_t s, const State &me) {
+        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (!(me.tw & TW_DEAD))
                 finish_particle<MODE_REBIN>(nxt, R, geo, T, topo, cap, dt, noise, force_out, s, me, false, 0, 0, 0,
                                             err);
@@ -990,7 +1001,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_slow(Grid cur, Grid nxt
         const RepGeom geo = load_geom(R);
         long long e_blk = 0;
         long long vir[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        for_each_own_record(cur, B, geo, cap, [&](uint32_t s, const State &me) {
+        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (me.tw & TW_DEAD) return;
             long long fx = 0, fy = 0, fz = 0, e = 0;
             if (!(me.tw & TW_OUTSIDE))
@@ -1008,12 +1019,10 @@ struct SearchWave {  // per-wave LDS of k_brick_search
     uint32_t s[64];  // bin slots of the wave's 64 particles
 };
 
-// reaction candidate search of one brick on the current buffer (see search_one for the rules),
-// fused with clearing the previous buffer (clear_old): the counters of the brick's cells, and (block
-// 0) its work-list and overflow lengths
+// reaction candidate search of one brick on the current buffer (see search_one for the rules)
 template <bool AH>
-__global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Grid old, int clear_old, ReplicaDev *reps,
-                                                                Tables T, const BrickDev *bricks, uint32_t brick0,
+__global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, ReplicaDev *reps, Tables T,
+                                                                const BrickDev *bricks, uint32_t brick0,
                                                                 uint32_t cap,
                                                                 int radius, int handler, Event *events,
                                                                 uint32_t *ev_count, uint32_t max_states,
@@ -1025,21 +1034,6 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Grid o
     const BrickDev B = bricks[bidx];
     const ReplicaDev &R = reps[B.r];
     const RepGeom geo = load_geom(R);
-    // clear the old buffer (it is not read again before it becomes the next target)
-    if (clear_old) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            *old.wl_count = 0u;
-            *old.ovf_count = 0u;
-        }
-        const uint32_t ncell = (uint32_t)(B.e[0] * B.e[1] * B.e[2]);
-        for (uint32_t ci = threadIdx.x; ci < ncell; ci += BRICK_THREADS) {
-            const uint32_t lz = ci % B.e[2], ly = (ci / B.e[2]) % B.e[1], lx = ci / (B.e[2] * B.e[1]);
-            old.counts[geo.cell_base +
-                       ((uint32_t)(B.o[0] + lx) * (uint32_t)geo.dims[1] + (uint32_t)(B.o[1] + ly)) *
-                           (uint32_t)geo.dims[2] +
-                       (uint32_t)(B.o[2] + lz)] = 0u;
-        }
-    }
     // a launch without reactions (handler 2) covers every replica; DetailedBalance searches every replica
     // with the Gillespie keys; else a replica's own choice wins
     if (handler == HANDLER_DETAILED_BALANCE) handler = 1;
@@ -1181,8 +1175,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search_slow(Grid cur, R
     if (n == 0) return;  // grid-uniform
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const BrickDev B = bricks[slow[2 + i]];
-        const RepGeom geo = load_geom(reps[B.r]);
-        for_each_own_record(cur, B, geo, cap, [&](uint32_t s, const State &me) {
+        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (!(me.tw & TW_DEAD))
                 search_one(cur, reps, T, cap, radius, handler, 0, events, ev_count, nullptr, 0, s, me, err);
         });

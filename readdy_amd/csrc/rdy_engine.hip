@@ -32,6 +32,8 @@ int set_err(int code, const std::string &msg) {
         if (e_ != hipSuccess) return set_err(RDY_ERR_HIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+constexpr int N_STATES = 4;  // even: the bin buffer of a state is its parity
+
 constexpr size_t STAGING_SMALL = 256u << 10;  // pinned bytes a small readback uses
 constexpr size_t STAGING_HALF = 4u << 20;     // one half of the pinned area a large one streams through
 
@@ -117,11 +119,13 @@ struct rdy_engine {
     // device pools
     ReplicaDev *reps = nullptr;
     State *bins[2] = {nullptr, nullptr};
-    uint32_t *counts[2] = {nullptr, nullptr};
+    // Cell counters of N_STATES buffers take turns over the two bin buffers: a walk inserts into the next state's
+    // counters, which are clear, and clears those of the state after it, so that no launch of its own has to.
+    uint32_t *counts[N_STATES] = {};
     uint32_t *wl[2] = {nullptr, nullptr};
     uint32_t *wl_count = nullptr;  // [2]
     uint32_t *ovf_cell[2] = {nullptr, nullptr};
-    uint32_t *ovf_count = nullptr;  // [2]
+    uint32_t *ovf_count = nullptr;  // [N_STATES]
     uint32_t ovf_cap = 0;
     bool auto_cap = false;
     uint32_t *tile_sums = nullptr;
@@ -137,7 +141,7 @@ struct rdy_engine {
     uint32_t *d_slow = nullptr;  // two lists of bricks left to the bin-reading kernels (forces, search)
     uint32_t n_bricks_ah = 0;    // leading bricks of bricks_h in halo mode on every axis
     bool bricks_dirty = false;   // replicas changed since the last brick upload
-    bool wl_valid[2] = {true, true};
+    bool wl_valid = true;  // the current buffer has a work list
     uint64_t cells_hwm = 0;  // end of the highest cell range handed out (the scan covers [0, hwm))
     Event *events = nullptr;
     uint32_t *ev_count = nullptr;
@@ -155,13 +159,11 @@ struct rdy_engine {
     // changed by reactions, the records moved again and the copies withdrawn; force_out and the
     // energies are formed on demand after a run (export_valid)
     Edit *edits = nullptr;
-    uint32_t *edit_count = nullptr;  // [3]: changed records, records to move again, copies to withdraw
+    uint32_t *edit_count = nullptr;  // [2]: changed records, records to move again
     uint32_t edit_cap = 0;
     uint32_t *aff_bits = nullptr;
     uint32_t *aff_list = nullptr;
     uint32_t aff_cap = 0;
-    uint2 *wd_list = nullptr;
-    uint32_t wd_cap = 0;
     bool export_valid = true;
     // tables
     PotDev *d_pots = nullptr;
@@ -217,9 +219,9 @@ struct rdy_engine {
     hipEvent_t staging_ev[2] = {nullptr, nullptr};
     double *d_noise = nullptr;
     size_t noise_cap = 0;
-    int cur = 0;
-    // graph
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    int cur = 0;  // state of the current buffer
+    // graphs of N_STATES fused steps, one per state that they start (and end) in
+    hipGraphExec_t gexec[N_STATES] = {};
     uint64_t g_version = ~0ull;
     int g_handler = -1;
     double g_dt = -1.0;
@@ -235,10 +237,14 @@ struct rdy_engine {
     double prof_ms = 0.0;
     uint64_t prof_n = 0;
 
-    Grid grid(int b) const {
-        return Grid{bins[b], counts[b], wl[b], wl_count + b, ovf_cell[b], ovf_count + b, (uint32_t)(max_cells * cap),
+    // the buffer of state s (0 .. N_STATES - 1)
+    Grid grid(int s) const {
+        const int b = s & 1;
+        return Grid{bins[b], counts[s], wl[b], wl_count + b, ovf_cell[b], ovf_count + s, (uint32_t)(max_cells * cap),
                     ovf_cap};
     }
+    int next() const { return (cur + 1) % N_STATES; }
+    int after_next() const { return (cur + 2) % N_STATES; }
     Topo topo() const { return Topo{fb, loc}; }
 };
 
@@ -632,15 +638,17 @@ int alloc_pools(rdy_engine *e) {
     for (int b = 0; b < 2; ++b) {
         HIP_TRY(dalloc(&e->bins[b], slots));
         HIP_TRY(dalloc(&e->ovf_cell[b], e->ovf_cap));
-        HIP_TRY(dalloc(&e->counts[b], e->max_cells));
-        HIP_TRY(hipMemsetAsync(e->counts[b], 0, e->max_cells * sizeof(uint32_t), e->stream));
         HIP_TRY(dalloc(&e->wl[b], e->max_particles));
+    }
+    for (uint32_t *&c : e->counts) {
+        HIP_TRY(dalloc(&c, e->max_cells));
+        HIP_TRY(hipMemsetAsync(c, 0, e->max_cells * sizeof(uint32_t), e->stream));
     }
     HIP_TRY(dalloc(&e->wl_count, 2));
     HIP_TRY(hipMemsetAsync(e->wl_count, 0, 2 * sizeof(uint32_t), e->stream));
     HIP_TRY(dalloc(&e->tile_sums, (e->max_cells + SCAN_TILE - 1) / SCAN_TILE + 2));
-    HIP_TRY(dalloc(&e->ovf_count, 2));
-    HIP_TRY(hipMemsetAsync(e->ovf_count, 0, 2 * sizeof(uint32_t), e->stream));
+    HIP_TRY(dalloc(&e->ovf_count, N_STATES));
+    HIP_TRY(hipMemsetAsync(e->ovf_count, 0, N_STATES * sizeof(uint32_t), e->stream));
     HIP_TRY(dalloc(&e->reps, e->max_reps));
     HIP_TRY(hipMemsetAsync(e->reps, 0, e->max_reps * sizeof(ReplicaDev), e->stream));
     HIP_TRY(dalloc(&e->events, (size_t)e->max_reps * e->ev_per_rep));
@@ -676,12 +684,10 @@ int ensure_step_pools(rdy_engine *e) {
     // changes the forces of its neighbours within the cutoff
     e->edit_cap = (uint32_t)std::min<uint64_t>(3ull * e->max_reps * e->ev_per_rep, 1ull << 22);
     e->aff_cap = (uint32_t)std::min<uint64_t>(32ull * e->edit_cap, std::max<uint64_t>(slots, 1ull << 16));
-    e->wd_cap = e->aff_cap;
     HIP_TRY(dalloc(&e->edits, e->edit_cap));
     HIP_TRY(dalloc(&e->aff_list, e->aff_cap));
-    HIP_TRY(dalloc(&e->wd_list, e->wd_cap));
-    HIP_TRY(dalloc(&e->edit_count, 3));
-    HIP_TRY(hipMemsetAsync(e->edit_count, 0, 3 * sizeof(uint32_t), e->stream));
+    HIP_TRY(dalloc(&e->edit_count, 2));
+    HIP_TRY(hipMemsetAsync(e->edit_count, 0, 2 * sizeof(uint32_t), e->stream));
     return RDY_OK;
 }
 
@@ -796,11 +802,11 @@ int upload_bricks(rdy_engine *e) {
     auto ah_end = std::stable_partition(e->bricks_h.begin(), e->bricks_h.end(),
                                         [](const BrickDev &b) { return b.whole == 0; });
     e->n_bricks_ah = (uint32_t)(ah_end - e->bricks_h.begin());
-    if (e->bricks_h.size() > e->d_bricks_cap) {
+    if (e->bricks_h.size() > e->d_bricks_cap || !e->d_slow) {  // (the slow lists exist without bricks too)
         HIP_TRY(hipStreamSynchronize(e->stream));
         if (e->d_bricks) HIP_TRY(hipFree(e->d_bricks));
         if (e->d_slow) HIP_TRY(hipFree(e->d_slow));
-        e->d_bricks_cap = std::max<size_t>(e->bricks_h.size(), 2 * e->d_bricks_cap);
+        e->d_bricks_cap = std::max<size_t>({e->bricks_h.size(), 2 * e->d_bricks_cap, 1});
         HIP_TRY(dalloc(&e->d_bricks, e->d_bricks_cap));
         HIP_TRY(dalloc(&e->d_slow, 2 * (e->d_bricks_cap + 2)));
         HIP_TRY(hipMemsetAsync(e->d_slow, 0, 2 * (e->d_bricks_cap + 2) * sizeof(uint32_t), e->stream));
@@ -988,9 +994,9 @@ void launch_bonded(rdy_engine *e, bool energy) {
 
 uint32_t wl_blocks(const rdy_engine *e) { return blocks_for(e->max_particles, e->block); }
 
-// rebuilds buffer b's work list in cell order from its cell counters
-void launch_wl_rebuild(rdy_engine *e, int b) {
-    Grid g = e->grid(b);
+// rebuilds the current buffer's work list in cell order from its cell counters
+void launch_wl_rebuild(rdy_engine *e) {
+    Grid g = e->grid(e->cur);
     const uint32_t nc = (uint32_t)std::max<uint64_t>(e->cells_hwm, 1);
     const uint32_t tiles = (nc + SCAN_TILE - 1) / SCAN_TILE;
     hipLaunchKernelGGL(k_wl_tiles, dim3(tiles), dim3(SCAN_THREADS), 0, e->stream, g, e->cap, nc, e->tile_sums);
@@ -998,106 +1004,95 @@ void launch_wl_rebuild(rdy_engine *e, int b) {
                        (uint32_t)e->max_particles, e->err);
     hipLaunchKernelGGL(k_wl_write, dim3(tiles), dim3(SCAN_THREADS), 0, e->stream, g, e->cap, nc,
                        (const uint32_t *)e->tile_sums, tiles, (uint32_t)e->max_particles);
-    e->wl_valid[b] = true;
+    e->wl_valid = true;
 }
 
 // the work list is only needed by per-particle helpers (gather, exports, the separate integrator)
 void ensure_wl(rdy_engine *e) {
-    if (!e->wl_valid[e->cur]) launch_wl_rebuild(e, e->cur);
+    if (!e->wl_valid) launch_wl_rebuild(e);
 }
 
-// clears buffer b's cell counters (brick-wise) and its work-list / overflow lengths
-void launch_clear_bricks(rdy_engine *e, int b, int grid_of_bricks_buffer) {
-    if (!e->bricks_h.empty())
-        hipLaunchKernelGGL(k_brick_search<false>, dim3(n_bricks(e)), dim3(BRICK_THREADS), 0, e->stream,
-                           e->grid(grid_of_bricks_buffer), e->grid(b), 1, e->reps, e->T, (const BrickDev *)e->d_bricks,
-                           0u, e->cap, e->radius, 2, e->events, e->ev_count, e->max_states, e->max_halo, 0u,
-                           slow_list(e, 1), e->err);
-    else
-        hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, e->stream, e->grid(b));
-}
+constexpr uint64_t GRAPH_MIN_STEPS = 32;
 
-// workgroups of the fix-up kernels (their waves / threads stride over the change lists)
-constexpr uint32_t FIX_BLOCKS = 1024;
+// workgroups of the fix-up kernels (their waves stride over the change lists): 1024 waves, one per changed record
+// of every step measured (about 230 at 1,000,000 particles), since a launch of 1024 workgroups takes longer to
+// hand out than a small system's changes take to make
+constexpr uint32_t FIX_BLOCKS = 256;
 
-// one walk of k_brick_step from cur into the other buffer (prologue: the first walk of a run)
-// the walk of a step (or the prologue); slow_later: the bricks listed for the bin-reading path are
-// walked by k_resolve_step instead of a follow-up launch
-void launch_walk(rdy_engine *e, int prologue, int handler, double dt, bool slow_later = false) {
-    const int c = e->cur, n = 1 - c;
-    if (e->prof && !prologue && e->prof_used < e->prof_ev.size())
-        (void)hipEventRecord(e->prof_ev[e->prof_used].first, e->stream);
+// one walk of k_brick_step from the current buffer into the next (flags: WALK_PROLOGUE, WALK_LAST).  The bricks
+// listed for the bin-reading path are walked by k_resolve_step when reactions follow, else by a launch here.
+void launch_walk(rdy_engine *e, int flags, int handler, double dt) {
+    const Grid cur = e->grid(e->cur), nxt = e->grid(e->next()), clear = e->grid(e->after_next());
+    const bool prof = e->prof && !(flags & WALK_PROLOGUE) && e->prof_used < e->prof_ev.size();
+    if (prof) (void)hipEventRecord(e->prof_ev[e->prof_used].first, e->stream);
     for_brick_groups(e, [&](auto ah, uint32_t nb, uint32_t b0) {
         hipLaunchKernelGGL((k_brick_step<decltype(ah)::value>), dim3(nb), dim3(BRICK_THREADS), e->brick_smem,
-                           e->stream, e->grid(c), e->grid(n), prologue, e->reps, e->T, e->topo(),
+                           e->stream, cur, nxt, clear, flags, (const ReplicaDev *)e->reps, e->T, e->topo(),
                            (const BrickDev *)e->d_bricks, b0, e->cap, e->radius, handler, dt, e->events, e->ev_count,
-                           e->max_states, e->max_halo, (uint32_t)e->brick_smem, slow_list(e, 0), e->err);
+                           e->max_states, e->max_halo, (uint32_t)e->brick_smem, slow_list(e, 0), e->edit_count, e->err);
     });
-    if (e->prof && !prologue && e->prof_used < e->prof_ev.size()) {
+    if (prof) {
         (void)hipEventRecord(e->prof_ev[e->prof_used].second, e->stream);
         e->prof_used++;
     }
-    if (slow_later) return;
-    hipLaunchKernelGGL(k_brick_step_slow, dim3(slow_blocks(e)), dim3(BRICK_THREADS), 0, e->stream, e->grid(c),
-                       e->grid(n), prologue, e->reps, e->T, e->topo(), (const BrickDev *)e->d_bricks, e->cap,
-                       e->radius, handler, dt, e->events, e->ev_count, slow_list(e, 0), e->err);
+    if (handler != RDY_HANDLER_NONE) return;
+    hipLaunchKernelGGL(k_brick_step_slow, dim3(slow_blocks(e)), dim3(BRICK_THREADS), 0, e->stream, cur, nxt, flags,
+                       e->reps, e->T, e->topo(), (const BrickDev *)e->d_bricks, e->cap, e->radius, dt, slow_list(e, 0),
+                       e->err);
+}
+
+// clears the bonded forces (engines with topologies); n_loc: topology slots kept for the topology reactions
+void launch_topo_begin(rdy_engine *e, uint64_t n_loc) {
+    const uint64_t nfb = e->fb ? 3 * e->topo_used : 0;
+    if (nfb == 0 && n_loc == 0) return;
+    hipLaunchKernelGGL(k_topo_begin, dim3(blocks_for(std::max(nfb, n_loc), 256)), dim3(256), 0, e->stream, e->fb,
+                       (uint32_t)nfb, (const uint32_t *)e->loc, e->loc_cur, (uint32_t)n_loc);
+}
+
+void advance_state(rdy_engine *e) {
+    e->wl_valid = false;
+    e->cur = e->next();
 }
 
 // the first walk of a run: the forces of the current state and step 1's move (bonded terms first)
 void launch_prologue(rdy_engine *e, double dt) {
     launch_bonded(e, false);
-    launch_walk(e, 1, (int)RDY_HANDLER_NONE, dt);
-    e->wl_valid[1 - e->cur] = false;
-    e->cur = 1 - e->cur;
+    launch_walk(e, WALK_PROLOGUE, (int)RDY_HANDLER_NONE, dt);
+    advance_state(e);
 }
 
-// the end of a run: the buffer the last walk read is cleared, and so are the bonded forces
-void launch_epilogue(rdy_engine *e) {
-    const uint64_t nc = std::max<uint64_t>(e->cells_hwm, 1);
-    const uint64_t nfb = e->fb ? 3 * e->topo_used : 0;
-    hipLaunchKernelGGL(k_clear_grid, dim3(blocks_for(std::max(nc, nfb), 256)), dim3(256), 0, e->stream,
-                       e->grid(1 - e->cur), (uint32_t)nc, e->fb, (uint32_t)nfb);
-}
+// the end of a run: the bonded forces are cleared (between runs they are formed where they are consumed)
+void launch_epilogue(rdy_engine *e) { launch_topo_begin(e, 0); }
 
 // one fused step over all replicas (SimulationLoop.h:280-300, rdy_step.hip): the walk over x'(t)
 // yields step t's candidates and, optimistically, step t+1's move; the reactions, the exact
 // corrections and the redone moves follow.  last: the launch's final step copies instead of moving.
 void launch_step(rdy_engine *e, int handler, double dt, int last) {
     const uint32_t nr = std::max<uint32_t>(e->n_reps_used, 1);
-    const int c = e->cur, n = 1 - c;
-    const uint64_t nc = std::max<uint64_t>(e->cells_hwm, 1);
-    const uint64_t nfb = e->fb ? 3 * e->topo_used : 0;
-    const uint64_t nloc = topo_reactions_on(e) ? e->topo_used : 0;
-    const uint64_t nthreads = std::max<uint64_t>(std::max<uint64_t>(std::max<uint64_t>(nr, (nc + 3) / 4), nfb), nloc);
-    hipLaunchKernelGGL(k_step_begin, dim3(blocks_for(nthreads, 256)), dim3(256), 0, e->stream, e->reps, nr, last,
-                       e->grid(n), (uint32_t)nc, e->fb, (uint32_t)nfb, e->edit_count, e->e_bonded,
-                       (const uint32_t *)e->loc, e->loc_cur, (uint32_t)nloc);
+    const Grid cur = e->grid(e->cur), nxt = e->grid(e->next());
+    const bool topo_rx = topo_reactions_on(e);
+    launch_topo_begin(e, topo_rx ? e->topo_used : 0);
     launch_bonded(e, false);
     const int h = (handler != RDY_HANDLER_NONE && e->n_rx > 0) ? handler : RDY_HANDLER_NONE;
-    launch_walk(e, 0, h, dt, h != RDY_HANDLER_NONE);
-    const bool topo_rx = topo_reactions_on(e);
+    launch_walk(e, last ? WALK_LAST : 0, h, dt);
+    if (h != RDY_HANDLER_NONE)
+        hipLaunchKernelGGL(k_resolve_step, dim3(nr), dim3(RESOLVE_THREADS), 0, e->stream, cur, nxt, e->reps, e->T,
+                           e->topo(), (const BrickDev *)e->d_bricks, e->cap, e->radius, h, dt, last, e->events,
+                           e->ev_count, slow_list(e, 0), e->rx_step, e->rx_total, (uint32_t)e->max_particles, e->edits,
+                           e->edit_count, e->edit_cap, rec_ptr(e), e->recording ? e->rec_count : nullptr, e->err);
+    else
+        hipLaunchKernelGGL(k_step_book, dim3(blocks_for(nr, 64)), dim3(64), 0, e->stream, e->reps, nr, last);
     if (h != RDY_HANDLER_NONE || topo_rx) {
-        if (h != RDY_HANDLER_NONE)
-        hipLaunchKernelGGL(k_resolve_step, dim3(nr), dim3(RESOLVE_THREADS), 0, e->stream, e->grid(c), e->grid(n),
-                           e->reps, e->T, e->topo(), (const BrickDev *)e->d_bricks, e->cap, e->radius, h, dt,
-                           e->events, e->ev_count, slow_list(e, 0), e->rx_step, e->rx_total,
-                           (uint32_t)e->max_particles, e->edits, e->edit_count, e->edit_cap, rec_ptr(e),
-                           e->recording ? e->rec_count : nullptr, e->err);
         // SimulationLoop.h:286-287: the topology reactions follow the reactions, on their result
         if (topo_rx) launch_topo_reactions(e, 1, e->edits, e->edit_count);
-        hipLaunchKernelGGL(k_fix_sites, dim3(FIX_BLOCKS), dim3(256), 0, e->stream, e->grid(c),
-                           (const ReplicaDev *)e->reps, e->T, e->cap, e->radius, (const Edit *)e->edits,
-                           (const uint32_t *)e->edit_count, e->edit_cap, e->aff_bits, e->aff_list, e->edit_count + 1,
-                           e->aff_cap, e->wd_list, e->edit_count + 2, e->wd_cap, e->err);
-        hipLaunchKernelGGL(k_fix_withdraw, dim3(FIX_BLOCKS), dim3(256), 0, e->stream, e->grid(c), e->grid(n),
-                           (const ReplicaDev *)e->reps, e->cap, (const uint2 *)e->wd_list,
-                           (const uint32_t *)(e->edit_count + 2), e->wd_cap);
-        hipLaunchKernelGGL(k_fix_advance, dim3(FIX_BLOCKS), dim3(256), 0, e->stream, e->grid(c), e->grid(n),
+        hipLaunchKernelGGL(k_fix_sites, dim3(FIX_BLOCKS), dim3(256), 0, e->stream, cur, nxt, (const ReplicaDev *)e->reps,
+                           e->T, e->cap, e->radius, (const Edit *)e->edits, (const uint32_t *)e->edit_count, e->edit_cap,
+                           e->aff_bits, e->aff_list, e->edit_count + 1, e->aff_cap, e->err);
+        hipLaunchKernelGGL(k_fix_advance, dim3(FIX_BLOCKS), dim3(256), 0, e->stream, cur, nxt,
                            (const ReplicaDev *)e->reps, e->T, e->topo(), e->cap, e->radius, dt, e->aff_bits,
                            (const uint32_t *)e->aff_list, (const uint32_t *)(e->edit_count + 1), e->aff_cap, e->err);
     }
-    e->wl_valid[n] = false;
-    e->cur = n;
+    advance_state(e);
 }
 
 void launch_forces(rdy_engine *e, double *force_out) {
@@ -1109,8 +1104,8 @@ void launch_forces(rdy_engine *e, double *force_out) {
     const int c = e->cur;
     for_brick_groups(e, [&](auto ah, uint32_t nb, uint32_t b0) {
         hipLaunchKernelGGL((k_brick<MODE_FORCES, decltype(ah)::value>), dim3(nb), dim3(BRICK_THREADS), e->brick_smem,
-                           e->stream, e->grid(c), e->grid(c), e->reps, e->T, e->topo(), (const BrickDev *)e->d_bricks,
-                           b0, e->cap, e->radius, 0.0, (const double *)nullptr, force_out, e->max_states, e->max_halo,
+                           e->stream, e->grid(c), e->grid(c), e->grid(c), e->reps, e->T, e->topo(),
+                           (const BrickDev *)e->d_bricks, b0, e->cap, e->radius, 0.0, (const double *)nullptr, force_out, e->max_states, e->max_halo,
                            (uint32_t)e->brick_smem, slow_list(e, 0), e->err, vir);
     });
     hipLaunchKernelGGL(k_brick_slow<MODE_FORCES>, dim3(slow_blocks(e)), dim3(BRICK_THREADS), 0, e->stream,
@@ -1259,14 +1254,16 @@ int rdy_engine_destroy(rdy_engine *e) {
     if (!e) return RDY_OK;
     (void)hipStreamSynchronize(e->stream);
     for (int b = 0; b < 2; ++b) {
-        if (e->gexec[b]) (void)hipGraphExecDestroy(e->gexec[b]);
         (void)hipFree(e->bins[b]);
-        (void)hipFree(e->counts[b]);
         (void)hipFree(e->wl[b]);
         (void)hipFree(e->ovf_cell[b]);
     }
+    for (int s = 0; s < N_STATES; ++s) {
+        if (e->gexec[s]) (void)hipGraphExecDestroy(e->gexec[s]);
+        (void)hipFree(e->counts[s]);
+    }
     void *ptrs[] = {e->wl_count, e->ovf_count, e->tile_sums, e->d_bricks, e->d_slow, e->reps, e->events, e->ev_count, e->recs, e->rec_count, e->rx_step, e->rx_total, e->e_bonded, e->virial, e->err,
-                    e->force_out, e->edits, e->edit_count, e->aff_bits, e->aff_list, e->wd_list, e->d_pots, e->d_pidx, e->d_rx, e->d_o1idx, e->d_o1list, e->d_o2list, e->d_o2idx,
+                    e->force_out, e->edits, e->edit_count, e->aff_bits, e->aff_list, e->d_pots, e->d_pidx, e->d_rx, e->d_o1idx, e->d_o1list, e->d_o2list, e->d_o2idx,
                     e->d_rowmax, e->d_dbpots, e->d_dbpidx, e->d_dbtable, e->d_dbkind, e->d_dbpref, e->d_dbradii, e->d_dbcdf, e->d_D, e->d_bd_scale, e->d_flavor, e->topo_of, e->topo_owner, e->treact, e->loc_cur, e->d_sr, e->ttype, e->tev, e->tev_count, e->tfus, e->tfus_count, e->tmrg, e->tmrg_count, e->adj_off, e->adj, e->str_step, e->str_total, e->fb, e->loc, e->scratch, e->d_noise, e->d_terms[0], e->d_terms[1],
                     e->d_terms[2]};
     for (void *p : ptrs)
@@ -1373,7 +1370,7 @@ int rdy_replica_remove(rdy_engine *e, uint32_t r) {
     if ((rc = put_field(e, r, offsetof(ReplicaDev, in_use), zero))) return rc;
     if ((rc = put_field(e, r, offsetof(ReplicaDev, active), zero))) return rc;
     HostReplica &H = e->reps_h[r];
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < N_STATES; ++b)
         hipLaunchKernelGGL(k_release_cells, dim3(blocks_for(H.n_cells, 256)), dim3(256), 0, e->stream, e->grid(b),
                            (uint32_t)H.cell_base, (uint32_t)H.n_cells);
     release_range(e->free_cells, H.cell_base, H.n_cells);
@@ -1382,7 +1379,7 @@ int rdy_replica_remove(rdy_engine *e, uint32_t r) {
     release_topo(e, H);
     H.in_use = false;
     e->version++;
-    e->wl_valid[0] = e->wl_valid[1] = false;
+    e->wl_valid = false;
     HIP_TRY(hipStreamSynchronize(e->stream));
     e->bricks_dirty = true;
     return RDY_OK;
@@ -1495,7 +1492,7 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
                            (uint32_t)e->max_particles, e->err);
     }
     H.handle_guess = hn + (uint64_t)hn / 2 + 4096;
-    e->wl_valid[e->cur] = false;
+    e->wl_valid = false;
     e->version++;
     return check_errors(e);
 }
@@ -1571,7 +1568,7 @@ static int gather(rdy_engine *e, uint32_t r, uint64_t cap, double *pos, uint32_t
     HostReplica &H = e->reps_h[r];
     const uint64_t ncap = std::min<uint64_t>(cap, e->max_particles);
     const Grid g = e->grid(e->cur);
-    const uint32_t blocks = blocks_for(H.n_cells, 256);
+    const uint32_t blocks = std::min(blocks_for(H.n_cells, 256), RANK_BLOCKS);
     for (int attempt = 0;; ++attempt) {
         // the bitmap covers the handles of the last read and half as many again; a replica that has grown
         // past it says how many it has, and the readback is repeated
@@ -1701,14 +1698,13 @@ int rdy_update_neighbor_list(rdy_engine *e) {
     if (int rb = ensure_bricks(e)) return rb;
     int rc = upload_tables(e, e->tables_dt > 0 ? e->tables_dt : 1.0);
     if (rc) return rc;
-    const int c = e->cur, n = 1 - c;
+    if (e->bricks_h.empty()) return RDY_OK;  // every replica has been removed
     hipLaunchKernelGGL((k_brick<MODE_REBIN, false>), dim3(n_bricks(e)), dim3(BRICK_THREADS), 0, e->stream,
-                       e->grid(c), e->grid(n), e->reps, e->T, e->topo(), (const BrickDev *)e->d_bricks, 0u, e->cap,
-                       e->radius, 0.0, (const double *)nullptr, (double *)nullptr, e->max_states, e->max_halo, 0u,
-                       slow_list(e, 0), e->err, (unsigned long long *)nullptr);
-    launch_clear_bricks(e, c, n);
-    e->wl_valid[n] = false;
-    e->cur = n;
+                       e->grid(e->cur), e->grid(e->next()), e->grid(e->after_next()), e->reps, e->T, e->topo(),
+                       (const BrickDev *)e->d_bricks, 0u, e->cap, e->radius, 0.0, (const double *)nullptr,
+                       (double *)nullptr, e->max_states, e->max_halo, 0u, slow_list(e, 0), e->err,
+                       (unsigned long long *)nullptr);
+    advance_state(e);
     return check_errors(e);
 }
 
@@ -1977,8 +1973,7 @@ int rdy_react(rdy_engine *e, int handler, double dt) {
     const int c = e->cur;
     for_brick_groups(e, [&](auto ah, uint32_t nb, uint32_t b0) {
         hipLaunchKernelGGL((k_brick_search<decltype(ah)::value>), dim3(nb), dim3(BRICK_THREADS), e->brick_smem,
-                           e->stream, e->grid(c), e->grid(c), 0, e->reps, e->T, (const BrickDev *)e->d_bricks, b0,
-                           e->cap, e->radius, handler, e->events, e->ev_count, e->max_states, e->max_halo,
+                           e->stream, e->grid(c), e->reps, e->T, (const BrickDev *)e->d_bricks, b0, e->cap, e->radius, handler, e->events, e->ev_count, e->max_states, e->max_halo,
                            (uint32_t)e->brick_smem, slow_list(e, 1), e->err);
     });
     hipLaunchKernelGGL(k_brick_search_slow, dim3(slow_blocks(e)), dim3(BRICK_THREADS), 0, e->stream, e->grid(c),
@@ -2069,7 +2064,7 @@ int rdy_run(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
     if (handler < 0 || handler > RDY_HANDLER_NONE) return set_err(RDY_ERR_INVALID, "unknown reaction handler");
     int rc = upload_tables(e, dt);
     if (rc) return rc;
-    if (n_steps == 0) return RDY_OK;
+    if (n_steps == 0 || e->bricks_h.empty()) return RDY_OK;  // nothing to step
     if ((rc = ensure_step_pools(e))) return rc;
     e->export_valid = false;
     launch_prologue(e, dt);
@@ -2130,45 +2125,47 @@ int rdy_run_graph(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
     if (e->in_session) return set_err(RDY_ERR_STATE, "a run is open: finish it with rdy_run_end");
     int rc = upload_tables(e, dt);
     if (rc) return rc;
-    if (n_steps == 0) return RDY_OK;
+    if (n_steps == 0 || e->bricks_h.empty()) return RDY_OK;  // nothing to step
     if ((rc = ensure_step_pools(e))) return rc;
     e->export_valid = false;
     launch_prologue(e, dt);
     const bool prof = e->prof;
     e->prof = false;
     if (e->g_version != e->version || e->g_handler != handler || e->g_dt != dt) {
-        for (int b = 0; b < 2; ++b) {
-            if (e->gexec[b]) HIP_TRY(hipGraphExecDestroy(e->gexec[b]));
-            e->gexec[b] = nullptr;
+        for (hipGraphExec_t &g : e->gexec) {
+            if (g) HIP_TRY(hipGraphExecDestroy(g));
+            g = nullptr;
         }
-        // capture two steps per parity so that every replay starts and ends on the same buffer
-        const int keep = e->cur;
-        for (int b = 0; b < 2; ++b) {
-            e->cur = b;
-            hipGraph_t g;
-            HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-            launch_step(e, handler, dt, 0);
-            launch_step(e, handler, dt, 0);
-            HIP_TRY(hipStreamEndCapture(e->stream, &g));
-            HIP_TRY(hipGraphInstantiate(&e->gexec[b], g, nullptr, nullptr, 0));
-            HIP_TRY(hipGraphDestroy(g));
-        }
-        e->cur = keep;
         e->g_version = e->version;
         e->g_handler = handler;
         e->g_dt = dt;
     }
-    // every step but the last from the graphs (the last one copies instead of moving)
-    const uint64_t generic = n_steps - 1, pairs = generic / 2;
-    for (uint64_t p = 0; p < pairs; ++p) {
-        HIP_TRY(hipGraphLaunch(e->gexec[e->cur], e->stream));
-        if ((p & 511) == 511)
-            if ((rc = check_errors(e))) return rc;
+    // every step but the last from the graph of N_STATES steps, which starts and ends in the same state (the last
+    // step copies instead of moving).  A capture costs about as much host time as GRAPH_MIN_STEPS launched steps.
+    uint64_t generic = n_steps - 1;
+    hipGraphExec_t &exec = e->gexec[e->cur];
+    if (!exec && generic >= GRAPH_MIN_STEPS) {
+        const int keep = e->cur;
+        hipGraph_t g;
+        HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
+        for (int k = 0; k < N_STATES; ++k) launch_step(e, handler, dt, 0);
+        e->cur = keep;
+        HIP_TRY(hipStreamEndCapture(e->stream, &g));
+        const hipError_t ge = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+        HIP_TRY(ge);
     }
-    if (generic & 1) launch_step(e, handler, dt, 0);
+    if (exec) {
+        for (uint64_t p = 0; p < generic / N_STATES; ++p) {
+            HIP_TRY(hipGraphLaunch(exec, e->stream));
+            if ((p & 255) == 255)
+                if ((rc = check_errors(e))) return rc;
+        }
+        generic %= N_STATES;
+    }
+    for (uint64_t k = 0; k < generic; ++k) launch_step(e, handler, dt, 0);
     launch_step(e, handler, dt, 1);
     launch_epilogue(e);
-    e->wl_valid[0] = e->wl_valid[1] = false;  // replays bypass launch_step's bookkeeping
     e->prof = prof;
     return check_errors(e);
 }
@@ -2758,7 +2755,7 @@ int rdy_append_topology_particles(rdy_engine *e, uint32_t r, uint64_t n, const u
     H.n_topo += (uint32_t)n;
     if ((rc = put_field(e, r, offsetof(ReplicaDev, n_topo), H.n_topo))) return rc;
     for (uint64_t i = 0; i < n; ++i) handles[i] = h0 + (uint32_t)i;
-    e->wl_valid[e->cur] = false;
+    e->wl_valid = false;
     e->export_valid = false;
     e->version++;
     return check_errors(e);

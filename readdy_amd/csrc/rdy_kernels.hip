@@ -201,11 +201,6 @@ __global__ void k_advance(ReplicaDev *reps, uint32_t n_reps, int mode, unsigned 
     }
 }
 
-__global__ void k_reset_counter(Grid old) {
-    *old.wl_count = 0u;
-    *old.ovf_count = 0u;
-}
-
 // -------------------------------------------------------------------------------------------------
 // work-list rebuild in cell order: an exclusive scan of the per-cell counters, then every cell writes
 // the slots of its members.  Neighbouring threads then hold neighbouring particles, so the stencil
@@ -1224,7 +1219,8 @@ __device__ __forceinline__ void resolve_replica(const Grid &cur, ReplicaDev *rep
     __syncthreads();
     const uint32_t hbase = R.handle_next;
     const RepGeom geo = load_geom(R);
-    // the fused step lists the changed records (edits) and flags inserted / retyped ones TW_NEW
+    // the fused step lists the changed records (edits) and flags inserted / retyped ones TW_NEW; its buffer's
+    // work list is not in use
     const bool fix = edits != nullptr;
     const uint32_t tw_new = fix ? TW_NEW : 0u;
     auto edit = [&](uint32_t slot, uint32_t kind, uint32_t old_type, uint32_t old_handle) {
@@ -1320,8 +1316,8 @@ __device__ __forceinline__ void resolve_replica(const Grid &cur, ReplicaDev *rep
             p1.h = hnew + 1u;
             cur.bins[e.s1].tw = a.tw | TW_DEAD;
             edit(e.s1, EDIT_KILLED, 0, 0);
-            edit(bin_insert(cur, geo, cap, p2, err, true, max_wl), EDIT_INSERTED, 0, 0);
-            edit(bin_insert(cur, geo, cap, p1, err, true, max_wl), EDIT_INSERTED, 0, 0);
+            edit(bin_insert(cur, geo, cap, p2, err, !fix, max_wl), EDIT_INSERTED, 0, 0);
+            edit(bin_insert(cur, geo, cap, p1, err, !fix, max_wl), EDIT_INSERTED, 0, 0);
             break;
         }
         case RX_FUSION: {
@@ -1340,7 +1336,7 @@ __device__ __forceinline__ void resolve_replica(const Grid &cur, ReplicaDev *rep
             cur.bins[e.s2].tw = bst.tw | TW_DEAD;
             edit(e.s1, EDIT_KILLED, 0, 0);
             edit(e.s2, EDIT_KILLED, 0, 0);
-            edit(bin_insert(cur, geo, cap, pr, err, true, max_wl), EDIT_INSERTED, 0, 0);
+            edit(bin_insert(cur, geo, cap, pr, err, !fix, max_wl), EDIT_INSERTED, 0, 0);
             break;
         }
         }
@@ -1452,18 +1448,20 @@ struct RankInfo {  // what k_rank_mark reports to the host
     uint32_t live, beyond, handle_next, pad;
 };
 
-// fn(slot) for the records of this thread's cell of the replica and for its share of the overflow records
+// fn(slot) for the records of the replica's cells and of the overflow region, spread over the grid's threads
+constexpr uint32_t RANK_BLOCKS = 1024;  // at most: each ends in one atomic on the count
+
 template <class Fn>
 __device__ __forceinline__ void replica_records(const Grid &g, uint32_t cap, uint32_t cell_base, uint32_t n_cells,
                                                 Fn &&fn) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n_cells) {
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (uint32_t i = i0; i < n_cells; i += stride) {
         const uint32_t cell = cell_base + i, n = min(g.counts[cell], cap);
         for (uint32_t k = 0; k < n; ++k) fn(cell * cap + k);
     }
     uint32_t no = *g.ovf_count;
     no = no < g.ovf_cap ? no : g.ovf_cap;
-    for (uint32_t o = i; o < no; o += gridDim.x * blockDim.x) fn(g.nbin + o);
+    for (uint32_t o = i0; o < no; o += stride) fn(g.nbin + o);
 }
 
 // words = 0: count only.  A handle beyond the bitmap (its size is the host's estimate) is reported: the host
@@ -1480,8 +1478,9 @@ __global__ __launch_bounds__(256) void k_rank_mark(Grid cur, const ReplicaDev *r
         if ((th.y >> 5) < words) atomicOr(&bits[th.y >> 5], 1u << (th.y & 31u));
         else info->beyond = 1u;
     });
-    for (int off = 32; off > 0; off >>= 1) live += __shfl_xor(live, off);
-    if (__lane_id() == 0 && live) atomicAdd(&info->live, live);
+    uint32_t total;
+    block_exclusive_scan(live, &total);
+    if (threadIdx.x == 0 && total) atomicAdd(&info->live, total);
     if (blockIdx.x == 0 && threadIdx.x == 0) info->handle_next = reps[r].handle_next;
 }
 

@@ -3,18 +3,22 @@
 // SimulationLoop.h:280-300 runs integrate -> NL -> reactions -> NL -> forces, and the forces of the
 // post-reaction state drive the next integration.  Here the state between two walks is x'(t), the
 // positions after step t's integration and before its reactions, and a step is
-//   k_step_begin    per-replica bookkeeping; clears the buffer the walk writes
 //   (bonded terms)  on x'(t); topology particles are never moved by reactions
 //   k_brick_step    one LDS-staged stencil walk over x'(t): the pair forces G (fixed point), the
 //                   reaction candidates of step t, and, optimistically, step t+1's Euler-Maruyama
-//                   move with G, re-binned into the other buffer
-//   k_resolve       step t's reactions on x'(t) (in place), listing every record it changes
-//   k_fix_sites     per changed record: lists the moved copies to withdraw (of killed and retyped
-//                   records, and of every surviving neighbour whose pair force with it changed) and
-//                   the records to move again (those neighbours, inserted and retyped records)
-//   k_fix_withdraw  withdraws the listed copies from the other buffer (found by handle)
+//                   move with G, re-binned into the next buffer; it also clears the cell counters
+//                   of the buffer after that
+//   k_resolve_step  the replicas' step counters; step t's reactions on x'(t) (in place), listing every
+//                   record they change (k_step_book does the counters when there are no reactions)
+//   k_fix_sites     per changed record: withdraws moved copies from the next buffer (of killed and
+//                   retyped records, and of every surviving neighbour whose pair force with it
+//                   changed) and lists the records to move again (those neighbours, inserted and
+//                   retyped records)
 //   k_fix_advance   forms each listed record's pair force afresh on the post-reaction state and
 //                   moves it again
+// A kernel boundary costs about 4.5 us whatever the kernel does, which is most of a small system's step:
+// hence the counters cleared two buffers ahead (four sets of counters take turns), the bookkeeping in the
+// resolve and the withdrawals in k_fix_sites.
 // A reaction changes the pair set only around the records it changes; every other record's G is
 // already the force of the post-reaction state, bit for bit (an integer sum of per-pair integers,
 // pair_fixed, over the same pairs), so its optimistic move stands, as the reference's order needs.
@@ -58,55 +62,73 @@ __device__ __forceinline__ uint32_t advance_particle(const Grid &nxt, const Repl
     return slot;
 }
 
-// Step t's bookkeeping before its walk: replicas with budget left take the step (Philox step t) and
-// integrate step t+1 in the same walk unless this is their last step or the launch's (last);
-// clears buffer `clear` (the walk's target; thread i its cell counters 4i .. 4i + 3), the change lists
-// and the bonded forces.
-// With topology reactions on, it also keeps each topology particle's slot in the buffer the walk reads
-// (loc_cur): the walk's moves point loc at the other buffer, and the topology reactions run after it.
-__global__ void k_step_begin(ReplicaDev *reps, uint32_t n_reps, int last, Grid clear, uint32_t n_cells,
-                             long long *fb, uint32_t n_fb, uint32_t *counters, unsigned long long *e_bonded,
-                             const uint32_t *loc, uint32_t *loc_cur, uint32_t n_loc) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n_loc) loc_cur[i] = loc[i];
-    if (i < n_reps) {
-        ReplicaDev &R = reps[i];
-        R.energy = 0ull;
-        e_bonded[i] = 0ull;
-        if (R.in_use && R.steps_left > 0) {
-            R.active = 1u;
-            R.step += 1u;
-            R.steps_left -= 1u;
-            R.steps_done += 1u;
-            R.integ = (R.steps_left > 0 && !last) ? 1u : 0u;
-        } else {
-            R.active = 0u;
-            R.integ = 0u;
-        }
-    }
-    const uint32_t c4 = 4u * i;  // the counters array starts 256-byte aligned (hipMalloc)
-    if (c4 + 3u < n_cells) reinterpret_cast<uint4 *>(clear.counts)[i] = make_uint4(0u, 0u, 0u, 0u);
-    else
-        for (uint32_t c = c4; c < n_cells; ++c) clear.counts[c] = 0u;
-    if (i < n_fb) fb[i] = 0;
-    if (i == 0) {
-        *clear.wl_count = 0u;
-        *clear.ovf_count = 0u;
-        counters[0] = 0u;  // changed records
-        counters[1] = 0u;  // records to move again
-        counters[2] = 0u;  // copies to withdraw
+// What step t's walk makes of a replica, from its counters before the step: take the step (active) with Philox
+// step R.step + 1, and integrate step t+1 in the same walk unless this is its last step or the launch's.  The
+// prologue takes no step and makes step 1's move.
+struct StepPlan {
+    bool active, integ;
+    uint32_t step, step_next;
+};
+constexpr int WALK_PROLOGUE = 1, WALK_LAST = 2;  // flags of a walk
+
+__device__ __forceinline__ StepPlan plan_step(const ReplicaDev &R, int flags) {
+    StepPlan p;
+    const uint64_t left = R.in_use ? R.steps_left : 0ull;
+    p.active = !(flags & WALK_PROLOGUE) && left > 0;
+    p.integ = (flags & WALK_PROLOGUE) ? left > 0 : (left > 1 && !(flags & WALK_LAST));
+    p.step = R.step + (p.active ? 1u : 0u);
+    p.step_next = p.step + 1u;
+    return p;
+}
+
+// the replica's counters after its walk of step t (one thread)
+__device__ __forceinline__ void book_step(ReplicaDev &R, int last) {
+    if (R.in_use && R.steps_left > 0) {
+        R.active = 1u;
+        R.step += 1u;
+        R.steps_left -= 1u;
+        R.steps_done += 1u;
+        R.integ = (R.steps_left > 0 && !last) ? 1u : 0u;
+    } else {
+        R.active = 0u;
+        R.integ = 0u;
     }
 }
 
-// clears a buffer and the bonded forces after a run (between runs only the current buffer holds
-// records, and the bonded forces are formed where they are consumed)
-__global__ void k_clear_grid(Grid g, uint32_t n_cells, long long *fb, uint32_t n_fb) {
+__global__ void k_step_book(ReplicaDev *reps, uint32_t n_reps, int last) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n_cells) g.counts[i] = 0u;
+    if (i < n_reps) book_step(reps[i], last);
+}
+
+// Engines with topologies only, before the bonded terms: clears the bonded forces and, with topology reactions
+// on, keeps each topology particle's slot in the buffer the walk reads (loc_cur): the walk's moves point loc at
+// the next buffer, and the topology reactions run after it.
+__global__ void k_topo_begin(long long *fb, uint32_t n_fb, const uint32_t *loc, uint32_t *loc_cur, uint32_t n_loc) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n_fb) fb[i] = 0;
-    if (i == 0) {
-        *g.wl_count = 0u;
-        *g.ovf_count = 0u;
+    if (i < n_loc) loc_cur[i] = loc[i];
+}
+
+// The counters of the brick's own cells in buffer `clear`, which becomes the target of the next step's walk.
+// hcn: the thread's halo cells (load_halo_counts).
+__device__ __forceinline__ void clear_own_cells(uint32_t *clear, const BrickDev &B, const Halo &Hs,
+                                                const HaloCounts &hcn) {
+    const uint32_t per = (Hs.nh + BRICK_THREADS - 1) / BRICK_THREADS, c0 = threadIdx.x * per;
+    auto own = [&](uint32_t hc) -> bool {
+        uint32_t hh[3];
+        Hs.decode(hc, hh[0], hh[1], hh[2]);
+        bool in = hc < Hs.nh;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) in = in && hh[a] - (uint32_t)B.h[a] < (uint32_t)B.e[a];
+        return in;
+    };
+    if (per <= STAGE_UNROLL) {
+#pragma unroll
+        for (uint32_t u = 0; u < STAGE_UNROLL; ++u)
+            if (u < per && own(c0 + u)) clear[hcn.cl[u]] = 0u;
+    } else {
+        for (uint32_t hc = c0; hc < c0 + per; ++hc)
+            if (own(hc)) clear[halo_global_cell(B, Hs, hc)] = 0u;
     }
 }
 
@@ -231,15 +253,16 @@ __device__ void order_inner_by_reach(const BrickSmem &m, uint32_t n_inner, const
 // The walk of one brick over cur = x'(t): the pair forces of the brick's own records (2^-32 fixed
 // point, summed in LDS per wave), step t's reaction candidates (order 1 and 2, the draws of
 // k_brick_search), and each particle moved to step t+1 (or copied) into nxt as soon as its force is
-// complete.  prologue: the first walk of a run (no candidates; moves replicas with steps left, Philox
-// step R.step + 1).  Replicas neither searching nor moving are copied without a walk.  Four waves per
+// complete.  flags: WALK_PROLOGUE, the first walk of a run (no candidates; moves replicas with steps
+// left, Philox step R.step + 1); WALK_LAST, the launch's last step.  Replicas neither searching nor moving are copied without a walk.  Four waves per
 // SIMD are asked of the register allocator (the move inside the walk loop would otherwise take the
 // kernel to three).
 template <bool AH>
 __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_brick_step(
-    Grid cur, Grid nxt, int prologue, ReplicaDev *reps, Tables T, Topo topo, const BrickDev *bricks, uint32_t brick0,
-    uint32_t cap, int radius, int handler, double dt, Event *events, uint32_t *ev_count, uint32_t max_states,
-    uint32_t max_halo, uint32_t smem_bytes, uint32_t *slow, uint32_t *err) {
+    Grid cur, Grid nxt, Grid clear, int flags, const ReplicaDev *reps, Tables T, Topo topo, const BrickDev *bricks,
+    uint32_t brick0, uint32_t cap, int radius, int handler, double dt, Event *events, uint32_t *ev_count,
+    uint32_t max_states, uint32_t max_halo, uint32_t smem_bytes, uint32_t *slow, uint32_t *change_counts,
+    uint32_t *err) {
     extern __shared__ __align__(16) char smem[];
     __shared__ ForceWave wave_lds[BRICK_WAVES];
     const bool staged_types = T.n_types <= MAX_STAGED_TYPES;
@@ -251,13 +274,20 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(4
     const Halo Hs = make_halo(B);
     const HaloCounts hcn = load_halo_counts(cur, B, Hs);
     const ReplicaDev &R = reps[B.r];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *nxt.wl_count = 0u;
+        *clear.ovf_count = 0u;
+        change_counts[0] = 0u;  // changed records
+        change_counts[1] = 0u;  // records to move again
+    }
+    clear_own_cells(clear.counts, B, Hs, hcn);
     if (!R.in_use) return;
     const RepGeom geo = load_geom(R);
-    const bool search = !prologue && R.active;                          // block-uniform
-    const bool integ = prologue ? (R.steps_left > 0) : (R.integ != 0u);  // block-uniform
-    const uint32_t step_next = R.step + 1u;
+    const StepPlan plan = plan_step(R, flags);  // block-uniform
+    const bool search = plan.active, integ = plan.integ;
+    const uint32_t step_next = plan.step_next;
     if (!search && !integ) {  // copy only: no forces needed
-        for_each_own_record(cur, B, geo, cap, [&](uint32_t s, const State &me) {
+        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (!(me.tw & TW_DEAD)) advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, false, me, 0, 0, 0, err);
         });
         return;
@@ -295,7 +325,7 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(4
     const float *reach_tab = o2_on ? st.reach : ft.reach;
     if (n_inner > BRICK_THREADS && 2 * n_inner <= transient_bytes(max_halo))  // block-uniform
         order_inner_by_reach(m, n_inner, reach_tab, nt, (uint16_t *)m.rings);
-    const uint32_t r = B.r, step = R.step;
+    const uint32_t r = B.r, step = plan.step;
     const uint64_t seed = R.seed;
     auto emit = [&](uint32_t rx, uint32_t s1, uint32_t s2, uint32_t h1, uint32_t h2, unsigned long long key) {
         uint32_t p = atomicAdd(&ev_count[r], 1u);
@@ -420,11 +450,11 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(4
     }
 }
 
-// the listed bricks of k_brick_step, neighbours read straight from the bins
-__global__ __launch_bounds__(BRICK_THREADS) void k_brick_step_slow(Grid cur, Grid nxt, int prologue, ReplicaDev *reps,
+// the listed bricks of a k_brick_step without candidates (a prologue, or a step without reactions), neighbours
+// read straight from the bins
+__global__ __launch_bounds__(BRICK_THREADS) void k_brick_step_slow(Grid cur, Grid nxt, int flags, ReplicaDev *reps,
                                                                    Tables T, Topo topo, const BrickDev *bricks,
-                                                                   uint32_t cap, int radius, int handler, double dt,
-                                                                   Event *events, uint32_t *ev_count, uint32_t *slow,
+                                                                   uint32_t cap, int radius, double dt, uint32_t *slow,
                                                                    uint32_t *err) {
     const uint32_t n = slow_count(slow);
     if (n == 0) return;  // grid-uniform
@@ -432,26 +462,23 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_step_slow(Grid cur, Gri
         const BrickDev B = bricks[slow[2 + i]];
         const ReplicaDev &R = reps[B.r];
         const RepGeom geo = load_geom(R);
-        const bool search = !prologue && R.active;
-        const bool integ = prologue ? (R.steps_left > 0) : (R.integ != 0u);
-        const uint32_t step_next = R.step + 1u;
-        for_each_own_record(cur, B, geo, cap, [&](uint32_t s, const State &me) {
+        const StepPlan plan = plan_step(R, flags);
+        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (me.tw & TW_DEAD) return;
             long long fx = 0, fy = 0, fz = 0, e = 0;
             if (!(me.tw & TW_OUTSIDE)) global_forces(cur, geo, cap, radius, T, s, me, fx, fy, fz, e);
-            if (search) search_one(cur, reps, T, cap, radius, handler, 0, events, ev_count, nullptr, 0, s, me, err);
-            advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, integ, me, fx, fy, fz, err);
+            advance_particle(nxt, R, geo, T, topo, cap, dt, plan.step_next, plan.integ, me, fx, fy, fz, err);
         });
     }
     release_slow_list(slow);
 }
 
-// A fused step's reactions (resolve_replica, one workgroup per replica), preceded by the replica's
+// A fused step's counters and reactions (resolve_replica, one workgroup per replica), preceded by the replica's
 // bricks that k_brick_step listed for the bin-reading path (their candidates join the replica's list
 // first).  The walk then needs no follow-up launch, which costs as much as a short kernel's work.
 __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid nxt, ReplicaDev *reps, Tables T,
                                                                   Topo topo, const BrickDev *bricks, uint32_t cap,
-                                                                  int radius, int handler, double dt,
+                                                                  int radius, int handler, double dt, int last,
                                                                   Event *events, uint32_t *ev_count, uint32_t *slow,
                                                                   unsigned long long *rx_step,
                                                                   unsigned long long *rx_total, uint32_t max_wl,
@@ -459,6 +486,8 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
                                                                   uint32_t edit_cap, RxRecord *recs,
                                                                   uint32_t *rec_count, uint32_t *err) {
     const uint32_t n = slow_count(slow);  // the same for every block: the walk has ended
+    if (threadIdx.x == 0) book_step(reps[blockIdx.x], last);
+    __syncthreads();
     for (uint32_t i = 0; i < n; ++i) {    // block-uniform
         const BrickDev B = bricks[slow[2 + i]];
         if (B.r != blockIdx.x) continue;
@@ -466,7 +495,7 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
         const RepGeom geo = load_geom(R);
         const bool integ = R.integ != 0u;
         const uint32_t step_next = R.step + 1u;
-        for_each_own_record(cur, B, geo, cap, [&](uint32_t s, const State &me) {
+        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (me.tw & TW_DEAD) return;
             long long fx = 0, fy = 0, fz = 0, e = 0;
             if (!(me.tw & TW_OUTSIDE)) global_forces(cur, geo, cap, radius, T, s, me, fx, fy, fz, e);
@@ -483,26 +512,41 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
     if (n) release_slow_list(slow);
 }
 
-// the cells of the (2r+1)^3 stencil of local cell cl, de-duplicated as axis_cells does, spread over
-// the lanes of a wave: fn(cell) for each cell of this lane
-template <class Fn>
-__device__ __forceinline__ void wave_stencil_cells(const RepGeom &geo, uint32_t cl, int radius, Fn &&fn) {
-    const int nz = geo.dims[2], ny = geo.dims[1];
-    const int iz = (int)(cl % (uint32_t)nz), iy = (int)((cl / (uint32_t)nz) % (uint32_t)ny);
-    const int ix = (int)(cl / ((uint32_t)nz * (uint32_t)ny));
-    const int nax = axis_count(ix, geo.dims[0], geo.pbc[0], radius);
-    const int nay = axis_count(iy, geo.dims[1], geo.pbc[1], radius);
-    const int naz = axis_count(iz, geo.dims[2], geo.pbc[2], radius);
-    const uint32_t ncell = (uint32_t)(nax * nay * naz);
-    for (uint32_t c = __lane_id(); c < ncell; c += 64) {
-        const int a = (int)(c / (uint32_t)(nay * naz)), rem = (int)(c % (uint32_t)(nay * naz));
-        const int b = rem / naz, cc = rem % naz;
-        fn(geo.cell_base +
-           ((uint32_t)axis_elem(a, ix, geo.dims[0], geo.pbc[0], radius) * (uint32_t)ny +
-            (uint32_t)axis_elem(b, iy, geo.dims[1], geo.pbc[1], radius)) *
-               (uint32_t)nz +
-           (uint32_t)axis_elem(cc, iz, geo.dims[2], geo.pbc[2], radius));
+// the cells of the (2r+1)^3 stencil of local cell cl, de-duplicated as axis_cells does
+struct StencilDims {
+    int i[3], na[3];
+    uint32_t n;
+};
+
+__device__ __forceinline__ StencilDims stencil_dims(const RepGeom &geo, uint32_t cl, int radius) {
+    const uint32_t nz = (uint32_t)geo.dims[2], ny = (uint32_t)geo.dims[1];
+    StencilDims d;
+    d.i[2] = (int)(cl % nz);
+    d.i[1] = (int)((cl / nz) % ny);
+    d.i[0] = (int)(cl / (nz * ny));
+    d.n = 1;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        d.na[a] = axis_count(d.i[a], geo.dims[a], geo.pbc[a], radius);
+        d.n *= (uint32_t)d.na[a];
     }
+    return d;
+}
+
+__device__ __forceinline__ uint32_t stencil_cell(const RepGeom &geo, const StencilDims &d, uint32_t c, int radius) {
+    const int yz = d.na[1] * d.na[2], a = (int)c / yz, rem = (int)c % yz, b = rem / d.na[2], k = rem % d.na[2];
+    return geo.cell_base + ((uint32_t)axis_elem(a, d.i[0], geo.dims[0], geo.pbc[0], radius) * (uint32_t)geo.dims[1] +
+                            (uint32_t)axis_elem(b, d.i[1], geo.dims[1], geo.pbc[1], radius)) *
+                               (uint32_t)geo.dims[2] +
+           (uint32_t)axis_elem(k, d.i[2], geo.dims[2], geo.pbc[2], radius);
+}
+
+// fn(cell) for every `lanes`-th cell of the stencil from cell `first` on
+template <class Fn>
+__device__ __forceinline__ void stencil_cells(const RepGeom &geo, uint32_t cl, int radius, uint32_t first,
+                                              uint32_t lanes, Fn &&fn) {
+    const StencilDims d = stencil_dims(geo, cl, radius);
+    for (uint32_t c = first; c < d.n; c += lanes) fn(stencil_cell(geo, d, c, radius));
 }
 
 // fn(slot) for every record of one cell of buffer g (overflow records included)
@@ -519,6 +563,79 @@ __device__ __forceinline__ void cell_records(const Grid &g, uint32_t cap, uint32
     }
 }
 
+// fn(slot, record) for every record of one cell, four records loaded together (a cell's records are one
+// round trip instead of one each)
+template <class Fn>
+__device__ __forceinline__ void cell_records4(const Grid &g, uint32_t cap, uint32_t cell, Fn &&fn) {
+    const uint32_t cnt = g.counts[cell];
+    const uint32_t mm = cnt < cap ? cnt : cap;
+    for (uint32_t q = 0; q < mm; q += 4) {
+        State o[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            if (q + u < mm) o[u] = g.bins[cell * cap + q + u];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            if (q + u < mm) fn(cell * cap + q + u, o[u]);
+    }
+    if (cnt > cap) {  // rare: a crowded cell spilled into the overflow region
+        uint32_t no = *g.ovf_count;
+        no = no < g.ovf_cap ? no : g.ovf_cap;
+        for (uint32_t o = 0; o < no; ++o)
+            if (g.ovf_cell[o] == cell) fn(g.nbin + o, g.bins[g.nbin + o]);
+    }
+}
+
+// Withdraws the moved copies of the wave's pending records from nxt: lanes with `has` name a record (its slot in
+// cur and the handle its copy carries).  Two records at a time, half a wave each, its lanes spread over the
+// cells around the record's cell; a copy that moved further than one cell is searched by the whole wave, at
+// last in the replica's whole grid.
+__device__ __forceinline__ void withdraw_copies(const Grid &cur, const Grid &nxt, const ReplicaDev &R,
+                                                const RepGeom &geo, uint32_t cap, bool has, uint32_t slot,
+                                                uint32_t handle) {
+    const uint32_t lane = __lane_id();
+    unsigned long long pending = __ballot(has);
+    while (pending) {
+        const int l0 = __ffsll((long long)pending) - 1;
+        pending &= pending - 1ull;
+        const int l1 = pending ? __ffsll((long long)pending) - 1 : -1;
+        if (pending) pending &= pending - 1ull;
+        const int src = lane < 32 ? l0 : l1;
+        const uint32_t s = (uint32_t)__shfl((int)slot, src < 0 ? l0 : src);
+        const uint32_t h = (uint32_t)__shfl((int)handle, src < 0 ? l0 : src);
+        const uint32_t cl = cell_of_slot(cur, s, cap) - geo.cell_base;
+        bool found = false;
+        auto probe = [&](uint32_t cell) {
+            cell_records4(nxt, cap, cell, [&](uint32_t s2, const State &o) {
+                if (o.h == h && !(o.tw & TW_DEAD)) {
+                    nxt.bins[s2].tw = o.tw | TW_DEAD;
+                    found = true;
+                }
+            });
+        };
+        if (src >= 0) stencil_cells(geo, cl, 1, lane & 31u, 32u, probe);
+        const unsigned long long f = __ballot(found);
+        for (int half = 0; half < 2; ++half) {  // wave-uniform
+            if ((f >> (32 * half)) & 0xFFFFFFFFull) continue;
+            const int l = half ? l1 : l0;
+            if (l < 0) continue;
+            const uint32_t sw = (uint32_t)__shfl((int)slot, l), hw = (uint32_t)__shfl((int)handle, l);
+            bool hit = false;
+            auto far = [&](uint32_t cell) {
+                cell_records4(nxt, cap, cell, [&](uint32_t s2, const State &o) {
+                    if (o.h == hw && !(o.tw & TW_DEAD)) {
+                        nxt.bins[s2].tw = o.tw | TW_DEAD;
+                        hit = true;
+                    }
+                });
+            };
+            stencil_cells(geo, cell_of_slot(cur, sw, cap) - geo.cell_base, 2, lane, 64u, far);
+            if (__ballot(hit)) continue;
+            for (uint32_t c = lane; c < R.n_cells; c += 64) far(geo.cell_base + c);
+        }
+    }
+}
+
 // Per changed record of step t's reactions, one wave each, its lanes spread over the record's
 // stencil cells; cur is x'(t) with the reactions applied, nxt holds the walk's optimistic moves.
 //   killed k:   its moved copy is withdrawn;
@@ -526,12 +643,13 @@ __device__ __forceinline__ void cell_records(const Grid &g, uint32_t cap, uint32
 //   retyped r:  its moved copy (under its old handle) is withdrawn and r is listed;
 // and, when the replica moves this step, every surviving old neighbour n (a live record without
 // TW_NEW) whose pair force from the changed record differs between before and after is listed
-// once (bit in aff_bits) for a fresh force and a new move, its moved copy withdrawn.
-__global__ __launch_bounds__(256) void k_fix_sites(Grid cur, const ReplicaDev *reps, Tables T, uint32_t cap,
+// once (bit in aff_bits) for a fresh force and a new move, its moved copy withdrawn.  Nothing is
+// inserted into nxt before every withdrawal is done (k_fix_advance), so the records below each
+// cell's count are stable while they are searched.
+__global__ __launch_bounds__(256) void k_fix_sites(Grid cur, Grid nxt, const ReplicaDev *reps, Tables T, uint32_t cap,
                                                    int radius, const Edit *edits, const uint32_t *edit_count,
                                                    uint32_t edit_cap, uint32_t *aff_bits, uint32_t *aff_list,
-                                                   uint32_t *aff_count, uint32_t aff_cap, uint2 *wd_list,
-                                                   uint32_t *wd_count, uint32_t wd_cap, uint32_t *err) {
+                                                   uint32_t *aff_count, uint32_t aff_cap, uint32_t *err) {
     const uint32_t lane = __lane_id();
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
@@ -543,81 +661,69 @@ __global__ __launch_bounds__(256) void k_fix_sites(Grid cur, const ReplicaDev *r
         if (p < aff_cap) aff_list[p] = s;
         else atomicAdd(&err[ERR_EDIT_OVERFLOW], 1u);
     };
-    auto withdraw = [&](uint32_t s, uint32_t h) {
-        const uint32_t p = atomicAdd(wd_count, 1u);
-        if (p < wd_cap) wd_list[p] = make_uint2(s, h);
-        else atomicAdd(&err[ERR_EDIT_OVERFLOW], 1u);
-    };
     for (uint32_t k = wave; k < n_edit; k += n_waves) {  // wave-uniform
         const Edit ed = edits[k];
         const uint32_t kind = ed.info & 3u, t_old = ed.info >> 2;
         const uint32_t slot = ed.slot;
         const ReplicaDev &R = reps[ed.r];
         const State st = cur.bins[slot];
-        if (lane == 0) {
-            if (kind == EDIT_KILLED) withdraw(slot, st.h);
-            if (kind == EDIT_RETYPED) withdraw(slot, ed.pad);  // the copy carries the old handle
-            if (kind != EDIT_KILLED) list(slot);
-        }
+        const RepGeom geo = load_geom(R);
+        if (lane == 0 && kind != EDIT_KILLED) list(slot);
+        // the copy carries the handle the record had
+        withdraw_copies(cur, nxt, R, geo, cap, lane == 0 && kind != EDIT_INSERTED, slot,
+                        kind == EDIT_RETYPED ? ed.pad : st.h);
         if (!R.integ || (st.tw & TW_OUTSIDE)) continue;  // copies only, or no neighbours
-        const RepGeom geo = load_geom(R);
         const uint32_t ts = tw_type(st.tw);
-        wave_stencil_cells(geo, cell_of_slot(cur, slot, cap) - geo.cell_base, radius, [&](uint32_t cell) {
-            cell_records(cur, cap, cell, [&](uint32_t s2) {
-                if (s2 == slot) return;
-                const State n = cur.bins[s2];
-                if (n.tw & (TW_DEAD | TW_OUTSIDE | TW_NEW)) return;
-                const uint32_t tn = tw_type(n.tw);
-                // the pair seen from n: x = site - n
-                const double dx = min_image(st.x - n.x, geo.box[0], geo.pbc[0]);
-                const double dy = min_image(st.y - n.y, geo.box[1], geo.pbc[1]);
-                const double dz = min_image(st.z - n.z, geo.box[2], geo.pbc[2]);
-                const double d2 = dist2(dx, dy, dz);
-                long long ax, ay, az, bx = 0, by = 0, bz = 0, pe;
-                pair_fixed<false>(T.pots, T.pidx[tn * nt + ts], dx, dy, dz, d2, ax, ay, az, pe);
-                if (kind == EDIT_RETYPED)
-                    pair_fixed<false>(T.pots, T.pidx[tn * nt + t_old], dx, dy, dz, d2, bx, by, bz, pe);
-                if (((ax - bx) | (ay - by) | (az - bz)) == 0) return;  // n's sum is unchanged
-                const uint32_t bit = 1u << (s2 & 31u);
-                if (atomicOr(&aff_bits[s2 >> 5], bit) & bit) return;  // listed by another site
-                list(s2);
-                withdraw(s2, n.h);
-            });
-        });
-    }
-}
-
-// Withdraws the listed moved copies from nxt: the live record of the listed handle, searched in the
-// cells around the record's cell (one wave each; a move longer than one cell widens the search,
-// up to the replica's whole grid)
-__global__ __launch_bounds__(256) void k_fix_withdraw(Grid cur, Grid nxt, const ReplicaDev *reps, uint32_t cap,
-                                                      const uint2 *wd_list, const uint32_t *wd_count,
-                                                      uint32_t wd_cap) {
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
-    uint32_t n = *wd_count;
-    n = n < wd_cap ? n : wd_cap;
-    for (uint32_t k = wave; k < n; k += n_waves) {  // wave-uniform
-        const uint2 w = wd_list[k];
-        const State st = cur.bins[w.x];
-        const ReplicaDev &R = reps[tw_replica(st.tw)];
-        const RepGeom geo = load_geom(R);
-        const uint32_t cl = cell_of_slot(cur, w.x, cap) - geo.cell_base;
-        bool found = false;
-        auto probe = [&](uint32_t cell) {
-            cell_records(nxt, cap, cell, [&](uint32_t s2) {
-                const State o = nxt.bins[s2];
-                if (o.h == w.y && !(o.tw & TW_DEAD)) {
-                    nxt.bins[s2].tw = o.tw | TW_DEAD;
-                    found = true;
-                }
-            });
+        // true when n's pair force changed and no other site has listed it
+        auto affected = [&](uint32_t s2, const State &n) -> bool {
+            if (s2 == slot || (n.tw & (TW_DEAD | TW_OUTSIDE | TW_NEW))) return false;
+            const uint32_t tn = tw_type(n.tw);
+            // the pair seen from n: x = site - n
+            const double dx = min_image(st.x - n.x, geo.box[0], geo.pbc[0]);
+            const double dy = min_image(st.y - n.y, geo.box[1], geo.pbc[1]);
+            const double dz = min_image(st.z - n.z, geo.box[2], geo.pbc[2]);
+            const double d2 = dist2(dx, dy, dz);
+            long long ax, ay, az, bx = 0, by = 0, bz = 0, pe;
+            pair_fixed<false>(T.pots, T.pidx[tn * nt + ts], dx, dy, dz, d2, ax, ay, az, pe);
+            if (kind == EDIT_RETYPED)
+                pair_fixed<false>(T.pots, T.pidx[tn * nt + t_old], dx, dy, dz, d2, bx, by, bz, pe);
+            if (((ax - bx) | (ay - by) | (az - bz)) == 0) return false;  // n's sum is unchanged
+            const uint32_t bit = 1u << (s2 & 31u);
+            return !(atomicOr(&aff_bits[s2 >> 5], bit) & bit);
         };
-        wave_stencil_cells(geo, cl, 1, probe);
-        if (__ballot(found)) continue;
-        wave_stencil_cells(geo, cl, 2, probe);
-        if (__ballot(found)) continue;
-        for (uint32_t c = __lane_id(); c < R.n_cells; c += 64) probe(geo.cell_base + c);
+        const uint32_t cl = cell_of_slot(cur, slot, cap) - geo.cell_base;
+        const StencilDims sd = stencil_dims(geo, cl, radius);
+        for (uint32_t c0 = 0; c0 < sd.n; c0 += 64) {  // wave-uniform
+            const bool mine = c0 + lane < sd.n;
+            const uint32_t cell = mine ? stencil_cell(geo, sd, c0 + lane, radius) : 0u;
+            const uint32_t cnt = mine ? cur.counts[cell] : 0u, mm = cnt < cap ? cnt : cap;
+            for (uint32_t q = 0; __ballot(q < mm); q += 4) {
+                State o[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u)
+                    if (q + u < mm) o[u] = cur.bins[cell * cap + q + u];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) {
+                    const uint32_t s2 = cell * cap + q + u;
+                    const bool hit = q + u < mm && affected(s2, o[u]);
+                    if (hit) list(s2);
+                    withdraw_copies(cur, nxt, R, geo, cap, hit, s2, hit ? o[u].h : 0u);
+                }
+            }
+            if (__ballot(cnt > cap)) {  // rare: crowded cells spilled into the overflow region
+                uint32_t no = *cur.ovf_count;
+                no = no < cur.ovf_cap ? no : cur.ovf_cap;
+                for (uint32_t v = 0; v < no; ++v) {
+                    const uint32_t s2 = cur.nbin + v;
+                    const bool in = cnt > cap && cur.ovf_cell[v] == cell;
+                    State n{};
+                    if (in) n = cur.bins[s2];
+                    const bool hit = in && affected(s2, n);
+                    if (hit) list(s2);
+                    withdraw_copies(cur, nxt, R, geo, cap, hit, s2, n.h);
+                }
+            }
+        }
     }
 }
 
@@ -643,10 +749,9 @@ __global__ __launch_bounds__(256) void k_fix_advance(Grid cur, Grid nxt, const R
         long long fx = 0, fy = 0, fz = 0;
         if (integ && !(me.tw & TW_OUTSIDE)) {
             const uint32_t t = tw_type(me.tw);
-            wave_stencil_cells(geo, cell_of_slot(cur, s, cap) - geo.cell_base, radius, [&](uint32_t cell) {
-                cell_records(cur, cap, cell, [&](uint32_t s2) {
+            stencil_cells(geo, cell_of_slot(cur, s, cap) - geo.cell_base, radius, lane, 64u, [&](uint32_t cell) {
+                cell_records4(cur, cap, cell, [&](uint32_t s2, const State &o) {
                     if (s2 == s) return;
-                    const State o = cur.bins[s2];
                     if (o.tw & (TW_DEAD | TW_OUTSIDE)) return;
                     // CPUCalculateForces.cpp:226-259: x = shortestDifference(x_i, x_j)
                     const double dx = min_image(o.x - me.x, geo.box[0], geo.pbc[0]);
