@@ -9,12 +9,16 @@
 // is farther than the cutoff by more than the FP32 rounding bound, so the exact pair set is
 // unchanged.  The exact work (FP64 min-image displacement, the reference gate d2 < rc^2, the pair
 // math, the reaction draws) runs on the survivors only, and not per lane: each wave streams its
-// survivors through a ring in LDS and evaluates them 64 at a time with every lane busy, because a
+// survivors through rings in LDS and evaluates them 64 at a time with every lane busy, because a
 // per-lane evaluation would make the whole wave execute the exact branch whenever any one lane
 // had a survivor (almost always).  Forces are gathered per particle as 64-bit fixed-point sums
 // (LDS atomics; integer addition is order-free, so the result stays deterministic).
 // A brick whose halo holds more particles than the LDS budget takes a slow path that reads
 // neighbours straight from the bins.
+//
+// Four consecutive records of one z-row of cells share a quad of lanes and their candidates: the quad
+// walks the rows of cells around them four candidates at a time, and the matrix cores form the 4 x 4
+// squared distances (mfma_pipeline).
 //
 // Per axis a brick is either in halo mode (extent e, halo r on both sides; the axis has at least 2r + 1
 // cells when it is periodic, so the cells of a stencil are distinct; when e + 2r exceeds the axis, halo
@@ -48,8 +52,14 @@ static_assert(sizeof(BrickDev) == 80, "brick record size");
 
 constexpr int BRICK_THREADS = 256;
 constexpr int BRICK_WAVES = BRICK_THREADS / 64;
-constexpr uint32_t BATCH = 4;       // candidates a lane takes from its current run per iteration
-constexpr uint32_t RING = 512;      // per-wave ring of prefilter survivors (power of two, >= 63 + 64 * BATCH)
+constexpr uint32_t BATCH = 2;       // candidates a lane takes from its current run per iteration (general walk)
+constexpr uint32_t RING = 256;      // per-wave ring of its survivors (power of two, >= 63 + 64 * BATCH)
+constexpr uint32_t QRING = 128;     // per-wave ring of harvested pairs of the matrix-core walk
+constexpr uint32_t ORING = 128;     // and of its sifted pairs (>= 63 + 64)
+constexpr uint32_t QSTEPS = 8;      // its steps between two harvests: 8 x 4 result bits fill a word
+constexpr size_t WAVE_RING_BYTES = 4 * QRING + 4 * ORING + 2 * 16 * QSTEPS;  // two rings and the steps' candidates
+static_assert(WAVE_RING_BYTES >= 4 * RING, "or the general walk's ring");
+constexpr float FAR_POS = 1.0e18f, FAR_SQ = 1.0e36f;  // a record that is no neighbour lies here
 constexpr uint32_t NO_ENTRY = 0xFFFFFFFFu;  // an idle lane's entry in the last batch of the ring
 
 __host__ __device__ inline uint32_t div_magic(uint32_t d) {
@@ -80,45 +90,60 @@ __device__ __forceinline__ Halo make_halo(const BrickDev &B) {
 }
 
 struct BrickSmem {  // carved out of dynamic LDS
-    float4 *P;         // [max_states] local-frame FP32 position, w = tw bits
+    float4 *P;         // [max_states + 1] local-frame FP32 position, w = its square; the last one is far away
     uint32_t *slot;    // [max_states] bin slot (the FP64 record is read from the bins when needed)
-    uint32_t *hstart;  // [max_halo + 1]
+    uint16_t *hstart;  // [max_halo + 1] (at most 60000 records are staged)
     uint16_t *hc_of;   // [max_states]
-    uint16_t *inner;   // [max_states]
-    // transient: the halo cells' counters and ids while staging, then the waves' survivor rings
-    uint32_t *hcnt;    // [max_halo]
-    uint32_t *hcell;   // [max_halo]
-    uint32_t *rings;   // [BRICK_WAVES][RING]
+    uint8_t *typ;      // [max_states] species (below MAX_STAGED_TYPES), TYP_OUTSIDE, TYP_DEAD
+    char *rings;       // [BRICK_WAVES][WAVE_RING_BYTES]
+    uint32_t far;      // index of the far record
 };
-
-__host__ __device__ inline size_t transient_bytes(uint32_t max_halo) {
-    const size_t staging = 8 * (size_t)max_halo, rings = 4 * (size_t)BRICK_WAVES * RING;
-    return staging > rings ? staging : rings;
-}
+constexpr uint8_t TYP_OUTSIDE = 0x40, TYP_DEAD = 0x80, TYP_MASK = 0x0F;
 
 __device__ __forceinline__ BrickSmem carve(char *base, uint32_t max_states, uint32_t max_halo) {
     BrickSmem m;
     char *p = base;
     m.P = (float4 *)p;
-    p += sizeof(float4) * max_states;
+    p += sizeof(float4) * (max_states + 1);
     m.slot = (uint32_t *)p;
     p += 4 * max_states;
-    m.hstart = (uint32_t *)p;
-    p += 4 * (max_halo + 1);
+    m.hstart = (uint16_t *)p;
+    p += 2 * (max_halo + 1);
     m.hc_of = (uint16_t *)p;
     p += 2 * max_states;
-    m.inner = (uint16_t *)p;
-    p += 2 * max_states;
+    m.typ = (uint8_t *)p;
+    p += max_states;
     p = base + ((p - base + 15) & ~(ptrdiff_t)15);
-    m.hcnt = (uint32_t *)p;
-    m.hcell = m.hcnt + max_halo;
-    m.rings = (uint32_t *)p;
+    m.rings = p;
+    m.far = max_states;
     return m;
 }
 
 __host__ __device__ inline size_t brick_smem_bytes(uint32_t max_states, uint32_t max_halo) {
-    const size_t fixed = (sizeof(float4) + 4 + 2 + 2) * (size_t)max_states + 4 * ((size_t)max_halo + 1);
-    return ((fixed + 15) & ~(size_t)15) + transient_bytes(max_halo);
+    const size_t fixed = sizeof(float4) * ((size_t)max_states + 1) + (4 + 2 + 1) * (size_t)max_states +
+                         2 * ((size_t)max_halo + 1);
+    return ((fixed + 15) & ~(size_t)15) + BRICK_WAVES * WAVE_RING_BYTES;
+}
+
+// Kernel arguments and records that a kernel only reads, through the constant address space: they come in
+// scalar loads, and laundering the pointer makes a part of a kernel load what it needs where it needs it.  (Kept in
+// registers from the start, a walk's arguments, geometry and tables exceed the scalar registers: 1441 of the 5976
+// vector instructions of k_brick_step moved spilled ones.)
+template <class T>
+__device__ __forceinline__ const T &read_only(const T *p) {
+    typedef const __attribute__((address_space(4))) T *C;
+    C c = (C)p;
+    asm volatile("" : "+s"(c));
+    return *(const T *)c;
+}
+
+// the kernel's arguments: its one by-value argument, the first of the kernarg segment
+template <class T>
+__device__ __forceinline__ const T &kernel_args() {
+    typedef const __attribute__((address_space(4))) T *C;
+    C c = (C)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(c));
+    return *(const T *)c;
 }
 
 struct Frame {       // local frame of a brick
@@ -126,6 +151,7 @@ struct Frame {       // local frame of a brick
     float L[3];      // box lengths (FP32) for whole-axis min image
     uint32_t whole;
     float margin;    // 16 * 2^-23 * largest local coordinate (FP32 rounding bound, 4x safety)
+    float expand;    // bound on the rounding of |a|^2 + |b|^2 - 2 ab against |a - b|^2 (mfma_pipeline)
 };
 
 __device__ __forceinline__ Frame make_frame(const BrickDev &B, const RepGeom &geo) {
@@ -141,6 +167,9 @@ __device__ __forceinline__ Frame make_frame(const BrickDev &B, const RepGeom &ge
     }
     f.whole = B.whole;
     f.margin = 16.0f * M * 1.1920929e-07f;
+    // |p|^2 <= 3 M^2 = S for every local position p.  With u = 2^-24: the squares carry 3 u S each, each of the
+    // four accumulations rounds a partial sum of at most 4 S, each product at most 2 S: below 40 u S = 2.4e-6 S
+    f.expand = 3.0e-5f * M * M;
     return f;
 }
 
@@ -149,210 +178,232 @@ __device__ __forceinline__ float prefilter_thr(float cut2_f, bool any, float mar
     return any ? cut2_f * (1.0f + 3.0e-6f) + 2.0f * sqrtf(cut2_f) * margin + margin * margin : -1.0f;
 }
 
-// the global cell of halo cell hc of brick B (periodic images wrapped), UINT32_MAX outside a
-// non-periodic edge; from the brick record alone
-__device__ __forceinline__ uint32_t halo_global_cell(const BrickDev &B, const Halo &Hs, uint32_t hc) {
-    uint32_t hh[3];
-    Hs.decode(hc, hh[0], hh[1], hh[2]);
-    int32_t c[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        int32_t x = B.o[a] - B.h[a] + (int32_t)hh[a];
-        if (x < 0 || x >= B.dims[a]) {
-            if (!(B.pbc & (1u << a))) return 0xFFFFFFFFu;
-            x = x < 0 ? x + B.dims[a] : x - B.dims[a];  // |overhang| <= r < dims
-        }
-        c[a] = x;
-    }
-    return B.cell_base + ((uint32_t)c[0] * (uint32_t)B.dims[1] + (uint32_t)c[1]) * (uint32_t)B.dims[2] + (uint32_t)c[2];
-}
+// Staging a brick.  A thread owns a chunk of consecutive halo cells: it reads their counters (one global round
+// trip, issued from the brick record alone, so that they travel with the replica's record), and a block scan
+// places every cell's records: their bin slots are listed in LDS.  Then the records are dealt out evenly over
+// the threads (the second round trip).  (Requesting a chunk's records before the scan saved a tenth of the
+// staging's latency, and its idle slots cost more instructions than that.)
+constexpr uint32_t STAGE_CELLS = 4;   // cells of a thread at a time
+constexpr uint32_t STAGE_UNROLL = 4;  // records of a thread in flight
 
-// Staging a brick: the counters of each thread's contiguous chunk of halo cells (one global round
-// trip, issued from the brick record alone, so that they travel with the replica's record), one
-// block scan that places every halo cell's records and lists the brick's own (inner) records, then
-// the records themselves, spread evenly over the threads (the second round trip).
-constexpr uint32_t STAGE_UNROLL = 4;  // loads of one thread in flight together
-
-struct HaloCounts {  // this thread's chunk of halo cells (registers): global cell and counter
-    uint32_t cl[STAGE_UNROLL], n[STAGE_UNROLL];
+struct HaloCells {  // a thread's cells (registers): global cell and records
+    uint32_t cl[STAGE_CELLS], n[STAGE_CELLS];
 };
 
-// chunk of thread tid: halo cells tid * per .. tid * per + per - 1 (per <= STAGE_UNROLL; larger halos
-// load their counters inside stage_brick)
-__device__ __forceinline__ HaloCounts load_halo_counts(const Grid &g, const BrickDev &B, const Halo &Hs) {
-    HaloCounts h;
-    const uint32_t nh = Hs.nh, per = (nh + BRICK_THREADS - 1) / BRICK_THREADS, c0 = threadIdx.x * per;
+__device__ __forceinline__ uint32_t cells_per_thread(const Halo &Hs) { return (Hs.nh + BRICK_THREADS - 1) / BRICK_THREADS; }
+
+// halo cells c0 .. c0 + count - 1 (count <= STAGE_CELLS); clear: the counters of the brick's own cells among them are
+// cleared in this buffer (null: none)
+__device__ __forceinline__ HaloCells load_halo_cells(const uint32_t *counts, uint32_t *clear, const BrickDev &B,
+                                                     const Halo &Hs, uint32_t c0, uint32_t count) {
+    HaloCells h;
+    uint32_t hh[3];
+    Hs.decode(c0, hh[0], hh[1], hh[2]);
 #pragma unroll
-    for (uint32_t u = 0; u < STAGE_UNROLL; ++u) {
-        h.cl[u] = 0xFFFFFFFFu;
-        h.n[u] = 0;
-        if (per <= STAGE_UNROLL && u < per && c0 + u < nh) {
-            h.cl[u] = halo_global_cell(B, Hs, c0 + u);
-            if (h.cl[u] != 0xFFFFFFFFu) h.n[u] = g.counts[h.cl[u]];
+    for (uint32_t u = 0; u < STAGE_CELLS; ++u) {
+        h.cl[u] = h.n[u] = 0;
+        if (u < count && c0 + u < Hs.nh) {
+            int32_t c[3];
+            bool own = true, valid = true;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const int32_t x = B.o[a] - B.h[a] + (int32_t)hh[a];
+                const bool lo = x < 0, hi = x >= B.dims[a];  // |overhang| <= r < dims
+                valid = valid && ((B.pbc >> a & 1u) || !(lo || hi));
+                c[a] = x + (lo ? B.dims[a] : 0) - (hi ? B.dims[a] : 0);
+                own = own && hh[a] - (uint32_t)B.h[a] < (uint32_t)B.e[a];
+            }
+            const uint32_t cl =
+                B.cell_base + ((uint32_t)c[0] * (uint32_t)B.dims[1] + (uint32_t)c[1]) * (uint32_t)B.dims[2] + (uint32_t)c[2];
+            if (valid) {
+                h.cl[u] = cl;
+                h.n[u] = counts[cl];
+            }
+            if (clear && own) clear[cl] = 0u;
+        }
+        if (++hh[2] == Hs.H2) {
+            hh[2] = 0;
+            if (++hh[1] == Hs.H1) {
+                hh[1] = 0;
+                ++hh[0];
+            }
         }
     }
     return h;
 }
 
-// inclusive-exclusive pair scan: the exclusive prefixes of a and b over the block and their totals
-// (two values, one pair of barriers)
-__device__ __forceinline__ uint2 block_exclusive_scan2(uint32_t a, uint32_t b, uint2 *total) {
-    __shared__ uint2 wave_sums[BRICK_WAVES];
-    const uint32_t lane = __lane_id(), wid = threadIdx.x / 64;
-    uint32_t x = a, y = b;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t xa = __shfl_up(x, off), ya = __shfl_up(y, off);
-        if (lane >= (uint32_t)off) {
-            x += xa;
-            y += ya;
-        }
-    }
-    if (lane == 63) wave_sums[wid] = make_uint2(x, y);
-    __syncthreads();
-    uint2 base = make_uint2(0u, 0u), tot = make_uint2(0u, 0u);
-#pragma unroll
-    for (uint32_t w = 0; w < BRICK_WAVES; ++w) {
-        const uint2 ws = wave_sums[w];
-        if (w < wid) {
-            base.x += ws.x;
-            base.y += ws.y;
-        }
-        tot.x += ws.x;
-        tot.y += ws.y;
-    }
-    __syncthreads();
-    *total = tot;
-    return make_uint2(base.x + x - a, base.y + y - b);
+// inclusive sum over the lanes of a wave (DPP row shifts and row broadcasts: no LDS round trips)
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);  // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);  // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);  // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);  // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// err[STAT_FULL_BRICKS]: the bricks whose halo holds more than max_states records (a wave each)
+__global__ void __launch_bounds__(BRICK_THREADS) k_brick_fill(const uint32_t *counts, const BrickDev *bricks, uint32_t nb,
+                                                              uint32_t max_states, uint32_t *err) {
+    const uint32_t b = blockIdx.x * BRICK_WAVES + threadIdx.x / 64;
+    if (b >= nb) return;
+    const BrickDev &B = bricks[b];
+    const Halo Hs = make_halo(B);
+    uint32_t sum = 0;
+    for (uint32_t c = __lane_id(); c < Hs.nh; c += 64) sum += load_halo_cells(counts, nullptr, B, Hs, c, 1).n[0];
+    sum = wave_inclusive_sum(sum);
+    if (__lane_id() == 63 && sum > max_states) atomicAdd(&err[STAT_FULL_BRICKS], 1u);
 }
 
 // stages buffer g around brick B into LDS; returns the number of staged records, or UINT32_MAX if
-// they do not fit (the caller then takes the slow path).  Also returns the number of inner records
-// (the brick's own cells), listed in m.inner in halo order.  hc: load_halo_counts of this brick.
-__device__ uint32_t stage_brick(const Grid &g, const BrickDev &B, const RepGeom &geo, const Frame &F, uint32_t cap,
-                                const BrickSmem &m, uint32_t max_states, const Halo &Hs, const HaloCounts &hcn,
-                                uint32_t *n_inner_out) {
-    __shared__ uint32_t s_total, s_inner;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t nh = Hs.nh;
-    const uint32_t per = (nh + BRICK_THREADS - 1) / BRICK_THREADS;
-    const uint32_t c0 = tid * per;
-    // a halo cell is inner when every coordinate lies in the brick's own range
-    auto inner_cell = [&](uint32_t hc) -> bool {
-        uint32_t hh[3];
-        Hs.decode(hc, hh[0], hh[1], hh[2]);
-        bool in = true;
+// they do not fit (the caller then takes the slow path).  h: load_halo_cells of the thread's cells
+// (only used when a thread has at most STAGE_CELLS).
+__device__ __forceinline__ uint32_t stage_brick(const Grid &g, const BrickDev &B, const RepGeom &geo, const Frame &F, uint32_t cap,
+                                const BrickSmem &m, uint32_t max_states, const Halo &Hs, HaloCells h) {
+    __shared__ uint32_t wave_sums[BRICK_WAVES];
+    const uint32_t tid = threadIdx.x, nh = Hs.nh, per = cells_per_thread(Hs), c0 = tid * per;
+    uint32_t off = 0, total = 0;
+    auto place = [&](uint32_t sum) {  // off = records before this thread's, total = all
+        const uint32_t incl = wave_inclusive_sum(sum), wid = tid / 64;
+        if (__lane_id() == 63) wave_sums[wid] = incl;
+        __syncthreads();
+        off = incl - sum;
+        total = 0;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) in = in && hh[a] >= (uint32_t)B.h[a] && hh[a] < (uint32_t)(B.h[a] + B.e[a]);
-        return in;
+        for (uint32_t w = 0; w < BRICK_WAVES; ++w) {
+            const uint32_t ws = wave_sums[w];
+            if (w < wid) off += ws;
+            total += ws;
+        }
     };
-    // 1. counters of this thread's halo cells c0 .. c0 + per - 1 (already loaded for small halos)
-    uint32_t sum = 0, sum_in = 0;
-    if (per <= STAGE_UNROLL) {
+    if (per > STAGE_CELLS) {  // a large halo: its counters are read twice
+        uint32_t sum = 0;
+        for (uint32_t u = 0; u < per; u += STAGE_CELLS) {
+            const HaloCells q = load_halo_cells(g.counts, nullptr, B, Hs, c0 + u, min(per - u, STAGE_CELLS));
+            sum += q.n[0] + q.n[1] + q.n[2] + q.n[3];
+        }
+        place(sum);
+    }
+    if (per <= STAGE_CELLS) place(h.n[0] + h.n[1] + h.n[2] + h.n[3]);
+    if (total > max_states) return 0xFFFFFFFFu;  // block-uniform
+    for (uint32_t u0 = 0; u0 < per; u0 += STAGE_CELLS) {  // once, but for large halos
+        if (per > STAGE_CELLS) h = load_halo_cells(g.counts, nullptr, B, Hs, c0 + u0, min(per - u0, STAGE_CELLS));
 #pragma unroll
-        for (uint32_t u = 0; u < STAGE_UNROLL; ++u) {
-            const uint32_t hc = c0 + u;
-            if (u < per && hc < nh) {
-                m.hcnt[hc] = hcn.n[u];
-                m.hcell[hc] = hcn.cl[u];
-                sum += hcn.n[u];
-                if (inner_cell(hc)) sum_in += hcn.n[u];
+        for (uint32_t u = 0; u < STAGE_CELLS; ++u) {
+            const uint32_t hc = c0 + u0 + u;
+            if (u0 + u >= per || hc >= nh) break;
+            m.hstart[hc] = (uint16_t)off;
+            for (uint32_t k = 0; k < h.n[u]; ++k) {
+                uint32_t s = h.cl[u] * cap + k;
+                if (k >= cap) {
+                    // the (k - cap)-th overflow record of a crowded cell (rare); beyond a truncated overflow
+                    // list the counter runs ahead of the records: a dead placeholder
+                    uint32_t no = *g.ovf_count;
+                    no = no < g.ovf_cap ? no : g.ovf_cap;
+                    s = 0xFFFFFFFFu;
+                    for (uint32_t o = 0, seen = 0; o < no; ++o)
+                        if (g.ovf_cell[o] == h.cl[u] && seen++ == k - cap) {
+                            s = g.nbin + o;
+                            break;
+                        }
+                }
+                m.slot[off + k] = s;
+                m.hc_of[off + k] = (uint16_t)hc;
             }
+            off += h.n[u];
         }
-    } else {
-        for (uint32_t hc = c0; hc < c0 + per && hc < nh; ++hc) {
-            const uint32_t cl = halo_global_cell(B, Hs, hc);
-            const uint32_t n = cl != 0xFFFFFFFFu ? g.counts[cl] : 0u;
-            m.hcnt[hc] = n;
-            m.hcell[hc] = cl;
-            sum += n;
-            if (inner_cell(hc)) sum_in += n;
-        }
-    }
-    // 2. exclusive prefixes over the halo cells: every record slot learns its halo cell, and the
-    // inner records are listed (in halo order)
-    uint2 tot;
-    const uint2 off2 = block_exclusive_scan2(sum, sum_in, &tot);
-    uint32_t off = off2.x, off_in = off2.y;
-    for (uint32_t hc = c0; hc < c0 + per && hc < nh; ++hc) {
-        m.hstart[hc] = off;
-        const uint32_t n = m.hcnt[hc];
-        for (uint32_t k = 0; k < n && off + k < max_states; ++k) m.hc_of[off + k] = (uint16_t)hc;
-        if (inner_cell(hc)) {
-            for (uint32_t k = 0; k < n && off_in + k < max_states; ++k) m.inner[off_in + k] = (uint16_t)(off + k);
-            off_in += n;
-        }
-        off += n;
-    }
-    if (tid == 0) {
-        m.hstart[nh] = tot.x;
-        s_total = tot.x;
-        s_inner = tot.y;
     }
     __syncthreads();
-    const uint32_t total = s_total;
-    if (total > max_states) return 0xFFFFFFFFu;
-    // 3. the records: thread tid copies records tid, tid + 256, ...
-    auto fetch_slot = [&](uint32_t j, uint32_t &hc) -> uint32_t {
-        hc = m.hc_of[j];
-        const uint32_t k = j - m.hstart[hc], cell = m.hcell[hc];
-        if (k < cap) return cell * cap + k;
-        // the (k - cap)-th overflow record of a crowded cell (rare); beyond a truncated overflow
-        // list the counter runs ahead of the records: a dead placeholder
-        uint32_t no = *g.ovf_count;
-        no = no < g.ovf_cap ? no : g.ovf_cap;
-        for (uint32_t o = 0, seen = 0; o < no; ++o)
-            if (g.ovf_cell[o] == cell && seen++ == k - cap) return g.nbin + o;
-        return 0xFFFFFFFFu;
-    };
-    auto put = [&](uint32_t j, uint32_t hc, uint32_t s, const State &st) {
-        if (s == 0xFFFFFFFFu) {
-            m.P[j] = make_float4(__uint_as_float(0x7FC00000u), 0.f, 0.f, __uint_as_float(TW_DEAD));
-            m.slot[j] = 0xFFFFFFFFu;
-            return;
-        }
-        uint32_t hh[3];
-        Hs.decode(hc, hh[0], hh[1], hh[2]);
-        double shift[3];  // unwraps halo images into the local frame
+    bool edge = false;  // some halo cell lies across a boundary (block-uniform)
+    for (int a = 0; a < 3; ++a) edge = edge || B.o[a] < B.h[a] || B.o[a] + B.e[a] + B.h[a] > B.dims[a];
+    auto put = [&](uint32_t j, const State &st) {
+        double lx = st.x - F.org[0], ly = st.y - F.org[1], lz = st.z - F.org[2];
+        if (edge) {  // unwraps halo images into the local frame (a whole axis has none)
+            uint32_t hh[3];
+            Hs.decode(m.hc_of[j], hh[0], hh[1], hh[2]);
+            double shift[3];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            shift[a] = 0.0;
-            if (!(F.whole & (1u << a))) {
+            for (int a = 0; a < 3; ++a) {
                 const int32_t u = B.o[a] - B.h[a] + (int32_t)hh[a];
-                if (u < 0) shift[a] = -geo.box[a];
-                else if (u >= geo.dims[a]) shift[a] = geo.box[a];
+                shift[a] = u < 0 ? -geo.box[a] : (u >= B.dims[a] ? geo.box[a] : 0.0);
             }
+            lx += shift[0];
+            ly += shift[1];
+            lz += shift[2];
         }
-        m.slot[j] = s;
-        // a dead or outside record is never a neighbour: its NaN position fails every distance test
-        const float nan = __uint_as_float(0x7FC00000u);
-        const bool gone = (st.tw & (TW_DEAD | TW_OUTSIDE)) != 0u;
-        const float lx = gone ? nan : (float)((st.x - F.org[0]) + shift[0]);
-        const float ly = (float)((st.y - F.org[1]) + shift[1]);
-        const float lz = (float)((st.z - F.org[2]) + shift[2]);
-        m.P[j] = make_float4(lx, ly, lz, __uint_as_float(st.tw));
+        const float fx = (float)lx, fy = (float)ly, fz = (float)lz;
+        // a dead or outside record is never a neighbour: it fails every distance test
+        const bool dead = (st.tw & TW_DEAD) != 0u, gone = dead || (st.tw & TW_OUTSIDE) != 0u;
+        m.P[j] = gone ? make_float4(FAR_POS, 0.f, 0.f, FAR_SQ) : make_float4(fx, fy, fz, prefilter_d2(fx, fy, fz));
+        m.typ[j] = (uint8_t)(tw_type(st.tw) | (gone ? TYP_OUTSIDE : 0u) | (dead ? TYP_DEAD : 0u));
     };
     for (uint32_t j0 = 0; j0 < total; j0 += STAGE_UNROLL * BRICK_THREADS) {
-        uint32_t sl[STAGE_UNROLL], hcs[STAGE_UNROLL];
         State st[STAGE_UNROLL];
 #pragma unroll
         for (uint32_t u = 0; u < STAGE_UNROLL; ++u) {
             const uint32_t j = j0 + u * BRICK_THREADS + tid;
-            sl[u] = 0xFFFFFFFFu;
-            hcs[u] = 0;
             if (j < total) {
-                sl[u] = fetch_slot(j, hcs[u]);
-                if (sl[u] != 0xFFFFFFFFu) st[u] = g.bins[sl[u]];
+                const uint32_t s = m.slot[j];
+                st[u].tw = TW_DEAD;
+                if (s != 0xFFFFFFFFu) st[u] = g.bins[s];
             }
         }
 #pragma unroll
         for (uint32_t u = 0; u < STAGE_UNROLL; ++u) {
             const uint32_t j = j0 + u * BRICK_THREADS + tid;
-            if (j < total) put(j, hcs[u], sl[u], st[u]);
+            if (j < total) put(j, st[u]);
         }
     }
+    if (tid == 0) {
+        m.hstart[nh] = (uint16_t)total;
+        m.P[m.far] = make_float4(0.f, 0.f, 0.f, FAR_SQ);
+    }
     __syncthreads();
-    *n_inner_out = s_inner;
     return total;
+}
+
+// The quads q0 .. q0 + 15 of the brick's own records, listed in the wave's own array (first record | number << 16):
+// the own records of a row of cells are consecutive, and each row is dealt into quads.  Returns the number of
+// quads of the brick.  Every wave lists its own, a row a lane.
+__device__ __forceinline__ uint32_t wave_quads(const BrickSmem &m, const BrickDev &B, const Halo &Hs, uint32_t *quads,
+                                               uint32_t q0) {
+    const uint32_t lane = __lane_id(), rows = (uint32_t)(B.e[0] * B.e[1]);
+    uint32_t n_quads = 0;
+    for (uint32_t r0 = 0; r0 < rows; r0 += 64) {  // wave-uniform
+        const uint32_t row = r0 + lane;
+        uint32_t a = 0, n = 0;
+        if (row < rows) {
+            const uint32_t x = fdiv(row, B.m_e1), y = row - x * (uint32_t)B.e[1];
+            const uint32_t hc = (x + (uint32_t)B.h[0]) * Hs.HH + (y + (uint32_t)B.h[1]) * Hs.H2 + (uint32_t)B.h[2];
+            a = m.hstart[hc];
+            n = m.hstart[hc + (uint32_t)B.e[2]] - a;
+        }
+        const uint32_t nq = (n + 3) / 4, incl = wave_inclusive_sum(nq);
+        const uint32_t at = n_quads + incl - nq - q0;  // (wraps below q0)
+        for (uint32_t k = 0; k < nq; ++k)
+            if (at + k < 16u) quads[at + k] = (a + 4 * k) | (min(n - 4 * k, 4u) << 16);
+        n_quads += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    }
+    return n_quads;
+}
+
+// The owner of this lane: the wave's quads (wave_quads from q0 on) take its lanes four by four.
+// j: the owner's staged record, t: its species and flags (valid: there is one, and it lives).
+struct OwnerLane {
+    uint32_t j, t;
+    bool valid;
+};
+__device__ __forceinline__ OwnerLane owner_lane(const BrickSmem &m, const uint32_t *quads, uint32_t q0, uint32_t n_quads) {
+    const uint32_t lane = __lane_id();
+    OwnerLane o{0, 0, false};
+    if (q0 + lane / 4 < n_quads) {
+        const uint32_t e = quads[lane / 4], k = lane & 3u, n = e >> 16;
+        o.j = (e & 0xFFFFu) + min(k, n - 1u);  // an idle lane repeats the quad's last record (its cell)
+        o.t = m.typ[o.j];
+        o.valid = k < n && !(o.t & TYP_DEAD);
+    }
+    return o;
 }
 
 // ---- stencil walkers: visit the staged records of the (2r+1)^3 stencil of halo cell hc as
@@ -380,64 +431,14 @@ __device__ __forceinline__ WalkCtx make_walk(const BrickDev &B, const RepGeom &g
     for (int a = 0; a < 3; ++a) {
         c.h[a] = B.h[a];
         c.cs[a] = (float)geo.cs[a];
-        c.inv_cs[a] = (float)(1.0 / geo.cs[a]);
+        c.inv_cs[a] = __builtin_amdgcn_rcpf(c.cs[a]);  // (1 ulp; the reaches carry more slack)
     }
     return c;
 }
 
-template <bool ALL_HALO>
-struct Walk;
-
-// every axis in halo mode: the cells within `reach` of the particle at local position p in halo
-// cell hc, per axis offsets lo..hi inside -r..r (cells that overlap [p - reach, p + reach]; reach
-// carries the FP32 rounding slack, so the range is a superset of the exact one), walked as
-// (hi0 - lo0 + 1) * (hi1 - lo1 + 1) z-runs of hi2 - lo2 + 1 cells
-template <>
-struct Walk<true> {
-    uint32_t q, qe, cur, ia, ib, nx, ny, nz, row_step;
-    __device__ __forceinline__ bool begin(const WalkCtx &c, uint32_t hc, const float4 &p, float reach,
-                                          const uint32_t *hs) {
-        uint32_t hh[3];
-        c.Hs.decode(hc, hh[0], hh[1], hh[2]);
-        const float pp[3] = {p.x, p.y, p.z};
-        int lo[3], hi[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float u = pp[a] - (float)((int)hh[a] - c.h[a]) * c.cs[a];  // position inside its cell
-            // clamped in FP32 first (a huge reach or a NaN position selects the full stencil)
-            lo[a] = min(0, (int)fmaxf(floorf((u - reach) * c.inv_cs[a]), -(float)c.radius));
-            hi[a] = max(0, (int)fminf(floorf((u + reach) * c.inv_cs[a]), (float)c.radius));
-        }
-        nx = (uint32_t)(hi[0] - lo[0] + 1);
-        ny = (uint32_t)(hi[1] - lo[1] + 1);
-        nz = (uint32_t)(hi[2] - lo[2] + 1);
-        row_step = c.Hs.HH - (ny - 1u) * c.Hs.H2;
-        cur = (uint32_t)((int)hc + lo[0] * (int)c.Hs.HH + lo[1] * (int)c.Hs.H2 + lo[2]);
-        ia = ib = 0;
-        q = hs[cur];
-        qe = hs[cur + nz];
-        return q < qe || advance(c, hs);
-    }
-    __device__ __forceinline__ bool advance(const WalkCtx &c, const uint32_t *hs) {
-        do {
-            if (++ib == ny) {
-                ib = 0;
-                if (++ia == nx) return false;
-                cur += row_step;
-            } else {
-                cur += c.Hs.H2;
-            }
-            q = hs[cur];
-            qe = hs[cur + nz];
-        } while (q >= qe);
-        return true;
-    }
-};
-
 // general case: per axis halo mode (offsets -r..r), whole-axis mode with all cells (dims <= 2r) or
 // whole-axis mode with wrapped offsets; z as one run unless wrapped
-template <>
-struct Walk<false> {
+struct Walk {
     int nx, ny, nzr;
     int bx, by, bz;  // base coordinates
     int mx, my, mz;  // axis modes: 0 halo, 1 whole (all cells), 2 whole (wrapped offsets)
@@ -466,7 +467,7 @@ struct Walk<false> {
         int v = base + k;  // |overhang| <= r < D
         return v < 0 ? v + D : (v >= D ? v - D : v);
     }
-    __device__ __forceinline__ void range(const WalkCtx &c, const uint32_t *hs) {
+    __device__ __forceinline__ void range(const WalkCtx &c, const uint16_t *hs) {
         const int x = elem(ia, bx, mx, c.dims[0]);
         const int y = elem(ib, by, my, c.dims[1]);
         const uint32_t row = ((uint32_t)x * c.Hs.H1 + (uint32_t)y) * c.Hs.H2;
@@ -481,8 +482,7 @@ struct Walk<false> {
         q = hs[row + (uint32_t)z0];
         qe = hs[row + (uint32_t)z1];
     }
-    __device__ __forceinline__ bool begin(const WalkCtx &c, uint32_t hc, const float4 &, float,
-                                          const uint32_t *hs) {
+    __device__ __forceinline__ bool begin(const WalkCtx &c, uint32_t hc, const uint16_t *hs) {
         uint32_t hx, hy, hz;
         c.Hs.decode(hc, hx, hy, hz);
         axis_mode(c.whole & 1u, c.dims[0], c.radius, (int)hx, nx, bx, mx);
@@ -503,7 +503,7 @@ struct Walk<false> {
         range(c, hs);
         return q < qe || advance(c, hs);
     }
-    __device__ __forceinline__ bool advance(const WalkCtx &c, const uint32_t *hs) {
+    __device__ __forceinline__ bool advance(const WalkCtx &c, const uint16_t *hs) {
         do {
             if (++iz >= nzr) {
                 iz = 0;
@@ -525,24 +525,23 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// The general walk (bricks with a whole-axis axis).
 // Streams candidate pairs through the wave's ring: every active lane walks the stencil of its own
-// staged record (halo cell hc, local position p, reach), taking up to BATCH candidates of its
-// current run per iteration (independent LDS reads), and offers each to keep(q, P[q]); survivors are
+// staged record (halo cell hc), taking up to BATCH candidates of its current run per iteration (independent LDS reads), and offers each to keep(q, P[q]); survivors are
 // appended as (lane << 16 | q) and evaluated by eval(entry) 64 at a time with all lanes of the
 // wave.  A lane's survivors of one iteration take consecutive ring places after those of the lower
 // lanes (one prefix over the lanes' survivor counts per iteration).  The last, partial batch too runs
 // eval on every lane, idle lanes with NO_ENTRY (so that eval may read other lanes' registers).  Must
 // be called by all 64 lanes of a wave (wave-uniform control flow around it).
-template <bool ALL_HALO, class Keep, class Eval>
-__device__ __forceinline__ void pair_pipeline(const WalkCtx &c, const uint32_t *hs, const float4 *P, uint32_t *ring,
-                                              bool active, uint32_t hc, const float4 &p, float reach, Keep &&keep,
-                                              Eval &&eval) {
+template <class Keep, class Eval>
+__device__ __forceinline__ void pair_pipeline(const WalkCtx &c, const uint16_t *hs, const float4 *P, uint32_t *ring,
+                                              bool active, uint32_t hc, Keep &&keep, Eval &&eval) {
     static_assert(BATCH <= 7, "survivor counts are ranked as three bit planes");
     const uint32_t lane = __lane_id();
-    Walk<ALL_HALO> w;
+    Walk w;
     w.q = w.qe = 0;
     bool more = false;
-    if (active) more = w.begin(c, hc, p, reach, hs);
+    if (active) more = w.begin(c, hc, hs);
     uint32_t head = 0, tail = 0;  // wave-uniform
     while (__ballot(more)) {
         uint32_t q0 = 0, nq = 0;
@@ -584,6 +583,167 @@ __device__ __forceinline__ void pair_pipeline(const WalkCtx &c, const uint32_t *
     }
 }
 
+// exchanges within a quad of lanes (DPP quad_perm) and broadcasts of one of its lanes
+template <int CTRL>
+__device__ __forceinline__ int quad_perm(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, true);
+}
+__device__ __forceinline__ int quad_min(int v) {
+    v = min(v, quad_perm<0xB1>(v));  // lanes 1 0 3 2
+    return min(v, quad_perm<0x4E>(v));  // lanes 2 3 0 1
+}
+__device__ __forceinline__ int quad_max(int v) {
+    v = max(v, quad_perm<0xB1>(v));
+    return max(v, quad_perm<0x4E>(v));
+}
+template <int LANE>
+__device__ __forceinline__ float quad_bcast(float v) {
+    return __int_as_float(quad_perm<LANE * 0x55>(__float_as_int(v)));
+}
+
+// The walk of bricks in halo mode on every axis.  A quad of lanes holds up to four consecutive records of one
+// row of cells (halo cell hc, local position p, reach; active: the lane's record looks for neighbours).  The
+// cells that any of them reaches form rows (2r + 1 by 2r + 1 at most, pruned by the records' positions) of one
+// z-range, each row one contiguous run of staged records.  Each step the quad takes four candidates, one a lane,
+// and the matrix cores form the 4 x 4 values |a|^2 + |b|^2 - 2 ab - threshold(a) (v_mfma_f32_4x4x1, sixteen
+// quads at once, K = x, y, z, 1; the owners' |a|^2 - threshold is the accumulator's start): lane l gets its
+// candidate against the quad's four records, and keeps the four signs as bits.  Every QSTEPS steps the wave
+// harvests the set bits into a ring of (owner lane << 16 | candidate) entries; these pass filter(entry) 64 at a
+// time (the pair's own threshold, and not the record itself), and the survivors eval(entry) 64 at a time with
+// all lanes of the wave (the last batch's idle lanes with NO_ENTRY, so that eval may read other lanes'
+// registers); after(done) runs once a turn of the loop, at last until it returns false.  Must be called by all 64
+// lanes of a wave.
+// A lane used to test its own candidates one by one, about 36 vector instructions each with the ring
+// bookkeeping (1900 of the 3400 of a wave of 49 records at 1,000,000 particles); a step of 256 tests is about 25.
+template <class Filter, class Eval, class After>
+__device__ __forceinline__ void mfma_pipeline(const WalkCtx &c, const uint16_t *hs, const float4 *P, uint32_t far,
+                                              char *wave_lds, bool active, uint32_t hc, const float4 &p, float reach,
+                                              float expand, Filter &&filter, Eval &&eval, After &&after) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const uint32_t lane = __lane_id();
+    uint32_t *ring = (uint32_t *)wave_lds, *out = ring + QRING;
+    uint16_t *cand = (uint16_t *)(out + ORING);
+    // the owner's side
+    const float own_far = active ? p.w - (reach * reach * (1.0f + 1.0e-6f) + expand) : FAR_SQ;
+    const float ax = active ? -2.0f * p.x : 0.f, ay = active ? -2.0f * p.y : 0.f, az = active ? -2.0f * p.z : 0.f;
+    const f4 start = {quad_bcast<0>(own_far), quad_bcast<1>(own_far), quad_bcast<2>(own_far), quad_bcast<3>(own_far)};
+    // the cells within reach of the quad's records: offsets in x and y from its row, halo cells in z
+    uint32_t hh[3];
+    c.Hs.decode(hc, hh[0], hh[1], hh[2]);
+    const float pp[3] = {p.x, p.y, p.z};
+    int lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float u = pp[a] - (float)((int)hh[a] - c.h[a]) * c.cs[a];  // position inside its cell
+        // clamped in FP32 first (a huge reach selects the full stencil)
+        const int l = min(0, (int)fmaxf(floorf((u - reach) * c.inv_cs[a]), -(float)c.radius));
+        const int h = max(0, (int)fminf(floorf((u + reach) * c.inv_cs[a]), (float)c.radius));
+        const int at = a == 2 ? (int)hh[2] : 0;
+        lo[a] = quad_min(active ? at + l : 0x7FFFFF);
+        hi[a] = quad_max(active ? at + h : -0x7FFFFF);
+    }
+    const bool any = hi[2] >= lo[2];  // the quad has an active record
+    const uint32_t ny = (uint32_t)(hi[1] - lo[1] + 1), nz = (uint32_t)(hi[2] - lo[2] + 1);
+    uint32_t left = any ? (uint32_t)(hi[0] - lo[0] + 1) * ny : 0u;  // rows of the quad not yet begun
+    const uint32_t x_step = c.Hs.HH - (ny - 1u) * c.Hs.H2;
+    uint32_t cur = any ? (uint32_t)((int)(hc - hh[2]) + lo[0] * (int)c.Hs.HH + lo[1] * (int)c.Hs.H2 + lo[2]) : 0u;
+    uint32_t iy = ny;
+    // The quads of a wave go through their rows together (a row's steps are those of the longest run of the
+    // sixteen), which leaves a step little more than its products; rows of their own cost a step three times
+    // the vector instructions and saved a fifth of the steps.  The next row's bounds are read ahead.
+    uint32_t nq = left ? hs[cur] : 0u, nqe = left ? hs[cur + nz] : 0u;
+    uint32_t q = 0, qe = 0;  // this lane's candidate and the end of the run
+    bool more = __ballot(left != 0u) != 0ull;  // rows left
+    // One loop with one copy of the filter and of the evaluation: walk until QSTEPS steps are done, harvest until the
+    // ring holds a batch, sift a batch, evaluate a batch.
+    uint32_t head = 0, tail = 0, ohead = 0, otail = 0;  // wave-uniform
+    uint32_t bits = 0, n = 0;                           // pending result bits, tests of the last walk
+    while (true) {
+        if (!__ballot(bits != 0u)) {
+            uint32_t s = 0;
+            while (s < QSTEPS) {
+                const bool in = q < qe;
+                if (!__ballot(in)) {  // the next row
+                    if (!more) break;
+                    q = nq + (lane & 3u);
+                    qe = nqe;
+                    left = left ? left - 1u : 0u;
+                    const bool turn = --iy == 0u;
+                    cur += turn ? x_step : c.Hs.H2;
+                    iy = turn ? ny : iy;
+                    nq = left ? hs[cur] : 0u;
+                    nqe = left ? hs[cur + nz] : 0u;
+                    more = __ballot(left != 0u) != 0ull;
+                    continue;
+                }
+                const uint32_t idx = in ? q : far;
+                const float4 b = P[idx];
+                cand[s * 16u + lane / 4] = (uint16_t)(q - (lane & 3u));  // the quad's first (one value, one place)
+                q += 4;
+                f4 d = __builtin_amdgcn_mfma_f32_4x4x1f32(ax, b.x, start, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_4x4x1f32(ay, b.y, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_4x4x1f32(az, b.z, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_4x4x1f32(1.0f, b.w, d, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[r]), 31);
+                ++s;
+            }
+            n = 4 * s;
+        }
+        // harvest: bit n - 1 - t is test t = 4 step + owner.  A lane's entries take consecutive places after those of
+        // the lower lanes; when they do not fit, one from each lane as long as the ring is short of a batch.
+        auto entry_of = [&]() -> uint32_t {  // the lowest pending bit's
+            const uint32_t t = n - 1u - (uint32_t)__builtin_ctz(bits);
+            bits &= bits - 1u;
+            return (((lane & 60u) | (t & 3u)) << 16) | (cand[(t >> 2) * 16u + lane / 4] + (lane & 3u));
+        };
+        unsigned long long mk = __ballot(bits != 0u);
+        if (mk && tail - head < 64) {
+            const uint32_t cnt = (uint32_t)__popc(bits), incl = wave_inclusive_sum(cnt);
+            const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            if (tail - head + all <= QRING) {
+                uint32_t at = tail + incl - cnt;
+                while (bits) ring[at++ & (QRING - 1)] = entry_of();
+                tail += all;
+                mk = 0ull;
+            } else {
+                while (mk && tail - head < 64) {
+                    if (bits) {
+                        const uint32_t at = tail + rank_in_mask(mk);
+                        ring[at & (QRING - 1)] = entry_of();
+                    }
+                    tail += (uint32_t)__popcll(mk);
+                    mk = __ballot(bits != 0u);
+                }
+            }
+        }
+        const bool last = !more && !mk && !__ballot(q < qe);
+        if (tail - head >= 64 || (last && tail != head)) {
+            const uint32_t k = min(64u, tail - head);
+            wave_lds_sync();
+            const uint32_t ent = ring[(head + lane) & (QRING - 1)];
+            const bool ok = lane < k && filter(ent);
+            const unsigned long long om = __ballot(ok);
+            if (ok) out[(otail + rank_in_mask(om)) & (ORING - 1)] = ent;
+            otail += (uint32_t)__popcll(om);
+            head += k;
+        }
+        const bool flush = last && tail == head;
+        if (otail - ohead >= 64 || (flush && otail != ohead)) {
+            wave_lds_sync();
+            eval(lane < otail - ohead ? out[(ohead + lane) & (ORING - 1)] : NO_ENTRY);
+            ohead += min(64u, otail - ohead);
+            wave_lds_sync();
+        }
+        const bool done = flush && otail == ohead;
+        if (!after(done) && done) break;
+    }
+}
+
+struct NoAfter {
+    __device__ __forceinline__ bool operator()(bool) const { return false; }
+};
+
 // ---- per-block type tables, carved from dynamic LDS ahead of the staged records -----------------
 // Staged bricks need n_types <= MAX_STAGED_TYPES (larger type counts take the slow path).
 constexpr uint32_t MAX_STAGED_TYPES = 16;
@@ -600,7 +760,7 @@ __host__ __device__ inline size_t force_table_bytes(uint32_t nt, uint32_t np) {
 // search tables (the fused forces + search kernel holds both; the others use one of them)
 __host__ __device__ inline size_t table_bytes(uint32_t nt, uint32_t np) {
     const size_t n2 = (size_t)nt * nt;
-    return force_table_bytes(nt, np) + align16(sizeof(RxPairIdx) * n2) + align16(4 * n2) + align16(4 * nt);
+    return force_table_bytes(nt, np) + align16(sizeof(RxPairIdx) * n2) + align16(4 * n2) + 2 * align16(4 * nt);
 }
 
 struct ForceTables {
@@ -614,6 +774,7 @@ struct SearchTables {
     RxPairIdx *o2;  // [nt * nt]
     float *thr;     // [nt * nt]
     float *reach;   // [nt] (< 0: no pair reactions)
+    uint32_t *o1;   // [nt] order-1 reactions of the type: first entry of the list | number << 16 (the fused walk)
 };
 
 // reach of a type from the FP32 squared cutoffs of its row, widened like the prefilter
@@ -686,10 +847,10 @@ __device__ __forceinline__ SearchTables load_search_tables(char *base, const Tab
 
 
 // FP32 min image of a local-frame displacement on whole-axis axes (halo axes need none)
-__device__ __forceinline__ void frame_min_image(const Frame &F, float &dx, float &dy, float &dz) {
-    if (F.whole & 1u) dx = dx > .5f * F.L[0] ? dx - F.L[0] : (dx <= -.5f * F.L[0] ? dx + F.L[0] : dx);
-    if (F.whole & 2u) dy = dy > .5f * F.L[1] ? dy - F.L[1] : (dy <= -.5f * F.L[1] ? dy + F.L[1] : dy);
-    if (F.whole & 4u) dz = dz > .5f * F.L[2] ? dz - F.L[2] : (dz <= -.5f * F.L[2] ? dz + F.L[2] : dz);
+__device__ __forceinline__ void frame_min_image(uint32_t whole, const float *L, float &dx, float &dy, float &dz) {
+    if (whole & 1u) dx = dx > .5f * L[0] ? dx - L[0] : (dx <= -.5f * L[0] ? dx + L[0] : dx);
+    if (whole & 2u) dy = dy > .5f * L[1] ? dy - L[1] : (dy <= -.5f * L[1] ? dy + L[1] : dy);
+    if (whole & 4u) dz = dz > .5f * L[2] ? dz - L[2] : (dz <= -.5f * L[2] ? dz + L[2] : dz);
 }
 
 // the pair sum reading neighbours from the bins (slow path for bricks that do not fit in LDS)
@@ -791,25 +952,29 @@ __device__ __forceinline__ void finish_particle(const Grid &nxt, const ReplicaDe
     if (slot != 0xFFFFFFFFu && (me.tw & TW_TOPO) && topo.loc) topo.loc[R.topo_base + me.h] = slot;
 }
 
+// the ci-th of the brick's own cells
+__device__ __forceinline__ uint32_t own_cell(const BrickDev &B, uint32_t ci) {
+    const uint32_t lz = ci % B.e[2], ly = (ci / B.e[2]) % B.e[1], lx = ci / (B.e[2] * B.e[1]);
+    return B.cell_base + ((uint32_t)(B.o[0] + lx) * (uint32_t)B.dims[1] + (uint32_t)(B.o[1] + ly)) * (uint32_t)B.dims[2] +
+           (uint32_t)(B.o[2] + lz);
+}
+
 // fn(cell) for the brick's own cells, spread over the block's threads
 template <class Fn>
 __device__ __forceinline__ void for_each_own_cell(const BrickDev &B, Fn &&fn) {
     const uint32_t ncell = (uint32_t)(B.e[0] * B.e[1] * B.e[2]);
-    for (uint32_t ci = threadIdx.x; ci < ncell; ci += BRICK_THREADS) {
-        const uint32_t lz = ci % B.e[2], ly = (ci / B.e[2]) % B.e[1], lx = ci / (B.e[2] * B.e[1]);
-        fn(B.cell_base + ((uint32_t)(B.o[0] + lx) * (uint32_t)B.dims[1] + (uint32_t)(B.o[1] + ly)) * (uint32_t)B.dims[2] +
-           (uint32_t)(B.o[2] + lz));
-    }
+    for (uint32_t ci = threadIdx.x; ci < ncell; ci += BRICK_THREADS) fn(own_cell(B, ci));
 }
 
-// visits the records of the brick's own cells straight from the bins: fn(slot, state)
+// visits the records of the brick's own cells straight from the bins: fn(slot, state), a slot a thread (a cell a
+// thread left most of the block idle)
 template <class Fn>
 __device__ __forceinline__ void for_each_own_record(const Grid &cur, const BrickDev &B, uint32_t cap, Fn &&fn) {
-    for_each_own_cell(B, [&](uint32_t cell) {
-        const uint32_t n = cur.counts[cell];
-        const uint32_t m = n < cap ? n : cap;
-        for (uint32_t k = 0; k < m; ++k) fn(cell * cap + k, cur.bins[cell * cap + k]);
-        if (n > cap) {
+    const uint32_t n_slots = (uint32_t)(B.e[0] * B.e[1] * B.e[2]) * cap;
+    for (uint32_t i = threadIdx.x; i < n_slots; i += BRICK_THREADS) {
+        const uint32_t cell = own_cell(B, i / cap), k = i % cap, n = cur.counts[cell];
+        if (k < n) fn(cell * cap + k, cur.bins[cell * cap + k]);
+        if (k == 0 && n > cap) {
             uint32_t no = *cur.ovf_count;
             no = no < cur.ovf_cap ? no : cur.ovf_cap;
             uint32_t seen = 0;
@@ -819,18 +984,27 @@ __device__ __forceinline__ void for_each_own_record(const Grid &cur, const Brick
                     fn(cur.nbin + o, cur.bins[cur.nbin + o]);
                 }
         }
-    });
+    }
 }
 
 struct ForceWave {  // per-wave LDS of k_brick
     unsigned long long acc[3][64];  // fixed-point force of the wave's 64 particles
-    uint32_t s[64];                 // their bin slots
+    uint32_t quads[16];             // its quads (wave_quads)
+    uint16_t j[64];                 // the particles' staged records
 };
+
+struct StepWave : ForceWave {  // per-wave LDS of k_brick_step
+    uint32_t draw[128];        // its reaction candidates (entries of the pairs' kind)
+};
+constexpr uint32_t NO_PARTNER = 0xFFFFu;  // an order-1 candidate's entry
 
 // Bricks whose halo does not fit in LDS are listed for a second kernel that reads neighbours
 // straight from the bins.  list: [0] count, [1] blocks of the second kernel done, [2..] bricks.
-__device__ __forceinline__ void list_slow_brick(uint32_t *list, uint32_t b) {
-    if (threadIdx.x == 0) list[2 + atomicAdd(&list[0], 1u)] = b;
+__device__ __forceinline__ void list_slow_brick(uint32_t *list, uint32_t b, uint32_t *err) {
+    if (threadIdx.x == 0) {
+        list[2 + atomicAdd(&list[0], 1u)] = b;
+        atomicAdd(&err[STAT_SLOW_BRICKS], 1u);
+    }
 }
 
 // count of listed bricks; with none listed the second kernel's blocks exit at once (and nothing
@@ -889,7 +1063,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
         return;
     }
     long long e_blk = 0;
-    uint32_t total = 0xFFFFFFFFu, n_inner = 0;
+    uint32_t total = 0xFFFFFFFFu;
     const uint32_t nt = T.n_types;
     BrickSmem m;
     ForceTables ft;
@@ -902,7 +1076,9 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
         }
         ft = load_force_tables(smem, T, F.margin);
         m = carve(smem + table_bytes(nt, T.n_pots), max_states, max_halo);
-        total = stage_brick(cur, B, geo, F, cap, m, max_states, Hs, load_halo_counts(cur, B, Hs), &n_inner);
+        total = stage_brick(cur, B, geo, F, cap, m, max_states, Hs,
+                            load_halo_cells(cur.counts, nullptr, B, Hs, threadIdx.x * cells_per_thread(Hs),
+                                            min(cells_per_thread(Hs), STAGE_CELLS)));
     }
     if (total != 0xFFFFFFFFu) {
         const WalkCtx wc = make_walk(B, geo, Hs, radius);
@@ -916,7 +1092,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
         auto eval = [&](uint32_t ent) {
             if (ent == NO_ENTRY) return;
             const uint32_t ol = ent >> 16, q = ent & 0xFFFFu;
-            const State me = cur.bins[W.s[ol]];
+            const State me = cur.bins[m.slot[W.j[ol]]];
             const State o = cur.bins[m.slot[q]];
             const PairIdx pi = ft.pidx[tw_type(me.tw) * nt + tw_type(o.tw)];
             // CPUCalculateForces.cpp:226-259: x_ij = shortestDifference(x_i, x_j), gate d2 < rc^2
@@ -925,8 +1101,9 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
             const double ddz = min_image(o.z - me.z, geo.box[2], geo.pbc[2]);
             const double d2 = dist2(ddx, ddy, ddz);
             long long px, py, pz, pe;
-            if (!pair_fixed(ft.pots, pi, ddx, ddy, ddz, d2, px, py, pz, pe)) return;
-            if (fixed_saturated(px) || fixed_saturated(py) || fixed_saturated(pz)) atomicAdd(&err[ERR_FORCE_RANGE], 1u);
+            bool saturated;
+            if (!pair_fixed(ft.pots, pi, ddx, ddy, ddz, d2, px, py, pz, pe, &saturated)) return;
+            if (saturated) atomicAdd(&err[ERR_FORCE_RANGE], 1u);
             atomicAdd(&W.acc[0][ol], (unsigned long long)px);
             atomicAdd(&W.acc[1][ol], (unsigned long long)py);
             atomicAdd(&W.acc[2][ol], (unsigned long long)pz);
@@ -934,41 +1111,50 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
             if (virial) pair_virial(ft.pots, pi, ddx, ddy, ddz, d2, vir);
         };
         auto rounds = [&]() {
-            for (uint32_t base = threadIdx.x & ~63u; base < n_inner; base += BRICK_THREADS) {  // wave-uniform
-                const uint32_t ii = base + lane;
-                bool valid = ii < n_inner;
-                uint32_t j = 0;
-                float4 pj = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (valid) {
-                    j = m.inner[ii];
-                    pj = m.P[j];
-                    valid = !(__float_as_uint(pj.w) & TW_DEAD);
-                }
+            for (uint32_t q0 = threadIdx.x / 64 * 16;; q0 += BRICK_THREADS / 4) {  // wave-uniform
+                const uint32_t n_quads = wave_quads(m, B, Hs, W.quads, q0);
+                if (q0 >= n_quads) break;
+                wave_lds_sync();
+                const OwnerLane ow = owner_lane(m, W.quads, q0, n_quads);
+                const uint32_t j = ow.j;
+                const bool valid = ow.valid;
                 State me{};
                 uint32_t sj = 0;
                 if (valid) {
                     sj = m.slot[j];
                     me = cur.bins[sj];
                 }
-                W.s[lane] = sj;
+                W.j[lane] = (uint16_t)j;
                 W.acc[0][lane] = 0ull;
                 W.acc[1][lane] = 0ull;
                 W.acc[2][lane] = 0ull;
                 wave_lds_sync();
-                const uint32_t t = tw_type(me.tw);
+                const float4 pj = m.P[j];
+                const uint32_t t = ow.t & TYP_MASK;
                 const float reach = ft.reach[t];
-                const bool active = valid && !(me.tw & TW_OUTSIDE) && reach >= 0.f;
-                const float *thr_row = ft.thr + t * nt;
-                // prefilter, branch-free: one LDS read of the candidate, one of the threshold
-                auto keep = [&](uint32_t q, const float4 &pq) -> bool {
-                    const uint32_t tw2 = __float_as_uint(pq.w);
-                    float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
-                    if constexpr (!AH) frame_min_image(F, dx, dy, dz);
-                    const float d2p = prefilter_d2(dx, dy, dz);
-                    const float thr = thr_row[tw_type(tw2)];
-                    return (q != j) & (d2p < thr);  // dead / outside records hold NaN positions
-                };
-                pair_pipeline<AH>(wc, m.hstart, m.P, m.rings + (threadIdx.x / 64) * RING, active, m.hc_of[j], pj, reach, keep, eval);
+                const bool active = valid && !(ow.t & TYP_OUTSIDE) && reach >= 0.f;
+                char *wave_ring = m.rings + (threadIdx.x / 64) * WAVE_RING_BYTES;
+                if constexpr (AH) {
+                    auto filter = [&](uint32_t ent) -> bool {
+                        const uint32_t q = ent & 0xFFFFu, jo = W.j[ent >> 16];
+                        const float4 a = m.P[jo], b = m.P[q];
+                        return (q != jo) &
+                               (prefilter_d2(b.x - a.x, b.y - a.y, b.z - a.z) < ft.thr[m.typ[jo] * nt + m.typ[q]]);
+                    };
+                    mfma_pipeline(wc, m.hstart, m.P, m.far, wave_ring, active, m.hc_of[j], pj, reach, F.expand, filter,
+                                  eval, NoAfter{});
+                } else {
+                    const float *thr_row = ft.thr + t * nt;
+                    // prefilter, branch-free: one LDS read of the candidate, one of the threshold
+                    auto keep = [&](uint32_t q, const float4 &pq) -> bool {
+                        float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
+                        frame_min_image(F.whole, F.L, dx, dy, dz);
+                        const float d2p = prefilter_d2(dx, dy, dz);
+                        const float thr = thr_row[m.typ[q]];
+                        return (q != j) & (d2p < thr);  // dead / outside records are far away
+                    };
+                    pair_pipeline(wc, m.hstart, m.P, (uint32_t *)wave_ring, active, m.hc_of[j], keep, eval);
+                }
                 wave_lds_sync();
                 if (valid)
                     finish_particle<MODE>(nxt, R, geo, T, topo, cap, dt, noise, force_out, sj, me, true,
@@ -981,7 +1167,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
         block_add_energy(reps, B.r, e_blk);
         if (virial) block_add_virial(virial, B.r, vir);
     } else {
-        list_slow_brick(slow, bidx);
+        list_slow_brick(slow, bidx, err);
     }
 }
 
@@ -1016,7 +1202,8 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_slow(Grid cur, Grid nxt
 }
 
 struct SearchWave {  // per-wave LDS of k_brick_search
-    uint32_t s[64];  // bin slots of the wave's 64 particles
+    uint32_t quads[16];
+    uint16_t j[64];  // staged records of the wave's 64 particles
 };
 
 // reaction candidate search of one brick on the current buffer (see search_one for the rules)
@@ -1034,16 +1221,12 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
     const BrickDev B = bricks[bidx];
     const ReplicaDev &R = reps[B.r];
     const RepGeom geo = load_geom(R);
-    // a launch without reactions (handler 2) covers every replica; DetailedBalance searches every replica
-    // with the Gillespie keys; else a replica's own choice wins
-    if (handler == HANDLER_DETAILED_BALANCE) handler = 1;
-    else if (handler <= 1 && R.handler >= 0) handler = R.handler;
-    if (handler > 1 || !R.in_use || !R.active) return;
+    if (replica_handler(R, handler) > 1 || !R.in_use || !R.active) return;
     const uint32_t nt = T.n_types;
     if (!T.has_o2 && T.o1idx[nt] == 0) return;  // no reactions
     const Frame F = make_frame(B, geo);
     const Halo Hs = make_halo(B);
-    uint32_t total = 0xFFFFFFFFu, n_inner = 0;
+    uint32_t total = 0xFFFFFFFFu;
     BrickSmem m;
     SearchTables st;
     if (nt <= MAX_STAGED_TYPES) {
@@ -1053,10 +1236,12 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
         }
         st = load_search_tables(smem, T, F.margin);
         m = carve(smem + table_bytes(nt, T.n_pots), max_states, max_halo);
-        total = stage_brick(cur, B, geo, F, cap, m, max_states, Hs, load_halo_counts(cur, B, Hs), &n_inner);
+        total = stage_brick(cur, B, geo, F, cap, m, max_states, Hs,
+                            load_halo_cells(cur.counts, nullptr, B, Hs, threadIdx.x * cells_per_thread(Hs),
+                                            min(cells_per_thread(Hs), STAGE_CELLS)));
     }
     if (total == 0xFFFFFFFFu) {
-        list_slow_brick(slow, bidx);
+        list_slow_brick(slow, bidx, err);
         return;
     }
     const uint32_t r = B.r, step = R.step;
@@ -1088,7 +1273,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
     auto eval = [&](uint32_t ent) {
         if (ent == NO_ENTRY) return;
         const uint32_t ol = ent >> 16, q = ent & 0xFFFFu;
-        const uint32_t s1 = W.s[ol], s2 = m.slot[q];
+        const uint32_t s1 = m.slot[W.j[ol]], s2 = m.slot[q];
         const State me = cur.bins[s1];
         const State o = cur.bins[s2];
         const uint32_t mh = me.h, t = tw_type(me.tw);
@@ -1108,21 +1293,18 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
             if (!(u53(x4[0], x4[1]) < X.p_accept)) continue;
             // entry1: the educt of type educts[0]; equal educt types: the lower handle
             const bool me_first = (X.educts[0] != X.educts[1]) ? (t == X.educts[0]) : (mh < o.h);
-            if (me_first) emit(rx, s1, s2, mh, o.h, event_key(handler, x4, X.rate));
-            else emit(rx, s2, s1, o.h, mh, event_key(handler, x4, X.rate));
+            if (me_first) emit(rx, s1, s2, mh, o.h, event_words(x4));
+            else emit(rx, s2, s1, o.h, mh, event_words(x4));
         }
     };
     auto rounds = [&]() {
-        for (uint32_t base = threadIdx.x & ~63u; base < n_inner; base += BRICK_THREADS) {  // wave-uniform
-            const uint32_t ii = base + lane;
-            bool valid = ii < n_inner;
-            uint32_t j = 0;
-            float4 pj = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (valid) {
-                j = m.inner[ii];
-                pj = m.P[j];
-                valid = !(__float_as_uint(pj.w) & TW_DEAD);
-            }
+        for (uint32_t q0 = threadIdx.x / 64 * 16;; q0 += BRICK_THREADS / 4) {  // wave-uniform
+            const uint32_t n_quads = wave_quads(m, B, Hs, W.quads, q0);
+            if (q0 >= n_quads) break;
+            wave_lds_sync();
+            const OwnerLane ow = owner_lane(m, W.quads, q0, n_quads);
+            const uint32_t j = ow.j;
+            const bool valid = ow.valid;
             State me{};
             uint32_t sj = 0;
             if (valid) {
@@ -1138,28 +1320,41 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
                     uint32_t x4[4];
                     philox(me.h, step, 1u | (rx << 8), 0u, seed, x4);
                     if (!(u53(x4[0], x4[1]) < X.p_accept)) continue;
-                    emit(rx, sj, sj, me.h, me.h, event_key(handler, x4, X.rate));
+                    emit(rx, sj, sj, me.h, me.h, event_words(x4));
                 }
             }
             if (!T.has_o2) continue;  // block-uniform
-            W.s[lane] = sj;
+            W.j[lane] = (uint16_t)j;
             wave_lds_sync();
+            const float4 pj = m.P[j];
             const float reach = st.reach[t];
             const bool active = valid && !(me.tw & TW_OUTSIDE) && reach >= 0.f;
-            const float *thr_row = st.thr + t * nt;
+            char *wave_ring = m.rings + (threadIdx.x / 64) * WAVE_RING_BYTES;
             // each unordered pair once: the lower type finds it; equal types: the lower bin slot
             // (which also excludes the particle itself); branch-free
-            auto keep = [&](uint32_t q, const float4 &pq) -> bool {
-                const uint32_t tw2 = __float_as_uint(pq.w);
-                const uint32_t t2 = tw_type(tw2);
-                float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
-                if constexpr (!AH) frame_min_image(F, dx, dy, dz);
-                const float d2p = prefilter_d2(dx, dy, dz);
-                const float thr = thr_row[t2];
-                const uint32_t sq = m.slot[q];
-                return ((tw2 & (TW_DEAD | TW_OUTSIDE)) == 0u) & ((t2 > t) | ((t2 == t) & (sq > sj))) & (d2p < thr);
-            };
-            pair_pipeline<AH>(wc, m.hstart, m.P, m.rings + (threadIdx.x / 64) * RING, active, m.hc_of[j], pj, reach, keep, eval);
+            if constexpr (AH) {
+                auto filter = [&](uint32_t ent) -> bool {
+                    const uint32_t q = ent & 0xFFFFu, ol = ent >> 16, jo = W.j[ol];
+                    const float4 a = m.P[jo], b = m.P[q];
+                    const uint32_t t1 = m.typ[jo], t2 = m.typ[q];
+                    return ((t2 > t1) | ((t2 == t1) & (m.slot[q] > m.slot[W.j[ol]]))) &
+                           (prefilter_d2(b.x - a.x, b.y - a.y, b.z - a.z) < st.thr[t1 * nt + t2]);
+                };
+                mfma_pipeline(wc, m.hstart, m.P, m.far, wave_ring, active, m.hc_of[j], pj, reach, F.expand, filter, eval,
+                              NoAfter{});
+            } else {
+                const float *thr_row = st.thr + t * nt;
+                auto keep = [&](uint32_t q, const float4 &pq) -> bool {
+                    const uint32_t t2 = m.typ[q];
+                    float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
+                    frame_min_image(F.whole, F.L, dx, dy, dz);
+                    const float d2p = prefilter_d2(dx, dy, dz);
+                    const float thr = thr_row[t2];
+                    const uint32_t sq = m.slot[q];
+                    return ((t2 > t) | ((t2 == t) & (sq > sj))) & (d2p < thr);
+                };
+                pair_pipeline(wc, m.hstart, m.P, (uint32_t *)wave_ring, active, m.hc_of[j], keep, eval);
+            }
             wave_lds_sync();
         }
     };
@@ -1169,7 +1364,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
 // the listed bricks of k_brick_search, searched straight from the bins
 __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search_slow(Grid cur, ReplicaDev *reps, Tables T,
                                                                      const BrickDev *bricks, uint32_t cap, int radius,
-                                                                     int handler, Event *events, uint32_t *ev_count,
+                                                                     Event *events, uint32_t *ev_count,
                                                                      uint32_t *slow, uint32_t *err) {
     const uint32_t n = slow_count(slow);
     if (n == 0) return;  // grid-uniform
@@ -1177,7 +1372,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search_slow(Grid cur, R
         const BrickDev B = bricks[slow[2 + i]];
         for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (!(me.tw & TW_DEAD))
-                search_one(cur, reps, T, cap, radius, handler, 0, events, ev_count, nullptr, 0, s, me, err);
+                search_one(cur, reps, T, cap, radius, 0, events, ev_count, nullptr, 0, s, me, err);
         });
     }
     release_slow_list(slow);

@@ -45,6 +45,7 @@ struct HostReplica {
     uint32_t topo_reserve = 0;  // handles reserved for topology-particle fusions (rdy_reserve_topology_particles)
     uint32_t tt_base = 0, n_tt = 0;  // topologies (their types) for spatial topology reactions
     bool has_particles = false;  // particles were uploaded since the replica was added
+    uint64_t n_uploaded = 0;     // particles of the last upload
     uint64_t handle_guess = 0;   // handles a readback makes room for (the last one read and some growth)
     ReplicaDev dev{};
 };
@@ -132,6 +133,9 @@ struct rdy_engine {
     // LDS-staged bricks
     uint32_t brick[3] = {0, 0, 0};
     uint32_t max_states = 0, max_halo = 0;
+    double brick_lam = 0, brick_cells = 0;  // what the shape was chosen for
+    double lam_boost = 1.0;                                  // raised until few bricks outgrow their staging capacity
+    uint32_t max_states_cfg = 0, brick_cfg[3] = {0, 0, 0};  // as the caller set them (0: chosen here)
     size_t brick_smem = 0;
     size_t tables_lds = 0;  // bytes of brick_smem reserved for the per-block type tables
     size_t lds_limit = 65536;
@@ -141,6 +145,7 @@ struct rdy_engine {
     uint32_t *d_slow = nullptr;  // two lists of bricks left to the bin-reading kernels (forces, search)
     uint32_t n_bricks_ah = 0;    // leading bricks of bricks_h in halo mode on every axis
     bool bricks_dirty = false;   // replicas changed since the last brick upload
+    bool fit_dirty = false;      // particles were uploaded since the shape was last fitted to them
     bool wl_valid = true;  // the current buffer has a work list
     uint64_t cells_hwm = 0;  // end of the highest cell range handed out (the scan covers [0, hwm))
     Event *events = nullptr;
@@ -276,14 +281,16 @@ int ensure_scratch(rdy_engine *e, size_t bytes) {
 int check_errors(rdy_engine *e) {
     hipError_t le = hipGetLastError();  // launch-time errors (e.g. a launch configuration the device rejects)
     if (le != hipSuccess) return set_err(RDY_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(le));
-    uint32_t h[N_ERR];
+    uint32_t h[N_STAT];
     HIP_TRY(hipMemcpyAsync(h, e->err, sizeof h, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     bool any = false;
     for (int i = 0; i < N_ERR; ++i) any = any || h[i];
-    if (!any) return RDY_OK;
-    HIP_TRY(hipMemsetAsync(e->err, 0, sizeof(uint32_t) * N_ERR, e->stream));
+    if (!any && !h[STAT_SLOW_BRICKS]) return RDY_OK;
+    HIP_TRY(hipMemsetAsync(e->err, 0, sizeof h, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
+    if (h[STAT_SLOW_BRICKS]) e->fit_dirty = true;  // the particles have gathered or multiplied
+    if (!any) return RDY_OK;
     if (h[ERR_FORCE_RANGE])
         return set_err(RDY_ERR_NUMERIC, "a force beyond the fixed-point range (|F| >= 1.68e7 per pair or particle, " +
                                             std::to_string(h[ERR_FORCE_RANGE]) +
@@ -349,6 +356,7 @@ int upload_tables(rdy_engine *e, double dt) {
             d.p[0] = (float)k;
             d.p[1] = (float)sigma;
             d.p[2] = q[3] != 0.0 ? (float)(k * (std::pow(sigma / rc, m) - std::pow(sigma / rc, n))) : 0.0f;
+            d.p[3] = -d.p[0] / (d.p[1] * d.p[1]);  // in FP32, as the force's factor was formed per pair
             break;
         }
         case RDY_POT_SCREENED_ELECTROSTATICS:
@@ -358,6 +366,7 @@ int upload_tables(rdy_engine *e, double dt) {
             d.p[1] = (float)q[1];
             d.p[2] = (float)q[2];
             d.p[3] = (float)q[3];
+            d.p[4] = d.p[2] * (float)d.ia / d.p[3];  // in FP32, likewise
             break;
         }
         uint32_t id = (uint32_t)pots.size();
@@ -663,8 +672,8 @@ int alloc_pools(rdy_engine *e) {
     HIP_TRY(hipMemsetAsync(e->e_bonded, 0, e->max_reps * 8, e->stream));
     HIP_TRY(dalloc(&e->virial, 9ull * e->max_reps));
     HIP_TRY(hipMemsetAsync(e->virial, 0, 9ull * e->max_reps * 8, e->stream));
-    HIP_TRY(dalloc(&e->err, N_ERR));
-    HIP_TRY(hipMemsetAsync(e->err, 0, N_ERR * sizeof(uint32_t), e->stream));
+    HIP_TRY(dalloc(&e->err, N_STAT));
+    HIP_TRY(hipMemsetAsync(e->err, 0, N_STAT * sizeof(uint32_t), e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     e->free_cells.clear();
     e->free_cells.push_back({0, e->max_cells});
@@ -820,10 +829,61 @@ int upload_bricks(rdy_engine *e) {
 
 uint32_t n_bricks(const rdy_engine *e) { return (uint32_t)std::max<size_t>(e->bricks_h.size(), 1); }
 
+int configure_bricks(rdy_engine *e, double lam, const int32_t *dims, double scale);
+
+// The shape follows the particles that were uploaded, not the budget that they may grow to (a budget of four times
+// the particles quartered the bricks: 21.7 us a walk of 2,000 particles, now 19): their mean occupancy, raised until
+// few bricks hold more than their staging capacity (chains gather by their length: a Poisson fill is too narrow).
+int fit_bricks(rdy_engine *e) {
+    double n = 0, cells = 0, largest = 0;
+    const int32_t *dims = nullptr;
+    for (const HostReplica &H : e->reps_h)
+        if (H.in_use && H.has_particles && H.n_uploaded) {
+            n += (double)H.n_uploaded;
+            cells += (double)H.n_cells;
+            if ((double)H.n_cells > largest) {
+                largest = (double)H.n_cells;
+                dims = H.dev.dims;
+            }
+        }
+    for (;;) {
+        // a change of 15% in occupancy, or of two in size, is inside the flat part of the choice
+        const double lam = dims ? n / cells * e->lam_boost : e->brick_lam;
+        if (std::abs(lam / e->brick_lam - 1.0) >= 0.15 || (dims && (cells >= 2.0 * e->brick_cells || cells <= 0.5 * e->brick_cells))) {
+            e->brick_cells = cells;
+            e->bricks_dirty = true;
+            e->version++;
+            if (int rc = configure_bricks(e, lam, dims, cells / largest)) return rc;
+        }
+        if (e->bricks_dirty) {
+            if (int rc = upload_bricks(e)) return rc;
+            e->bricks_dirty = false;
+        }
+        if (!dims || e->max_states_cfg || e->lam_boost > 64.0) return RDY_OK;
+        uint32_t full = 0;
+        HIP_TRY(hipMemsetAsync(e->err + STAT_FULL_BRICKS, 0, sizeof(uint32_t), e->stream));
+        const uint32_t nb = (uint32_t)e->bricks_h.size();
+        hipLaunchKernelGGL(k_brick_fill, dim3(blocks_for(nb, BRICK_WAVES)), dim3(BRICK_THREADS), 0, e->stream,
+                           (const uint32_t *)e->grid(e->cur).counts, (const BrickDev *)e->d_bricks, nb, e->max_states,
+                           e->err);
+        HIP_TRY(hipMemcpyAsync(&full, e->err + STAT_FULL_BRICKS, sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
+        HIP_TRY(hipStreamSynchronize(e->stream));
+        // a brick left to the bin-reading path costs up to a thousand staged ones (one workgroup a replica takes them:
+        // 31 of 2,000 bricks of chains took 20 ms a step), until the others would have to shrink to nothing for it
+        if (full == 0 || (e->lam_boost > 4.0 && full <= nb / 64)) return RDY_OK;
+        e->lam_boost *= 1.25;
+    }
+}
+
 // brick tables of the current replicas on the device (before any brick launch or graph capture)
 int ensure_bricks(rdy_engine *e) {
+    int rc = RDY_OK;
+    if (e->fit_dirty) {
+        if ((rc = fit_bricks(e))) return rc;
+        e->fit_dirty = false;
+    }
     if (!e->bricks_dirty) return RDY_OK;
-    int rc = upload_bricks(e);
+    rc = upload_bricks(e);
     if (rc == RDY_OK) e->bricks_dirty = false;
     return rc;
 }
@@ -887,53 +947,97 @@ void launch_topo_reactions(rdy_engine *e, int require_active, Edit *edits, uint3
 // blocks of the bin-reading kernels (they loop over the listed bricks; none listed: they just exit)
 uint32_t slow_blocks(const rdy_engine *e) { return std::min<uint32_t>(n_bricks(e), 256u); }
 
-// brick shape and LDS budget from the expected particles per cell (overridable in the config)
-// Brick shape for mean cell occupancy lam on the grid dims: the brick's own particles fill one round
-// of the block's lanes (mean + 3 sigma <= BRICK_THREADS; two rounds above 3 particles per cell,
-// where one-round bricks would be tiny), since a brick whose particles spill into a further round
-// keeps its whole block waiting on one wave.  Among those shapes the one with the fewest staged cells
-// over the whole grid (halos included) plus a fixed cost per brick (its round trips, counted as
-// 64 / lam cells) wins; ties go to the larger brick.
-void choose_brick(double lam, const int32_t *dims, int radius, uint32_t out[3]) {
+// LDS bytes of a walk's block beside its staged records' budget, set by configure_bricks
+constexpr size_t LDS_PER_CU = 160 * 1024, LDS_GRAIN = 1280;
+
+// staged records a brick of `halo` cells needs at least, for mean cell occupancy lam: the expected number and five
+// standard deviations of a uniform (Poisson) fill
+uint32_t least_states(double lam, double halo) {
+    const double mean = std::max(lam, 0.25) * halo;
+    return (uint32_t)std::min(60000.0, mean + 5.0 * std::sqrt(mean) + 16.0);
+}
+
+// mean and variance of ceil(n / 4) for n Poisson distributed with mean mu: the quads of a row of cells
+void quads_of_row(double mu, double *mean, double *var) {
+    double p = std::exp(-mu), e1 = 0, e2 = 0, all = 0;
+    for (int n = 0; n < 4096 && all < 1.0 - 1e-9; ++n) {
+        const double c = (n + 3) / 4;
+        e1 += p * c;
+        e2 += p * c * c;
+        all += p;
+        p *= mu / (n + 1);
+        if (mu > 600.0) {  // exp(-mu) underflows: rows this full are dealt evenly
+            *mean = mu / 4 + 0.375;
+            *var = mu / 16 + 0.1;
+            return;
+        }
+    }
+    *mean = e1;
+    *var = e2 - e1 * e1;
+}
+
+// Brick shape for mean cell occupancy lam on the grid dims (`scale` grids like it): the shape of least modelled time
+// among near-cubes to z-rows of 2.5 times their width whose quads of records (mean + 1.7 sigma) fit one round of a
+// block's 64.  In cycles, a wave costs its share of the staging and, per 16 quads, a fixed part (the move, the draws)
+// and its steps (the rows of the stencil by the longest of sixteen runs); blocks overlap by how many fit in a CU's
+// LDS, and a last round that is partly empty, or a system smaller than one round, costs the latency of a block.
+// The constants are fitted to the measured walks of 110 shapes over nine systems of 500 to 1,000,000 particles; a
+// shape within 10% of the best of a system's sweep is what the fit gives (1,000,000 particles at one a cell:
+// 4 x 5 x 10 139 us, 5 x 5 x 7 145, 4 x 4 x 8 174; 700,000 at two a cell: 4 x 5 x 4 106 us, 3 x 3 x 8 120,
+// 2 x 3 x 12 137; 200,000 at 0.6: 5 x 5 x 12 46 us, 4 x 4 x 12 56; 2,000 at 0.25: 3 x 3 x 3 19 us, 4 x 4 x 7 21).
+void choose_brick(double lam, const int32_t *dims, double scale, int radius, size_t other_lds, uint32_t out[3]) {
     lam = std::max(lam, 1.0 / 64.0);
-    const double x = (-3.0 + std::sqrt(9.0 + 4.0 * BRICK_THREADS)) / 2.0;  // sqrt of the one-round mean
-    const double vmax = (lam >= 3.0 ? 2.0 : 1.0) * x * x / lam;
+    const double r = radius;
     double best = 0.0;
     bool found = false;
-    for (uint32_t ex = 1; ex <= 16; ++ex)
-        for (uint32_t ey = 1; ey <= 16; ++ey)
-            for (uint32_t ez = 1; ez <= 16; ++ez) {
-                const double V = (double)ex * ey * ez;
-                const double halo = (double)(ex + 2 * radius) * (ey + 2 * radius) * (ez + 2 * radius);
-                if (V > vmax || halo * std::max(lam, 0.25) > 1500.0) continue;
-                double staged = 1.0, n_bricks = 1.0;
-                const uint32_t ee[3] = {ex, ey, ez};
-                for (int a = 0; a < 3; ++a) {
-                    const double D = (double)dims[a];
-                    if (D < 2.0 * radius + 1.0) {
-                        staged *= D;  // whole-axis brick: no halo
-                    } else {
-                        const double n = std::ceil(D / ee[a]);
-                        staged *= D + 2.0 * radius * n;
-                        n_bricks *= n;
-                    }
+    for (uint32_t ez = 1; ez <= 32; ++ez) {
+        const bool whole_z = dims[2] < 2 * radius + 1;
+        const double nz = whole_z ? 1.0 : std::ceil(dims[2] / (double)ez), lz = dims[2] / nz;
+        if (ez > 1 && std::ceil(dims[2] / (double)(ez - 1)) == nz && !whole_z) continue;  // the same split
+        if (whole_z && ez > 1) continue;
+        double q1, qv;
+        quads_of_row(lam * lz, &q1, &qv);
+        const double span = std::min(lz, 1.0 + 3.0 / lam), run = lam * (span + 2.0 * r);
+        const double steps = (2 * r + 1) * (2 * r + 1) * ((run + 1.8 * std::sqrt(run)) / 4.0 + 0.5);
+        for (uint32_t ex = 1; ex <= 16; ++ex)
+            for (uint32_t ey = ex; ey <= ex + 1; ++ey) {
+                if (!whole_z && (ez < ex || 2 * ez > 5 * ex)) continue;
+                const uint32_t ee[2] = {ex, ey};
+                double n[2], l[2];
+                for (int a = 0; a < 2; ++a) {
+                    n[a] = dims[a] < 2 * radius + 1 ? 1.0 : std::ceil(dims[a] / (double)ee[a]);
+                    l[a] = dims[a] / n[a];
                 }
-                const double cost = staged + n_bricks * 64.0 / lam;
-                const uint32_t vol = ex * ey * ez, bvol = out[0] * out[1] * out[2];
-                if (!found || cost < best * (1.0 - 1e-9) || (cost <= best * (1.0 + 1e-9) && vol > bvol)) {
+                const double rows = l[0] * l[1], Q = rows * q1, sd = std::sqrt(rows * qv);
+                const bool smallest = ex == 1 && ey == 1 && ez == 1;
+                if (Q + 1.7 * sd > 64.0 && !smallest) continue;
+                const double cells = (l[0] + 2 * r) * (l[1] + 2 * r) * (lz + 2 * r);
+                const double halo = (ex + 2 * r) * (ey + 2 * r) * (ez + 2 * r);
+                const size_t lds = (other_lds + brick_smem_bytes(least_states(lam, halo), (uint32_t)halo) + LDS_GRAIN - 1) /
+                                   LDS_GRAIN * LDS_GRAIN;
+                if (lds > LDS_PER_CU && !smallest) continue;
+                const double k = std::max(1.0, std::min(5.0, std::floor((double)LDS_PER_CU / (double)lds)));
+                const double nb = n[0] * n[1] * nz * scale, full = nb / (256.0 * k);
+                const double block = 4.0 * (3500.0 + 1400.0 * cells * (1.0 + lam) / 256.0) +
+                                     std::max(1.0, Q / 16.0 + 0.5) * (7500.0 + 85.0 * steps);
+                const double thr = nb * block / (1024.0 * (1.0 - std::exp(-0.25 * k)));
+                const double lat = 25000.0 + 250.0 * lam * Q + 40.0 * cells + 330.0 * steps;
+                const double cost =
+                    full <= 1.0 ? lat + 0.3 * thr
+                                : thr * (1.0 + 0.5 * (std::ceil(full) / full - 1.0)) + 0.5 * lat;
+                if (!found || cost < best) {
                     best = cost;
                     out[0] = ex, out[1] = ey, out[2] = ez;
                     found = true;
                 }
             }
-    if (!found) out[0] = out[1] = out[2] = 2;
+    }
 }
 
-int configure_bricks(rdy_engine *e, double lam, const int32_t *dims) {
-    if (e->brick[0] == 0 || e->brick[1] == 0 || e->brick[2] == 0) choose_brick(lam, dims, e->radius, e->brick);
-    e->max_halo = 1;
-    for (int a = 0; a < 3; ++a) e->max_halo *= e->brick[a] + 2u * (uint32_t)e->radius;
-    if (e->max_halo > 60000) return set_err(RDY_ERR_INVALID, "brick plus halo exceeds 60000 cells");
+constexpr size_t WALK_BLOCKS_PER_CU = 5;  // the walk's registers allow five waves a SIMD
+
+// brick shape and staging capacity for mean cell occupancy lam (overridable in the configuration)
+int configure_bricks(rdy_engine *e, double lam, const int32_t *dims, double scale) {
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device) == hipSuccess && v > 0)
         e->lds_limit = (size_t)v;
@@ -953,14 +1057,26 @@ int configure_bricks(rdy_engine *e, double lam, const int32_t *dims) {
     const size_t tables =
         table_bytes(std::min(e->n_types, MAX_STAGED_TYPES), (uint32_t)(2 * e->pots_in.size()));
     e->tables_lds = tables;
+    e->brick_lam = lam;
+    for (int a = 0; a < 3; ++a) e->brick[a] = e->brick_cfg[a];
+    if (e->brick[0] == 0 || e->brick[1] == 0 || e->brick[2] == 0)
+        choose_brick(lam, dims, scale, e->radius, static_lds + tables + 256, e->brick);
+    e->max_halo = 1;
+    for (int a = 0; a < 3; ++a) e->max_halo *= e->brick[a] + 2u * (uint32_t)e->radius;
+    if (e->max_halo > 60000) return set_err(RDY_ERR_INVALID, "brick plus halo exceeds 60000 cells");
     if (e->lds_limit < static_lds + tables + 8192) return set_err(RDY_ERR_INVALID, "not enough LDS per workgroup");
     const size_t budget = e->lds_limit - static_lds - tables - 256;
-    // staged records: the expected halo occupancy plus ten standard deviations of a uniform (Poisson)
-    // fill; fuller halos (clustered systems) take the slow path
-    uint32_t want = e->max_states;
+    // staged records: what the workgroups that fit in a CU's LDS side by side leave beyond the least; fuller halos
+    // (clustered systems) take the slow path
+    uint32_t want = e->max_states_cfg;
     if (want == 0) {
-        const double mean = std::max(lam, 0.25) * e->max_halo;
-        want = (uint32_t)std::max(512.0, mean + 10.0 * std::sqrt(mean) + 64.0);
+        want = least_states(lam, e->max_halo);
+        const uint32_t most = (uint32_t)std::min(60000.0, 4.0 * std::max(lam, 0.25) * e->max_halo + 512.0);
+        auto whole = [&](uint32_t n) {
+            return (static_lds + tables + brick_smem_bytes(n, e->max_halo) + 256 + LDS_GRAIN - 1) / LDS_GRAIN * LDS_GRAIN;
+        };
+        const size_t side_by_side = std::min<size_t>(LDS_PER_CU / whole(want), WALK_BLOCKS_PER_CU);
+        while (side_by_side && want + 8 <= most && whole(want + 8) * side_by_side <= LDS_PER_CU) want += 8;
     }
     want = std::min<uint32_t>(want, 60000);
     while (want > 256 && brick_smem_bytes(want, e->max_halo) > budget) want -= 128;
@@ -1025,11 +1141,32 @@ void launch_walk(rdy_engine *e, int flags, int handler, double dt) {
     const Grid cur = e->grid(e->cur), nxt = e->grid(e->next()), clear = e->grid(e->after_next());
     const bool prof = e->prof && !(flags & WALK_PROLOGUE) && e->prof_used < e->prof_ev.size();
     if (prof) (void)hipEventRecord(e->prof_ev[e->prof_used].first, e->stream);
+    WalkArgs a{};
+    a.cur = cur;
+    a.nxt = nxt;
+    a.clear_counts = clear.counts;
+    a.clear_ovf = clear.ovf_count;
+    a.reps = e->reps;
+    a.T = e->T;
+    a.topo = e->topo();
+    a.bricks = e->d_bricks;
+    a.events = e->events;
+    a.ev_count = e->ev_count;
+    a.slow = slow_list(e, 0);
+    a.change_counts = e->edit_count;
+    a.err = e->err;
+    a.dt = dt;
+    a.cap = e->cap;
+    a.max_states = e->max_states;
+    a.max_halo = e->max_halo;
+    a.smem_bytes = (uint32_t)e->brick_smem;
+    a.flags = flags;
+    a.radius = e->radius;
+    a.handler = handler;
     for_brick_groups(e, [&](auto ah, uint32_t nb, uint32_t b0) {
-        hipLaunchKernelGGL((k_brick_step<decltype(ah)::value>), dim3(nb), dim3(BRICK_THREADS), e->brick_smem,
-                           e->stream, cur, nxt, clear, flags, (const ReplicaDev *)e->reps, e->T, e->topo(),
-                           (const BrickDev *)e->d_bricks, b0, e->cap, e->radius, handler, dt, e->events, e->ev_count,
-                           e->max_states, e->max_halo, (uint32_t)e->brick_smem, slow_list(e, 0), e->edit_count, e->err);
+        a.brick0 = b0;
+        hipLaunchKernelGGL((k_brick_step<decltype(ah)::value>), dim3(nb), dim3(BRICK_THREADS), e->brick_smem, e->stream,
+                           a);
     });
     if (prof) {
         (void)hipEventRecord(e->prof_ev[e->prof_used].second, e->stream);
@@ -1230,8 +1367,8 @@ int rdy_engine_create(const rdy_context_desc *ctx, const rdy_engine_config *cfg,
     }
     e->cap = c.bin_capacity ? c.bin_capacity : 16;
     e->auto_cap = c.bin_capacity == 0;
-    for (int a = 0; a < 3; ++a) e->brick[a] = c.brick[a];
-    e->max_states = c.lds_states;
+    for (int a = 0; a < 3; ++a) e->brick_cfg[a] = c.brick[a];
+    e->max_states_cfg = c.lds_states;
     e->block = c.block_size ? c.block_size : 256;
     if (e->block % 64 || e->block > 1024) {
         delete e;
@@ -1311,7 +1448,7 @@ int rdy_replica_add(rdy_engine *e, const rdy_replica_desc *d, uint32_t *replica_
             uint32_t c = (uint32_t)std::ceil(lam + 7.0 * std::sqrt(lam) + 6.0);
             e->cap = std::max<uint32_t>(8, (c + 3) / 4 * 4);
         }
-        int rcc = configure_bricks(e, lam_raw, dims);
+        int rcc = configure_bricks(e, lam_raw, dims, e->max_reps);
         if (rcc) return rcc;
         int rc = alloc_pools(e);
         if (rc) return rc;
@@ -1409,6 +1546,8 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
                            (uint32_t)e->max_particles);
     }
     H.has_particles = true;
+    e->fit_dirty = true;
+    H.n_uploaded = n;
     // the bonded terms name the replaced particles' handles: the caller sets them again
     if ((rc = drop_terms(e, r))) return rc;
     release_topo(e, H);
@@ -1977,17 +2116,16 @@ int rdy_react(rdy_engine *e, int handler, double dt) {
                            (uint32_t)e->brick_smem, slow_list(e, 1), e->err);
     });
     hipLaunchKernelGGL(k_brick_search_slow, dim3(slow_blocks(e)), dim3(BRICK_THREADS), 0, e->stream, e->grid(c),
-                       e->reps, e->T, (const BrickDev *)e->d_bricks, e->cap, e->radius, handler, e->events,
-                       e->ev_count, slow_list(e, 1), e->err);
+                       e->reps, e->T, (const BrickDev *)e->d_bricks, e->cap, e->radius, e->events, e->ev_count,
+                       slow_list(e, 1), e->err);
     if (db)
         hipLaunchKernelGGL(k_detailed_balance, dim3(nr), dim3(RESOLVE_THREADS), 0, e->stream, e->grid(c), e->reps,
                            e->T, e->cap, e->events, e->ev_count, e->rx_step, e->rx_total, (uint32_t)e->max_particles,
                            rec_ptr(e), e->recording ? e->rec_count : nullptr, e->err, e->db);
     else
         hipLaunchKernelGGL(k_resolve, dim3(nr), dim3(RESOLVE_THREADS), 0, e->stream, e->grid(c), e->reps, e->T,
-                           e->cap, e->events, e->ev_count, e->rx_step, e->rx_total, 0, (uint32_t)e->max_particles,
-                           (Edit *)nullptr, (uint32_t *)nullptr, 0u, rec_ptr(e),
-                           e->recording ? e->rec_count : nullptr, e->err);
+                           e->cap, e->events, e->ev_count, e->rx_step, e->rx_total, handler,
+                           (uint32_t)e->max_particles, rec_ptr(e), e->recording ? e->rec_count : nullptr, e->err);
     return check_errors(e);
 }
 
@@ -2131,37 +2269,40 @@ int rdy_run_graph(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
     launch_prologue(e, dt);
     const bool prof = e->prof;
     e->prof = false;
-    if (e->g_version != e->version || e->g_handler != handler || e->g_dt != dt) {
-        for (hipGraphExec_t &g : e->gexec) {
-            if (g) HIP_TRY(hipGraphExecDestroy(g));
-            g = nullptr;
-        }
-        e->g_version = e->version;
-        e->g_handler = handler;
-        e->g_dt = dt;
-    }
     // every step but the last from the graph of N_STATES steps, which starts and ends in the same state (the last
     // step copies instead of moving).  A capture costs about as much host time as GRAPH_MIN_STEPS launched steps.
     uint64_t generic = n_steps - 1;
-    hipGraphExec_t &exec = e->gexec[e->cur];
-    if (!exec && generic >= GRAPH_MIN_STEPS) {
-        const int keep = e->cur;
-        hipGraph_t g;
-        HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < N_STATES; ++k) launch_step(e, handler, dt, 0);
-        e->cur = keep;
-        HIP_TRY(hipStreamEndCapture(e->stream, &g));
-        const hipError_t ge = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        HIP_TRY(ge);
-    }
-    if (exec) {
-        for (uint64_t p = 0; p < generic / N_STATES; ++p) {
-            HIP_TRY(hipGraphLaunch(exec, e->stream));
-            if ((p & 255) == 255)
-                if ((rc = check_errors(e))) return rc;
+    uint32_t stretch = 64;  // launches between two looks at the errors
+    while (generic >= N_STATES) {
+        if (e->g_version != e->version || e->g_handler != handler || e->g_dt != dt) {
+            for (hipGraphExec_t &g : e->gexec) {
+                if (g) HIP_TRY(hipGraphExecDestroy(g));
+                g = nullptr;
+            }
+            e->g_version = e->version;
+            e->g_handler = handler;
+            e->g_dt = dt;
         }
-        generic %= N_STATES;
+        hipGraphExec_t &exec = e->gexec[e->cur];
+        if (!exec) {
+            if (generic < GRAPH_MIN_STEPS) break;
+            const int keep = e->cur;
+            hipGraph_t g;
+            HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
+            for (int k = 0; k < N_STATES; ++k) launch_step(e, handler, dt, 0);
+            e->cur = keep;
+            HIP_TRY(hipStreamEndCapture(e->stream, &g));
+            const hipError_t ge = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(g);
+            HIP_TRY(ge);
+        }
+        for (uint32_t p = 0; p < stretch && generic >= N_STATES; ++p, generic -= N_STATES)
+            HIP_TRY(hipGraphLaunch(exec, e->stream));
+        if (generic >= N_STATES) {  // a longer run looks after its errors, and its bricks, on the way
+            if ((rc = check_errors(e))) return rc;
+            if ((rc = ensure_bricks(e))) return rc;
+            stretch = 256;
+        }
     }
     for (uint64_t k = 0; k < generic; ++k) launch_step(e, handler, dt, 0);
     launch_step(e, handler, dt, 1);
@@ -2230,7 +2371,7 @@ int rdy_reaction_candidates(rdy_engine *e, uint32_t r, uint64_t cap, uint32_t *r
     HIP_TRY(hipMemsetAsync(cnt, 0, 4, e->stream));
     ensure_wl(e);
     hipLaunchKernelGGL(k_search, dim3(wl_blocks(e)), dim3(e->block), 0, e->stream, e->grid(e->cur), e->reps, e->T,
-                       e->cap, e->radius, 0, 1, e->events, cnt, out, (uint32_t)cap, r, (uint32_t)e->max_particles,
+                       e->cap, e->radius, 1, e->events, cnt, out, (uint32_t)cap, r, (uint32_t)e->max_particles,
                        e->err);
     uint32_t hc = 0;
     HIP_TRY(hipMemcpyAsync(&hc, cnt, 4, hipMemcpyDeviceToHost, e->stream));

@@ -54,7 +54,7 @@ struct Topo {
 };
 
 struct Event {
-    unsigned long long key;
+    unsigned long long key;  // the draw's words that order the events (event_words)
     uint32_t s1, s2;  // slots of entry1 / entry2 (equal for order-1)
     uint32_t h1, h2;
     uint32_t rx;
@@ -105,7 +105,9 @@ struct DbTables {
 // error flags, all counters
 enum : int { ERR_BIN_OVERFLOW = 0, ERR_EVENT_OVERFLOW = 1, ERR_WL_OVERFLOW = 2, ERR_NONFINITE = 3, ERR_EVENT_LDS = 4,
              ERR_LDS_SEARCH = 5, ERR_LDS_LAYOUT = 6, ERR_EDIT_OVERFLOW = 7, ERR_FORCE_RANGE = 8, ERR_TOPO_RESERVE = 9,
-             N_ERR = 10 };
+             N_ERR = 10,
+             // no errors: bricks left to the bin-reading path, and those that would be (k_brick_fill)
+             STAT_SLOW_BRICKS = N_ERR, STAT_FULL_BRICKS, N_STAT };
 
 constexpr int MODE_FORCES = 0;  // forces + energy of the current buffer
 constexpr int MODE_STEP = 1;    // forces, Euler-Maruyama step, re-bin into the other buffer

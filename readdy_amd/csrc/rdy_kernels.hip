@@ -668,25 +668,36 @@ __global__ void k_break_bonds(Grid cur, const ReplicaDev *reps, Topo topo, const
 // u < 1 - exp(-rate dt) is drawn per candidate from Philox keyed by the pair's handles, so the
 // candidate set and the draws do not depend on slots, thread order or batching.
 // -------------------------------------------------------------------------------------------------
-__device__ __forceinline__ unsigned long long event_key(int handler, const uint32_t x4[4], double rate) {
-    if (handler == 0) return ((unsigned long long)x4[2] << 32) | x4[3];
-    double u = u53(x4[2], x4[3]) + 0x1p-54;
+// The words of an accepted candidate's draw that order the events.  The searches keep them as they are; the resolve
+// forms the order's key from them (order_key), since the logarithm of a Gillespie key, formed for every candidate
+// where it was drawn, was 100 FP64 instructions of every wave that held one.
+__device__ __forceinline__ unsigned long long event_words(const uint32_t x4[4]) {
+    return ((unsigned long long)x4[2] << 32) | x4[3];
+}
+
+__device__ __forceinline__ unsigned long long order_key(int handler, unsigned long long words, double rate) {
+    if (handler == 0) return words;
+    double u = u53((uint32_t)(words >> 32), (uint32_t)words) + 0x1p-54;
     double k = -log(u) / rate;  // Efraimidis-Spirakis key, positive: bit order == numeric order
     return (unsigned long long)__double_as_longlong(k);
 }
 
+// the handler of a replica: DetailedBalance selects every replica's events with the Gillespie keys, a launch
+// without reactions (2) covers every replica, else the replica's own choice wins
+__device__ __forceinline__ int replica_handler(const ReplicaDev &R, int handler) {
+    if (handler == HANDLER_DETAILED_BALANCE) return 1;
+    return handler <= 1 && R.handler >= 0 ? R.handler : handler;
+}
+
 // candidates of the particle in slot s (searching from the smaller (type, bin slot) of every pair)
 __device__ __forceinline__ void search_one(const Grid &cur, ReplicaDev *reps, const Tables &T, uint32_t cap, int radius,
-                           int handler, int candidates_only, Event *events, uint32_t *ev_count, uint32_t *cand_rows,
+                           int candidates_only, Event *events, uint32_t *ev_count, uint32_t *cand_rows,
                            uint32_t cand_cap, uint32_t s, const State &me, uint32_t *err) {
     const uint32_t r = tw_replica(me.tw);
     const ReplicaDev &R = reps[r];
     const uint32_t t = tw_type(me.tw);
     const uint32_t step = R.step;
     const uint64_t seed = R.seed;
-    if (handler == HANDLER_DETAILED_BALANCE) handler = 1;  // Gillespie keys for every replica
-    else if (handler <= 1 && R.handler >= 0) handler = R.handler;  // the replica's own handler
-
     auto emit = [&](uint32_t rx, uint32_t s1, uint32_t s2, uint32_t h1, uint32_t h2, unsigned long long key,
                     uint32_t ne) {
         if (candidates_only) {
@@ -723,7 +734,7 @@ __device__ __forceinline__ void search_one(const Grid &cur, ReplicaDev *reps, co
         uint32_t x4[4];
         philox(me.h, step, 1u | (rx << 8), 0u, seed, x4);
         if (!candidates_only && !(u53(x4[0], x4[1]) < X.p_accept)) continue;
-        emit(rx, s, s, me.h, me.h, event_key(handler, x4, X.rate), 1u);
+        emit(rx, s, s, me.h, me.h, event_words(x4), 1u);
     }
     // order 2
     if (!T.has_o2 || (me.tw & TW_OUTSIDE)) return;
@@ -755,14 +766,14 @@ __device__ __forceinline__ void search_one(const Grid &cur, ReplicaDev *reps, co
             bool me_first;
             if (X.educts[0] != X.educts[1]) me_first = (t == X.educts[0]);
             else me_first = me.h < o.h;
-            if (me_first) emit(rx, s, s2, me.h, o.h, event_key(handler, x4, X.rate), 2u);
-            else emit(rx, s2, s, o.h, me.h, event_key(handler, x4, X.rate), 2u);
+            if (me_first) emit(rx, s, s2, me.h, o.h, event_words(x4), 2u);
+            else emit(rx, s2, s, o.h, me.h, event_words(x4), 2u);
         }
     });
 }
 
 __global__ __launch_bounds__(256) void k_search(Grid cur, ReplicaDev *reps, Tables T, uint32_t cap, int radius,
-                                                 int handler, int candidates_only, Event *events,
+                                                 int candidates_only, Event *events,
                                                  uint32_t *ev_count, uint32_t *cand_rows, uint32_t cand_cap,
                                                  uint32_t only_replica, uint32_t max_wl, uint32_t *err) {
     const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
@@ -776,7 +787,7 @@ __global__ __launch_bounds__(256) void k_search(Grid cur, ReplicaDev *reps, Tabl
     const uint32_t r = tw_replica(me.tw);
     if (candidates_only && r != only_replica) return;
     if (!candidates_only && !reps[r].active) return;
-    search_one(cur, reps, T, cap, radius, handler, candidates_only, events, ev_count, cand_rows, cand_cap, s, me, err);
+    search_one(cur, reps, T, cap, radius, candidates_only, events, ev_count, cand_rows, cand_cap, s, me, err);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1037,7 +1048,8 @@ __device__ __forceinline__ void detailed_balance_events(const Grid &cur, const R
 template <bool DB = false>
 __device__ __forceinline__ void resolve_replica(const Grid &cur, ReplicaDev *reps, const Tables &T, uint32_t cap,
                                                 Event *events, uint32_t *ev_count, unsigned long long *rx_step,
-                                                unsigned long long *rx_total, int require_active, uint32_t max_wl,
+                                                unsigned long long *rx_total, int handler, int require_active,
+                                                uint32_t max_wl,
                                                 Edit *edits, uint32_t *edit_count, uint32_t edit_cap,
                                                 RxRecord *recs, uint32_t *rec_count, uint32_t *err,
                                                 const DbTables D = DbTables{}) {
@@ -1080,11 +1092,12 @@ __device__ __forceinline__ void resolve_replica(const Grid &cur, ReplicaDev *rep
         ne = E;
     }
     const Event *ev = events + R.ev_base;
+    const int own_handler = replica_handler(R, handler);
     // load and pad to a power of two
     uint32_t np2 = 1;
     while (np2 < ne) np2 <<= 1;
     for (uint32_t k = tid; k < np2; k += blockDim.x) {
-        skey[k] = k < ne ? ev[k].key : ~0ull;
+        skey[k] = k < ne ? order_key(own_handler, ev[k].key, T.rx[ev[k].rx].rate) : ~0ull;
         sidx[k] = k;
     }
     __syncthreads();
@@ -1369,11 +1382,10 @@ __device__ __forceinline__ void resolve_replica(const Grid &cur, ReplicaDev *rep
 __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve(Grid cur, ReplicaDev *reps, Tables T, uint32_t cap,
                                                              Event *events, uint32_t *ev_count,
                                                              unsigned long long *rx_step, unsigned long long *rx_total,
-                                                             int require_active, uint32_t max_wl, Edit *edits,
-                                                             uint32_t *edit_count, uint32_t edit_cap, RxRecord *recs,
+                                                             int handler, uint32_t max_wl, RxRecord *recs,
                                                              uint32_t *rec_count, uint32_t *err) {
-    resolve_replica(cur, reps, T, cap, events, ev_count, rx_step, rx_total, require_active, max_wl, edits, edit_count,
-                    edit_cap, recs, rec_count, err);
+    resolve_replica(cur, reps, T, cap, events, ev_count, rx_step, rx_total, handler, 0, max_wl, (Edit *)nullptr,
+                    (uint32_t *)nullptr, 0u, recs, rec_count, err);
 }
 
 // SCPUDetailedBalance::perform's event loop, one workgroup per replica (the candidates come from the
@@ -1384,7 +1396,8 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_detailed_balance(Grid cur, 
                                                                       unsigned long long *rx_total, uint32_t max_wl,
                                                                       RxRecord *recs, uint32_t *rec_count,
                                                                       uint32_t *err, DbTables D) {
-    resolve_replica<true>(cur, reps, T, cap, events, ev_count, rx_step, rx_total, 0, max_wl, (Edit *)nullptr,
+    resolve_replica<true>(cur, reps, T, cap, events, ev_count, rx_step, rx_total, HANDLER_DETAILED_BALANCE, 0, max_wl,
+                          (Edit *)nullptr,
                           (uint32_t *)nullptr, 0u, recs, rec_count, err, D);
 }
 

@@ -109,29 +109,6 @@ __global__ void k_topo_begin(long long *fb, uint32_t n_fb, const uint32_t *loc, 
     if (i < n_loc) loc_cur[i] = loc[i];
 }
 
-// The counters of the brick's own cells in buffer `clear`, which becomes the target of the next step's walk.
-// hcn: the thread's halo cells (load_halo_counts).
-__device__ __forceinline__ void clear_own_cells(uint32_t *clear, const BrickDev &B, const Halo &Hs,
-                                                const HaloCounts &hcn) {
-    const uint32_t per = (Hs.nh + BRICK_THREADS - 1) / BRICK_THREADS, c0 = threadIdx.x * per;
-    auto own = [&](uint32_t hc) -> bool {
-        uint32_t hh[3];
-        Hs.decode(hc, hh[0], hh[1], hh[2]);
-        bool in = hc < Hs.nh;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) in = in && hh[a] - (uint32_t)B.h[a] < (uint32_t)B.e[a];
-        return in;
-    };
-    if (per <= STAGE_UNROLL) {
-#pragma unroll
-        for (uint32_t u = 0; u < STAGE_UNROLL; ++u)
-            if (u < per && own(c0 + u)) clear[hcn.cl[u]] = 0u;
-    } else {
-        for (uint32_t hc = c0; hc < c0 + per; ++hc)
-            if (own(hc)) clear[halo_global_cell(B, Hs, hc)] = 0u;
-    }
-}
-
 // The type tables of the walk, read into registers before the brick and its replica are known (one
 // entry per thread: n_types <= MAX_STAGED_TYPES gives n_types^2 <= BRICK_THREADS), so that their loads
 // overlap the brick's, then placed in LDS with the thresholds of the brick's frame: the force tables
@@ -144,6 +121,7 @@ struct TablePrefetch {  // raw words (registers, not a stack object)
     uint2 ri;
     uint4 pot0, pot1, pot2;
     float2 rm;
+    uint32_t o1a, o1b;
 };
 static_assert(sizeof(PairIdx) == 16 && sizeof(RxPairIdx) == 8 && sizeof(PotDev) == 48, "table entry sizes");
 
@@ -160,7 +138,11 @@ __device__ __forceinline__ TablePrefetch prefetch_tables(const Tables &T) {
         f.pot1 = q[1];
         f.pot2 = q[2];
     }
-    if (k < T.n_types) f.rm = T.rowmax[k];
+    if (k < T.n_types) {
+        f.rm = T.rowmax[k];
+        f.o1a = T.o1idx[k];
+        f.o1b = T.o1idx[k + 1];
+    }
     return f;
 }
 
@@ -181,6 +163,8 @@ __device__ __forceinline__ void place_tables(char *base, const Tables &T, const 
     st.thr = (float *)p;
     p += align16(4 * n2);
     st.reach = (float *)p;
+    p += align16(4 * nt);
+    st.o1 = (uint32_t *)p;
     if (k < n2) {
         reinterpret_cast<uint4 *>(ft.pidx)[k] = f.pi;
         reinterpret_cast<uint2 *>(st.o2)[k] = f.ri;
@@ -201,153 +185,182 @@ __device__ __forceinline__ void place_tables(char *base, const Tables &T, const 
         const float rf = reach_of(f.rm.x, f.rm.x >= 0.f, margin);
         ft.reach[k] = rf;
         st.reach[k] = fmaxf(rf, reach_of(f.rm.y, f.rm.y >= 0.f, margin));
+        st.o1[k] = f.o1a | ((f.o1b - f.o1a) << 16);
     }
-}
-
-// Orders the brick's own records so that those of the longest-reach types come first (a stable
-// partition of m.inner): a wave then holds particles of like stencil reach, and the short-reach waves
-// finish early instead of idling behind their long-reach lanes.  tmp: n_inner halves of free LDS.
-// block_exclusive_scan keeps one sum per wave of a SCAN_THREADS block.
-static_assert(BRICK_THREADS == SCAN_THREADS, "order_inner_by_reach scans a brick block with block_exclusive_scan");
-__device__ void order_inner_by_reach(const BrickSmem &m, uint32_t n_inner, const float *reach_tab, uint32_t nt,
-                                     uint16_t *tmp) {
-    __shared__ float s_rmax;
-    if (threadIdx.x == 0) {
-        float r = -1.f;
-        for (uint32_t t = 0; t < nt; ++t) r = fmaxf(r, reach_tab[t]);
-        s_rmax = r;
-    }
-    __syncthreads();
-    const float rmax = s_rmax;
-    auto longest = [&](uint32_t j) -> bool {
-        const uint32_t tw = __float_as_uint(m.P[j].w);
-        return !(tw & TW_DEAD) && reach_tab[tw_type(tw)] >= rmax;
-    };
-    uint32_t n0 = 0;
-    for (uint32_t c0 = 0; c0 < n_inner; c0 += BRICK_THREADS) {  // count the long-reach records
-        const uint32_t ii = c0 + threadIdx.x;
-        uint32_t tot;
-        block_exclusive_scan(ii < n_inner && longest(m.inner[ii]) ? 1u : 0u, &tot);
-        n0 += tot;
-    }
-    uint32_t o0 = 0, o1 = n0;
-    for (uint32_t c0 = 0; c0 < n_inner; c0 += BRICK_THREADS) {
-        const uint32_t ii = c0 + threadIdx.x;
-        uint32_t j = 0;
-        bool f = false;
-        if (ii < n_inner) {
-            j = m.inner[ii];
-            f = longest(j);
-        }
-        uint32_t t0;
-        const uint32_t r0 = block_exclusive_scan(f ? 1u : 0u, &t0);
-        if (ii < n_inner) tmp[f ? o0 + r0 : o1 + (ii - c0 - r0)] = (uint16_t)j;
-        o0 += t0;
-        o1 += min(n_inner - c0, (uint32_t)BRICK_THREADS) - t0;
-    }
-    __syncthreads();
-    for (uint32_t ii = threadIdx.x; ii < n_inner; ii += BRICK_THREADS) m.inner[ii] = tmp[ii];
-    __syncthreads();
 }
 
 // The walk of one brick over cur = x'(t): the pair forces of the brick's own records (2^-32 fixed
 // point, summed in LDS per wave), step t's reaction candidates (order 1 and 2, the draws of
 // k_brick_search), and each particle moved to step t+1 (or copied) into nxt as soon as its force is
 // complete.  flags: WALK_PROLOGUE, the first walk of a run (no candidates; moves replicas with steps
-// left, Philox step R.step + 1); WALK_LAST, the launch's last step.  Replicas neither searching nor moving are copied without a walk.  Four waves per
+// left, Philox step R.step + 1); WALK_LAST, the launch's last step.  Replicas neither searching nor moving are copied without a walk.  Five waves per
 // SIMD are asked of the register allocator (the move inside the walk loop would otherwise take the
 // kernel to three).
+struct WalkArgs {
+    Grid cur, nxt;
+    uint32_t *clear_counts, *clear_ovf;
+    const ReplicaDev *reps;
+    Tables T;
+    Topo topo;
+    const BrickDev *bricks;
+    Event *events;
+    uint32_t *ev_count, *slow, *change_counts, *err;
+    double dt;
+    uint32_t brick0, cap, max_states, max_halo, smem_bytes;
+    int32_t flags, radius, handler;
+};
+
 template <bool AH>
-__global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_brick_step(
-    Grid cur, Grid nxt, Grid clear, int flags, const ReplicaDev *reps, Tables T, Topo topo, const BrickDev *bricks,
-    uint32_t brick0, uint32_t cap, int radius, int handler, double dt, Event *events, uint32_t *ev_count,
-    uint32_t max_states, uint32_t max_halo, uint32_t smem_bytes, uint32_t *slow, uint32_t *change_counts,
-    uint32_t *err) {
+__global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(5))) void k_brick_step(WalkArgs) {
     extern __shared__ __align__(16) char smem[];
-    __shared__ ForceWave wave_lds[BRICK_WAVES];
-    const bool staged_types = T.n_types <= MAX_STAGED_TYPES;
-    TablePrefetch tpf;
-    if (staged_types) tpf = prefetch_tables(T);
-    const uint32_t bidx = brick0 + xcd_block(blockIdx.x, gridDim.x);
-    const BrickDev B = bricks[bidx];
-    // the halo counters load from the brick record alone, alongside the replica's record
-    const Halo Hs = make_halo(B);
-    const HaloCounts hcn = load_halo_counts(cur, B, Hs);
-    const ReplicaDev &R = reps[B.r];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *nxt.wl_count = 0u;
-        *clear.ovf_count = 0u;
-        change_counts[0] = 0u;  // changed records
-        change_counts[1] = 0u;  // records to move again
-    }
-    clear_own_cells(clear.counts, B, Hs, hcn);
-    if (!R.in_use) return;
-    const RepGeom geo = load_geom(R);
-    const StepPlan plan = plan_step(R, flags);  // block-uniform
-    const bool search = plan.active, integ = plan.integ;
-    const uint32_t step_next = plan.step_next;
-    if (!search && !integ) {  // copy only: no forces needed
-        for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
-            if (!(me.tw & TW_DEAD)) advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, false, me, 0, 0, 0, err);
-        });
-        return;
-    }
-    // a launch without reactions (handler > 1) covers every replica; else a replica's own choice wins
-    if (handler <= 1 && R.handler >= 0) handler = R.handler;
-    const bool rx_on = search && handler <= 1 && T.n_rx > 0;  // block-uniform
-    const bool o2_on = rx_on && T.has_o2;
-    const uint32_t nt = T.n_types;
-    const Frame F = make_frame(B, geo);
-    uint32_t total = 0xFFFFFFFFu, n_inner = 0;
+    __shared__ StepWave wave_lds[BRICK_WAVES];
     BrickSmem m;
     ForceTables ft;
     SearchTables st;
-    if (staged_types) {
-        if (table_bytes(nt, T.n_pots) + brick_smem_bytes(max_states, max_halo) > smem_bytes) {  // block-uniform
-            if (threadIdx.x == 0) atomicAdd(&err[ERR_LDS_LAYOUT], 1u);
+    WalkCtx wc;
+    float expand;
+    uint32_t r, nt, bidx;
+    const float *thr_tab, *reach_tab;
+    bool rx_on, o2_on;
+    bool inside;           // no halo cell across a boundary, and the brick with its halo spans less than half of
+                           // every axis: raw differences are minimum images
+    float lbox[3];         // FP32 box and axis modes for the general walk
+    {  // staging, and the bricks that are only copied
+        const WalkArgs &a = kernel_args<WalkArgs>();
+        nt = a.T.n_types;
+        const bool staged_types = nt <= MAX_STAGED_TYPES;
+        TablePrefetch tpf;
+        if (staged_types) tpf = prefetch_tables(a.T);
+        bidx = a.brick0 + xcd_block(blockIdx.x, gridDim.x);
+        const BrickDev &B = read_only(a.bricks + bidx);
+        // the halo counters load from the brick record alone, alongside the replica's record
+        const Halo Hs = make_halo(B);
+        const uint32_t per = cells_per_thread(Hs);
+        const HaloCells hcn = load_halo_cells(a.cur.counts, a.clear_counts, B, Hs, threadIdx.x * per, min(per, STAGE_CELLS));
+        for (uint32_t u = STAGE_CELLS; u < per; u += STAGE_CELLS)  // a large halo's further cells: cleared here
+            (void)load_halo_cells(a.cur.counts, a.clear_counts, B, Hs, threadIdx.x * per + u, min(per - u, STAGE_CELLS));
+        r = B.r;
+        const ReplicaDev &R = read_only(a.reps + r);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            *a.nxt.wl_count = 0u;
+            *a.clear_ovf = 0u;
+            a.change_counts[0] = 0u;  // changed records
+            a.change_counts[1] = 0u;  // records to move again
+        }
+        if (!R.in_use) return;
+        const RepGeom geo = load_geom(R);
+        const StepPlan plan = plan_step(R, a.flags);  // block-uniform
+        if (!plan.active && !plan.integ) {  // copy only: no forces needed
+            for_each_own_record(a.cur, B, a.cap, [&](uint32_t s, const State &me) {
+                if (!(me.tw & TW_DEAD))
+                    advance_particle(a.nxt, R, geo, a.T, a.topo, a.cap, a.dt, plan.step_next, false, me, 0, 0, 0, a.err);
+            });
             return;
         }
-        // with reactions on, the walk reaches the larger of the force and reaction cutoffs
-        place_tables(smem, T, tpf, F.margin, ft, st);
-        m = carve(smem + table_bytes(nt, T.n_pots), max_states, max_halo);
-        total = stage_brick(cur, B, geo, F, cap, m, max_states, Hs, hcn, &n_inner);
-    }
-    if (total == 0xFFFFFFFFu) {
-        list_slow_brick(slow, bidx);
-        return;
-    }
-    const WalkCtx wc = make_walk(B, geo, Hs, radius);
-    if (AH != (wc.whole == 0)) {  // launch and brick disagree (host invariant): refuse the brick
-        if (threadIdx.x == 0) atomicAdd(&err[ERR_LDS_LAYOUT], 1u);
-        return;
-    }
-    const float *thr_tab = o2_on ? st.thr : ft.thr;
-    const float *reach_tab = o2_on ? st.reach : ft.reach;
-    if (n_inner > BRICK_THREADS && 2 * n_inner <= transient_bytes(max_halo))  // block-uniform
-        order_inner_by_reach(m, n_inner, reach_tab, nt, (uint16_t *)m.rings);
-    const uint32_t r = B.r, step = plan.step;
-    const uint64_t seed = R.seed;
-    auto emit = [&](uint32_t rx, uint32_t s1, uint32_t s2, uint32_t h1, uint32_t h2, unsigned long long key) {
-        uint32_t p = atomicAdd(&ev_count[r], 1u);
-        if (p < R.ev_cap) {
-            Event ev;
-            ev.key = key;
-            ev.s1 = s1;
-            ev.s2 = s2;
-            ev.h1 = h1;
-            ev.h2 = h2;
-            ev.rx = rx;
-            ev.pad = 0;
-            events[R.ev_base + p] = ev;
-        } else {
-            atomicAdd(&err[ERR_EVENT_OVERFLOW], 1u);
+        rx_on = plan.active && replica_handler(R, a.handler) <= 1 && a.T.n_rx > 0;  // block-uniform
+        o2_on = rx_on && a.T.has_o2;
+        inside = true;
+        for (int k = 0; k < 3; ++k)
+            inside = inside && B.o[k] >= B.h[k] && B.o[k] + B.e[k] + B.h[k] <= B.dims[k] &&
+                     2 * (B.e[k] + 2 * B.h[k]) < B.dims[k];
+        const Frame F = make_frame(B, geo);
+        expand = F.expand;
+        for (int k = 0; k < 3; ++k) lbox[k] = F.L[k];
+        uint32_t total = 0xFFFFFFFFu;
+        if (staged_types) {
+            if (table_bytes(nt, a.T.n_pots) + brick_smem_bytes(a.max_states, a.max_halo) > a.smem_bytes) {  // block-uniform
+                if (threadIdx.x == 0) atomicAdd(&a.err[ERR_LDS_LAYOUT], 1u);
+                return;
+            }
+            // with reactions on, the walk reaches the larger of the force and reaction cutoffs
+            place_tables(smem, a.T, tpf, F.margin, ft, st);
+            m = carve(smem + table_bytes(nt, a.T.n_pots), a.max_states, a.max_halo);
+            total = stage_brick(a.cur, B, geo, F, a.cap, m, a.max_states, Hs, hcn);
         }
-    };
-    ForceWave &W = wave_lds[threadIdx.x / 64];
+        if (total == 0xFFFFFFFFu) {
+            list_slow_brick(a.slow, bidx, a.err);
+            return;
+        }
+        wc = make_walk(B, geo, Hs, a.radius);
+        if (AH != (wc.whole == 0)) {  // launch and brick disagree (host invariant): refuse the brick
+            if (threadIdx.x == 0) atomicAdd(&a.err[ERR_LDS_LAYOUT], 1u);
+            return;
+        }
+        thr_tab = o2_on ? st.thr : ft.thr;
+        reach_tab = o2_on ? st.reach : ft.reach;
+    }
+    StepWave &W = wave_lds[threadIdx.x / 64];
     const uint32_t lane = __lane_id();
     // a surviving pair (entry = owner lane << 16 | staged neighbour): the exact FP64 gates, the
     // pair force on the owner, and (each unordered pair once) the order-2 draws
     State me{};  // this lane's own record in the current round (the walk's owner records)
+    // The draws of the wave's reaction candidates: entries as the pairs', with NO_PARTNER for an order-1
+    // candidate.  Almost every batch of pairs holds a candidate or two, and a wave a dozen: one batch of draws
+    // for all of them costs the wave one Philox block instead of one a batch.
+    uint32_t n_draw = 0;  // wave-uniform
+    auto draw = [&]() {   // makes the last 64 listed draws
+        wave_lds_sync();
+        const uint32_t first = n_draw > 64u ? n_draw - 64u : 0u;
+        const uint32_t ent = first + lane < n_draw ? W.draw[first + lane] : NO_ENTRY;
+        const uint32_t ol = ent == NO_ENTRY ? 0u : ent >> 16, q = ent & 0xFFFFu;
+        State own;
+        own.x = __shfl(me.x, (int)ol);
+        own.y = __shfl(me.y, (int)ol);
+        own.z = __shfl(me.z, (int)ol);
+        own.tw = __shfl(me.tw, (int)ol);
+        own.h = __shfl(me.h, (int)ol);
+        n_draw = first;
+        if (ent == NO_ENTRY) return;
+        const WalkArgs &a = kernel_args<WalkArgs>();
+        const ReplicaDev &R = read_only(a.reps + r);
+        const uint32_t s1 = m.slot[W.j[ol]], t1 = tw_type(own.tw), step = plan_step(R, a.flags).step;
+        const bool pair = q != NO_PARTNER;
+        uint32_t s2 = s1, h2 = own.h, t2 = t1;
+        double d2 = 0.0;
+        if (pair) {
+            s2 = m.slot[q];
+            const State o = a.cur.bins[s2];
+            h2 = o.h;
+            t2 = tw_type(o.tw);
+            // distSquared(neighbor.pos, entry.pos) (CPUUncontrolledApproximation.cpp:108)
+            d2 = dist2(min_image(o.x - own.x, R.box[0], R.pbc[0]), min_image(o.y - own.y, R.box[1], R.pbc[1]),
+                       min_image(o.z - own.z, R.box[2], R.pbc[2]));
+        }
+        const RxPairIdx ri = st.o2[t1 * nt + t2];
+        const uint32_t o1 = st.o1[t1];
+        uint32_t k = pair ? ri.start : (o1 & 0xFFFFu);
+        const uint32_t ke = k + (pair ? ri.count : (o1 >> 16));
+        for (; k < ke; ++k) {
+            const uint32_t rx = pair ? a.T.o2list[k] : a.T.o1list[k];
+            const RxDev X = a.T.rx[rx];
+            if (!(X.rate > 0) || (pair && !(d2 < X.educt_dist2))) continue;
+            uint32_t x4[4];
+            philox(min(own.h, h2), step, (pair ? 2u : 1u) | (rx << 8), pair ? max(own.h, h2) : 0u, R.seed, x4);
+            if (!(u53(x4[0], x4[1]) < X.p_accept)) continue;
+            // entry1: the educt of type educts[0]; equal educt types: the lower handle
+            const bool me_first =
+                !pair || ((X.educts[0] != X.educts[1]) ? (t1 == X.educts[0]) : (own.h < h2));
+            const uint32_t p = atomicAdd(&a.ev_count[r], 1u);
+            if (p < R.ev_cap) {
+                Event ev;
+                ev.key = event_words(x4);
+                ev.s1 = me_first ? s1 : s2;
+                ev.s2 = me_first ? s2 : s1;
+                ev.h1 = me_first ? own.h : h2;
+                ev.h2 = me_first ? h2 : own.h;
+                ev.rx = rx;
+                ev.pad = 0;
+                a.events[R.ev_base + p] = ev;
+            } else {
+                atomicAdd(&a.err[ERR_EVENT_OVERFLOW], 1u);
+            }
+        }
+    };
+    auto list_draw = [&](bool want, uint32_t ent) {  // every lane of the wave comes along
+        const unsigned long long mk = __ballot(want);
+        if (want) W.draw[n_draw + rank_in_mask(mk)] = ent;
+        n_draw += (uint32_t)__popcll(mk);
+    };
     auto eval = [&](uint32_t ent) {
         // the owner's record from the owner lane's registers (every lane takes part in the shuffles)
         const uint32_t ol = ent == NO_ENTRY ? 0u : ent >> 16, q = ent & 0xFFFFu;
@@ -357,96 +370,114 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(4
         me_o.z = __shfl(me.z, (int)ol);
         me_o.tw = __shfl(me.tw, (int)ol);
         me_o.h = __shfl(me.h, (int)ol);
-        if (ent == NO_ENTRY) return;
-        const State &me = me_o;
-        const uint32_t s1 = W.s[ol], s2 = m.slot[q];
-        const State o = cur.bins[s2];
-        const uint32_t t1 = tw_type(me.tw), t2 = tw_type(o.tw);
-        // CPUCalculateForces.cpp:226-259: x_ij = shortestDifference(x_i, x_j), gate d2 < rc^2.
-        // The reaction gate measures distSquared(x_j, x_i) (CPUUncontrolledApproximation.cpp:108):
-        // the same square, since a - b = -(b - a) and the minimum image is symmetric in magnitude.
-        const double ddx = min_image(o.x - me.x, geo.box[0], geo.pbc[0]);
-        const double ddy = min_image(o.y - me.y, geo.box[1], geo.pbc[1]);
-        const double ddz = min_image(o.z - me.z, geo.box[2], geo.pbc[2]);
-        const double d2 = dist2(ddx, ddy, ddz);
-        long long px, py, pz, pe;
-        if (pair_fixed<false>(ft.pots, ft.pidx[t1 * nt + t2], ddx, ddy, ddz, d2, px, py, pz, pe)) {
-            if (fixed_saturated(px) || fixed_saturated(py) || fixed_saturated(pz)) atomicAdd(&err[ERR_FORCE_RANGE], 1u);
-            atomicAdd(&W.acc[0][ol], (unsigned long long)px);
-            atomicAdd(&W.acc[1][ol], (unsigned long long)py);
-            atomicAdd(&W.acc[2][ol], (unsigned long long)pz);
-        }
-        // each unordered pair once: the lower type finds it; equal types: the lower bin slot
-        if (o2_on && ((t2 > t1) || (t2 == t1 && s2 > s1))) {
-            const RxPairIdx ri = st.o2[t1 * nt + t2];
-            const uint32_t mh = me.h;
-            const uint32_t lo = mh < o.h ? mh : o.h, hi = mh < o.h ? o.h : mh;
-            for (uint32_t p = 0; p < ri.count; ++p) {
-                const uint32_t rx = T.o2list[ri.start + p];
-                const RxDev X = T.rx[rx];
-                if (!(X.rate > 0 && d2 < X.educt_dist2)) continue;
-                uint32_t x4[4];
-                philox(lo, step, 2u | (rx << 8), hi, seed, x4);
-                if (!(u53(x4[0], x4[1]) < X.p_accept)) continue;
-                // entry1: the educt of type educts[0]; equal educt types: the lower handle
-                const bool me_first = (X.educts[0] != X.educts[1]) ? (t1 == X.educts[0]) : (mh < o.h);
-                if (me_first) emit(rx, s1, s2, mh, o.h, event_key(handler, x4, X.rate));
-                else emit(rx, s2, s1, o.h, mh, event_key(handler, x4, X.rate));
+        bool react = false;
+        if (ent != NO_ENTRY) {
+            const WalkArgs &a = kernel_args<WalkArgs>();
+            const ReplicaDev &R = read_only(a.reps + r);
+            const State &me = me_o;
+            const uint32_t s2 = m.slot[q];
+            const State o = a.cur.bins[s2];
+            const uint32_t t1 = tw_type(me.tw), t2 = tw_type(o.tw);
+            // CPUCalculateForces.cpp:226-259: x_ij = shortestDifference(x_i, x_j), gate d2 < rc^2.
+            // The reaction gate measures distSquared(x_j, x_i) (CPUUncontrolledApproximation.cpp:108):
+            // the same square, since a - b = -(b - a) and the minimum image is symmetric in magnitude.
+            double ddx = o.x - me.x, ddy = o.y - me.y, ddz = o.z - me.z;
+            if (!inside) {
+                ddx = min_image(ddx, R.box[0], R.pbc[0]);
+                ddy = min_image(ddy, R.box[1], R.pbc[1]);
+                ddz = min_image(ddz, R.box[2], R.pbc[2]);
+            }
+            const double d2 = dist2(ddx, ddy, ddz);
+            long long px, py, pz, pe;
+            bool saturated;
+            if (pair_fixed<false>(ft.pots, ft.pidx[t1 * nt + t2], ddx, ddy, ddz, d2, px, py, pz, pe, &saturated)) {
+                if (saturated) atomicAdd(&a.err[ERR_FORCE_RANGE], 1u);
+                atomicAdd(&W.acc[0][ol], (unsigned long long)px);
+                atomicAdd(&W.acc[1][ol], (unsigned long long)py);
+                atomicAdd(&W.acc[2][ol], (unsigned long long)pz);
+            }
+            // order-2 candidates, each unordered pair once: the lower type finds it; equal types: the lower bin
+            // slot.  Their draws wait in a list of the wave (list_draw), with those of order 1
+            if (o2_on && ((t2 > t1) || (t2 == t1 && s2 > m.slot[W.j[ol]]))) {
+                const RxPairIdx ri = st.o2[t1 * nt + t2];
+                react = ri.count != 0 && d2 < (double)ri.maxr2_f * (1.0 + 1.0e-6);
             }
         }
+        if (__ballot(react)) list_draw(react, ent);
     };
-    for (uint32_t base = threadIdx.x & ~63u; base < n_inner; base += BRICK_THREADS) {  // wave-uniform
-        const uint32_t ii = base + lane;
-        bool valid = ii < n_inner;
-        uint32_t j = 0;
-        float4 pj = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (valid) {
-            j = m.inner[ii];
-            pj = m.P[j];
-            valid = !(__float_as_uint(pj.w) & TW_DEAD);
+    for (uint32_t q0 = threadIdx.x / 64 * 16;; q0 += BRICK_THREADS / 4) {  // wave-uniform
+        uint32_t n_quads;
+        {
+            const BrickDev &B = read_only(kernel_args<WalkArgs>().bricks + bidx);
+            n_quads = wave_quads(m, B, make_halo(B), W.quads, q0);
         }
+        if (q0 >= n_quads) break;
+        wave_lds_sync();
+        const OwnerLane ow = owner_lane(m, W.quads, q0, n_quads);
+        const uint32_t j = ow.j;
+        const bool valid = ow.valid;
         me = State{};
         uint32_t sj = 0;
-        if (valid) {
-            sj = m.slot[j];
-            me = cur.bins[sj];
-        }
-        W.s[lane] = sj;
-        W.acc[0][lane] = 0ull;
-        W.acc[1][lane] = 0ull;
-        W.acc[2][lane] = 0ull;
-        wave_lds_sync();
-        const uint32_t t = tw_type(me.tw);
-        if (rx_on && valid) {  // order 1 (CPUUncontrolledApproximation.cpp:81-95)
-            for (uint32_t k = T.o1idx[t]; k < T.o1idx[t + 1]; ++k) {
-                const uint32_t rx = T.o1list[k];
-                const RxDev X = T.rx[rx];
-                if (!(X.rate > 0)) continue;
-                uint32_t x4[4];
-                philox(me.h, step, 1u | (rx << 8), 0u, seed, x4);
-                if (!(u53(x4[0], x4[1]) < X.p_accept)) continue;
-                emit(rx, sj, sj, me.h, me.h, event_key(handler, x4, X.rate));
+        {
+            const WalkArgs &a = kernel_args<WalkArgs>();
+            if (valid) {
+                sj = m.slot[j];
+                me = a.cur.bins[sj];  // (first needed by the first batch of pairs)
             }
+            W.j[lane] = (uint16_t)j;
+            W.acc[0][lane] = 0ull;
+            W.acc[1][lane] = 0ull;
+            W.acc[2][lane] = 0ull;
+            wave_lds_sync();
         }
+        const uint32_t t = ow.t & TYP_MASK;
+        // order 1 (CPUUncontrolledApproximation.cpp:81-95)
+        if (rx_on) list_draw(valid && (st.o1[t] >> 16) != 0u, (lane << 16) | NO_PARTNER);
         const float reach = reach_tab[t];
-        const bool active = valid && !(me.tw & TW_OUTSIDE) && reach >= 0.f;
-        const float *thr_row = thr_tab + t * nt;
-        // prefilter, branch-free: one LDS read of the candidate, one of the threshold
-        auto keep = [&](uint32_t q, const float4 &pq) -> bool {
-            const uint32_t tw2 = __float_as_uint(pq.w);
-            float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
-            if constexpr (!AH) frame_min_image(F, dx, dy, dz);
-            const float d2p = prefilter_d2(dx, dy, dz);
-            const float thr = thr_row[tw_type(tw2)];
-            return (q != j) & (d2p < thr);  // dead / outside records hold NaN positions
-        };
-        pair_pipeline<AH>(wc, m.hstart, m.P, m.rings + (threadIdx.x / 64) * RING, active, m.hc_of[j], pj, reach, keep,
-                          eval);
+        const bool active = valid && !(ow.t & TYP_OUTSIDE) && reach >= 0.f;
+        const float4 pj = m.P[j];
+        char *wave_ring = m.rings + (threadIdx.x / 64) * WAVE_RING_BYTES;
+        if constexpr (AH) {
+            auto filter = [&](uint32_t ent) -> bool {
+                const uint32_t q = ent & 0xFFFFu, jo = W.j[ent >> 16];
+                const float4 a = m.P[jo], b = m.P[q];
+                return (q != jo) & (prefilter_d2(b.x - a.x, b.y - a.y, b.z - a.z) < thr_tab[m.typ[jo] * nt + m.typ[q]]);
+            };
+            // draws a full list as it comes, and the rest when the pairs are done
+            auto after = [&](bool done) -> bool {
+                if (n_draw >= 64 || (done && n_draw)) draw();
+                return n_draw != 0;
+            };
+            mfma_pipeline(wc, m.hstart, m.P, m.far, wave_ring, active, m.hc_of[j], pj, reach, expand, filter, eval, after);
+        } else {
+            const float *thr_row = thr_tab + t * nt;
+            // prefilter, branch-free: one LDS read of the candidate, one of the threshold
+            auto keep = [&](uint32_t q, const float4 &pq) -> bool {
+                float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
+                frame_min_image(wc.whole, lbox, dx, dy, dz);
+                const float d2p = prefilter_d2(dx, dy, dz);
+                const float thr = thr_row[m.typ[q]];
+                return (q != j) & (d2p < thr);  // dead / outside records are far away
+            };
+            auto eval_draw = [&](uint32_t ent) {
+                eval(ent);
+                if (n_draw >= 64) draw();
+            };
+            if (n_draw >= 64) draw();
+            pair_pipeline(wc, m.hstart, m.P, (uint32_t *)wave_ring, active, m.hc_of[j], keep, eval_draw);
+            if (n_draw) draw();
+        }
         wave_lds_sync();
         // the move with the finished pair force, from the owner's registers
         const long long fx = (long long)W.acc[0][lane], fy = (long long)W.acc[1][lane], fz = (long long)W.acc[2][lane];
         wave_lds_sync();
-        if (valid) advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, integ, me, fx, fy, fz, err);
+        if (valid) {
+            const WalkArgs &a = kernel_args<WalkArgs>();
+            const ReplicaDev &R = read_only(a.reps + r);
+            const StepPlan plan = plan_step(R, a.flags);
+            advance_particle(a.nxt, R, load_geom(R), a.T, a.topo, a.cap, a.dt, plan.step_next, plan.integ, me, fx, fy, fz,
+                             a.err);
+        }
     }
 }
 
@@ -499,7 +530,7 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
             if (me.tw & TW_DEAD) return;
             long long fx = 0, fy = 0, fz = 0, e = 0;
             if (!(me.tw & TW_OUTSIDE)) global_forces(cur, geo, cap, radius, T, s, me, fx, fy, fz, e);
-            if (R.active) search_one(cur, reps, T, cap, radius, handler, 0, events, ev_count, nullptr, 0, s, me, err);
+            if (R.active) search_one(cur, reps, T, cap, radius, 0, events, ev_count, nullptr, 0, s, me, err);
             advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, integ, me, fx, fy, fz, err);
         });
     }
@@ -507,7 +538,7 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
         __syncthreads();
         __threadfence();  // the listed bricks' candidates before the replica's list is read
     }
-    resolve_replica(cur, reps, T, cap, events, ev_count, rx_step, rx_total, 1, max_wl, edits, edit_count, edit_cap,
+    resolve_replica(cur, reps, T, cap, events, ev_count, rx_step, rx_total, handler, 1, max_wl, edits, edit_count, edit_cap,
                     recs, rec_count, err);
     if (n) release_slow_list(slow);
 }

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void k_topo_search(Grid cur, const ReplicaDev 
                 continue;
             }
             TopoEvent ev;
-            ev.key = event_key(1, x4, X.rate);
+            ev.key = order_key(1, event_words(x4), X.rate);
             ev.s_top = slot;
             ev.s_free = s2;
             ev.h_top = me.h;
