@@ -2452,6 +2452,54 @@ int rdy_count_types(rdy_engine *e, uint64_t *counts, uint32_t n_reps) {
     return RDY_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// Bricks for k_rdf_bricks: cubes of about 64 particles, fewer where that leaves compute units idle, with the halo in
+// at most 40 KB of LDS (four blocks a CU).  False: k_rdf takes the call (borders beyond half a periodic box, a halo
+// that does not fit).
+bool plan_rdf(const rdy_engine *e, uint32_t r, double rmax, const int *rad, uint32_t n_borders, RdfPlan &p) {
+    const HostReplica &H = e->reps_h[r];
+    const ReplicaDev &R = H.dev;
+    if (!(rmax > 0.0) || !(rmax < 1.0e30) || H.n_cells == 0) return false;
+    for (int a = 0; a < 3; ++a)
+        if (R.pbc[a] && R.dims[a] < 2 * rad[a] + 2) return false;
+    const double lam = (double)H.n_uploaded / (double)H.n_cells * e->lam_boost;
+    for (uint32_t edge = 8; edge >= 1; --edge) {
+        uint64_t halo = 1, own = 1, bricks = 1;
+        for (int a = 0; a < 3; ++a) {
+            p.e[a] = std::min<uint32_t>(edge, (uint32_t)R.dims[a]);
+            p.nb[a] = ((uint32_t)R.dims[a] + p.e[a] - 1) / p.e[a];
+            p.rad[a] = rad[a];
+            own *= p.e[a];
+            bricks *= p.nb[a];
+            halo *= p.e[a] + 2ull * (uint64_t)rad[a];
+        }
+        if (edge > 1 && (lam * (double)own > 128.0 || (edge > 2 && bricks < 512))) continue;
+        if (halo >= 60000 || bricks >= (1ull << 31)) continue;
+        const double mean = std::max(lam, 0.25) * (double)halo;
+        const double most = 1.2 * mean + 6.0 * std::sqrt(mean) + 64.0;
+        if (most > 60000.0) continue;
+        p.max_halo = (uint32_t)halo;
+        p.n_bricks = (uint32_t)bricks;
+        p.max_states = (uint32_t)most;
+        const double mine = std::max(lam, 0.25) * (double)own;
+        p.max_own = (uint32_t)(1.5 * mine + 6.0 * std::sqrt(mine) + 32.0);
+        const size_t lds = (rdf_smem_bytes(n_borders, p) + RDF_STATIC_LDS + LDS_GRAIN - 1) / LDS_GRAIN * LDS_GRAIN;
+        if (lds <= 40 * 1024 || (edge == 1 && lds <= 60 * 1024)) {
+            // as many blocks as the card holds at once (k_rdf_bricks' registers allow four a CU): each takes its share
+            p.n_blocks = std::min(p.n_bricks, 256u * (uint32_t)std::min<size_t>(4, LDS_PER_CU / lds));
+            return true;
+        }
+    }
+    return false;
+}
+
+}  // namespace
+
+extern "C" {
+
 int rdy_rdf_counts(rdy_engine *e, uint32_t r, const double *borders, uint32_t n_borders, const uint32_t *from_types,
                    uint32_t n_from_types, const uint32_t *to_types, uint32_t n_to_types, uint64_t *counts,
                    uint64_t *n_from) {
@@ -2483,33 +2531,52 @@ int rdy_rdf_counts(rdy_engine *e, uint32_t r, const double *borders, uint32_t n_
     const uint32_t outside_cap = (uint32_t)std::min<uint64_t>(e->max_particles, 1u << 20);
     const size_t nbins = n_borders - 1;
     size_t off_b = 0, off_m = off_b + 8 * (size_t)n_borders, off_c = (off_m + 8 * words + 15) & ~(size_t)15;
-    size_t off_n = off_c + 8 * nbins, off_o = off_n + 16, bytes = off_o + 4 * (size_t)outside_cap;
+    RdfPlan plan{};
+    const bool bricks = plan_rdf(e, r, rmax, rad, n_borders, plan);
+    const size_t full_words = bricks ? (plan.n_bricks + 31) / 32 : 0;
+    size_t off_n = off_c + 8 * nbins, off_f = off_n + 16, off_o = off_f + 4 * full_words,
+           bytes = off_o + 4 * (size_t)outside_cap;
     if ((rc = ensure_scratch(e, bytes))) return rc;
     char *base = (char *)e->scratch;
     double *d_b = (double *)(base + off_b);
     uint32_t *d_m = (uint32_t *)(base + off_m);
     unsigned long long *d_c = (unsigned long long *)(base + off_c);
     unsigned long long *d_n = (unsigned long long *)(base + off_n);
-    uint32_t *d_no = (uint32_t *)(d_n + 1);
+    uint32_t *d_no = (uint32_t *)(d_n + 1);  // records outside, bricks left to k_rdf
+    uint32_t *d_full = (uint32_t *)(base + off_f);
     uint32_t *d_out = (uint32_t *)(base + off_o);
     HIP_TRY(hipMemcpyAsync(d_b, borders, 8 * (size_t)n_borders, hipMemcpyHostToDevice, e->stream));
     HIP_TRY(hipMemcpyAsync(d_m, masks.data(), 8 * (size_t)words, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(hipMemsetAsync(d_c, 0, 8 * nbins + 16, e->stream));
-    ensure_wl(e);
+    HIP_TRY(hipMemsetAsync(d_c, 0, 8 * nbins + 16 + 4 * full_words, e->stream));
     const Grid g = e->grid(e->cur);
-    hipLaunchKernelGGL(k_rdf, dim3(blocks_for(e->max_particles, 256)), dim3(256), 0, e->stream, g,
-                       (const ReplicaDev *)e->reps, r, e->cap, (const double *)d_b, n_borders, (const uint32_t *)d_m,
-                       (const uint32_t *)(d_m + words), rad[0], rad[1], rad[2], d_c, d_n, d_out, outside_cap, d_no,
-                       (uint32_t)e->max_particles);
-    uint32_t no = 0;
-    HIP_TRY(hipMemcpyAsync(&no, d_no, 4, hipMemcpyDeviceToHost, e->stream));
+    auto general = [&](const uint32_t *only) {
+        ensure_wl(e);
+        hipLaunchKernelGGL(k_rdf, dim3(blocks_for(e->max_particles, 256)), dim3(256), 0, e->stream, e->grid(e->cur),
+                           (const ReplicaDev *)e->reps, r, e->cap, (const double *)d_b, n_borders,
+                           (const uint32_t *)d_m, (const uint32_t *)(d_m + words), rad[0], rad[1], rad[2], d_c, d_n,
+                           d_out, outside_cap, d_no, (uint32_t)e->max_particles, plan, only);
+    };
+    if (bricks)
+        hipLaunchKernelGGL(k_rdf_bricks, dim3(plan.n_blocks), dim3(256),
+                           rdf_smem_bytes(n_borders, plan), e->stream, g, (const ReplicaDev *)e->reps, r, e->cap, plan,
+                           (const double *)d_b, n_borders, (const uint32_t *)d_m, (const uint32_t *)(d_m + words), d_c,
+                           d_n, d_out, outside_cap, d_no, d_no + 1, d_full);
+    else general(nullptr);
+    uint32_t left[2] = {0, 0}, &no = left[0];
+    HIP_TRY(hipMemcpyAsync(left, d_no, 8, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
+    if (left[1]) {
+        general(d_full);
+        HIP_TRY(hipMemcpyAsync(left, d_no, 4, hipMemcpyDeviceToHost, e->stream));
+        HIP_TRY(hipStreamSynchronize(e->stream));
+    }
     if (no > outside_cap) return set_err(RDY_ERR_CAPACITY, "radial distribution: too many particles outside the box");
     if (no) {
         const uint64_t pairs = (uint64_t)no * e->max_particles;
         if ((pairs + 255) / 256 > 0x7FFFFFFFull)
             return set_err(RDY_ERR_CAPACITY, "radial distribution: too many particles outside the box");
-        hipLaunchKernelGGL(k_rdf_outside, dim3((uint32_t)((pairs + 255) / 256)), dim3(256), 0, e->stream, g,
+        ensure_wl(e);
+        hipLaunchKernelGGL(k_rdf_outside, dim3((uint32_t)((pairs + 255) / 256)), dim3(256), 0, e->stream, e->grid(e->cur),
                            (const ReplicaDev *)e->reps, r, (const double *)d_b, n_borders, (const uint32_t *)d_m,
                            (const uint32_t *)(d_m + words), d_c, (const uint32_t *)d_out, (const uint32_t *)d_no,
                            (uint32_t)e->max_particles);
