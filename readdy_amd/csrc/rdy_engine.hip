@@ -137,6 +137,7 @@ struct rdy_engine {
     double lam_boost = 1.0;                                  // raised until few bricks outgrow their staging capacity
     uint32_t max_states_cfg = 0, brick_cfg[3] = {0, 0, 0};  // as the caller set them (0: chosen here)
     size_t brick_smem = 0;
+    size_t brick_static_lds = 0;
     size_t tables_lds = 0;  // bytes of brick_smem reserved for the per-block type tables
     size_t lds_limit = 65536;
     std::vector<BrickDev> bricks_h;
@@ -1042,12 +1043,13 @@ int configure_bricks(rdy_engine *e, double lam, const int32_t *dims, double scal
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device) == hipSuccess && v > 0)
         e->lds_limit = (size_t)v;
     // static LDS of the brick kernels comes out of the same per-workgroup budget
-    size_t static_lds = 0;
+    size_t &static_lds = e->brick_static_lds;
     const void *kernels[] = {(const void *)k_brick_step<true>,         (const void *)k_brick_step<false>,
                              (const void *)k_brick<MODE_FORCES, true>, (const void *)k_brick<MODE_FORCES, false>,
                              (const void *)k_brick<MODE_REBIN, false>, (const void *)k_brick_search<true>,
                              (const void *)k_brick_search<false>};
     for (const void *k : kernels) {
+        if (e->brick_lam > 0) break;  // known from the first fit
         hipFuncAttributes fa;
         if (hipFuncGetAttributes(&fa, k) == hipSuccess) static_lds = std::max(static_lds, (size_t)fa.sharedSizeBytes);
     }
