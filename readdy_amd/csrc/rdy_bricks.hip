@@ -98,6 +98,8 @@ struct BrickSmem {  // carved out of dynamic LDS
     char *rings;       // [BRICK_WAVES][WAVE_RING_BYTES]
     uint32_t far;      // index of the far record
 };
+// A flagged record (typ >= TYP_OUTSIDE) is no neighbour: the matrix-core walk refuses it by its distance, the general
+// walk by the flag; a table of the types is indexed by typ & TYP_MASK wherever a flagged record can come.
 constexpr uint8_t TYP_OUTSIDE = 0x40, TYP_DEAD = 0x80, TYP_MASK = 0x0F;
 
 __device__ __forceinline__ BrickSmem carve(char *base, uint32_t max_states, uint32_t max_halo) {
@@ -1148,11 +1150,10 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
                     const float *thr_row = ft.thr + t * nt;
                     // prefilter, branch-free: one LDS read of the candidate, one of the threshold
                     auto keep = [&](uint32_t q, const float4 &pq) -> bool {
+                        const uint32_t tq = m.typ[q];
                         float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
                         frame_min_image(F.whole, F.L, dx, dy, dz);
-                        const float d2p = prefilter_d2(dx, dy, dz);
-                        const float thr = thr_row[m.typ[q]];
-                        return (q != j) & (d2p < thr);  // dead / outside records are far away
+                        return (q != j) & (tq < TYP_OUTSIDE) & (prefilter_d2(dx, dy, dz) < thr_row[tq & TYP_MASK]);
                     };
                     pair_pipeline(wc, m.hstart, m.P, (uint32_t *)wave_ring, active, m.hc_of[j], keep, eval);
                 }
@@ -1346,13 +1347,13 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
             } else {
                 const float *thr_row = st.thr + t * nt;
                 auto keep = [&](uint32_t q, const float4 &pq) -> bool {
-                    const uint32_t t2 = m.typ[q];
+                    const uint32_t tq = m.typ[q], t2 = tq & TYP_MASK;
                     float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
                     frame_min_image(F.whole, F.L, dx, dy, dz);
                     const float d2p = prefilter_d2(dx, dy, dz);
                     const float thr = thr_row[t2];
                     const uint32_t sq = m.slot[q];
-                    return ((t2 > t) | ((t2 == t) & (sq > sj))) & (d2p < thr);
+                    return ((t2 > t) | ((t2 == t) & (sq > sj))) & (tq < TYP_OUTSIDE) & (d2p < thr);
                 };
                 pair_pipeline(wc, m.hstart, m.P, (uint32_t *)wave_ring, active, m.hc_of[j], keep, eval);
             }

@@ -453,11 +453,10 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(5
             const float *thr_row = thr_tab + t * nt;
             // prefilter, branch-free: one LDS read of the candidate, one of the threshold
             auto keep = [&](uint32_t q, const float4 &pq) -> bool {
+                const uint32_t tq = m.typ[q];
                 float dx = pq.x - pj.x, dy = pq.y - pj.y, dz = pq.z - pj.z;
                 frame_min_image(wc.whole, lbox, dx, dy, dz);
-                const float d2p = prefilter_d2(dx, dy, dz);
-                const float thr = thr_row[m.typ[q]];
-                return (q != j) & (d2p < thr);  // dead / outside records are far away
+                return (q != j) & (tq < TYP_OUTSIDE) & (prefilter_d2(dx, dy, dz) < thr_row[tq & TYP_MASK]);
             };
             auto eval_draw = [&](uint32_t ent) {
                 eval(ent);

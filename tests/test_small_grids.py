@@ -65,3 +65,70 @@ def test_forces_and_steps_on_short_axes(radius, dims, pbc, brick):
     assert np.array_equal(e.reaction_totals(r), e2.reaction_totals(r2))
     e.close()
     e2.close()
+
+
+def _walled(n_types, radius, seed=8, **kw):
+    """two cells on the periodic axis (the general walk), open axes with a fifth of the particles beyond their walls"""
+    box = [6.0, 2.0 / radius * (1.0 + 1e-9), 5.0]
+    rng = np.random.default_rng(seed)
+    n = 240
+    pos = (rng.random((n, 3)) - 0.5) * box
+    out = rng.random(n) < 0.2
+    axis = rng.choice([0, 2], n)
+    beyond = np.where(rng.random(n) < 0.5, -1.0, 1.0) * (0.5 * np.array(box)[axis] + 0.4 * rng.random(n))
+    pos[out, axis[out]] = beyond[out]
+    types = rng.integers(0, n_types, n).astype(np.uint32)
+    pots = [(L.POT_HARMONIC_REPULSION, a, b, [10.0, 1.0]) for a in range(n_types) for b in range(a, n_types)]
+    rxs = [dict(kind=L.RX_FUSION, educts=[a, (a + 1) % n_types], products=[(a + 2) % n_types], rate=60.0,
+                educt_distance=0.9) for a in range(n_types)]
+    rxs += [dict(kind=L.RX_FISSION, educts=[a], products=[a, (a + 1) % n_types], rate=20.0, product_distance=0.8)
+            for a in range(n_types)]
+    e = Engine(n_types, np.ones(n_types), potentials=pots, reactions=rxs, cell_radius=radius, nl_cutoff=1.0, **kw)
+    r = e.add_replica(box, (0, 1, 0), seed=3, max_particles=8 * n)
+    e.set_particles(r, pos, types)
+    return e, r, box, pos, types, pots
+
+
+@pytest.mark.parametrize("n_types", [2, 4, 5, 8, 16])
+@pytest.mark.parametrize("radius", [1, 2])
+def test_outside_and_dead_records_are_no_neighbours_in_the_general_walk(n_types, radius):
+    """The staged species of such a record carries a flag beyond every table of the species: it is refused by that
+    flag.  Forces against the oracle; separate actions and fused runs, and separate reactions right after a fused run
+    (whose buffer holds the withdrawn copies), against the bin-reading path."""
+    e, r, box, pos, types, pots = _walled(n_types, radius)
+    s, q, *_ = _walled(n_types, radius, lds_states=1)
+    o = po.System(n_types, box, [0, 1, 0], diffusion=[1.0] * n_types)
+    for _, a, b, p in pots:
+        o.add_pair_potential(po.POT_HARMONIC_REPULSION, a, b, p)
+    o.add_particles(pos, types.astype(np.int32), ids=np.arange(len(types)))
+    o.nl_setup(1.0)
+    energy = o.calculate_forces()
+    f_ref = o.particles()[3][np.argsort(o.particles()[2])]
+    for x, i in ((e, r), (s, q)):
+        x.calculate_forces()
+        f = x.get_forces(i)[0]
+        assert np.linalg.norm(f - f_ref) <= 1e-5 * np.linalg.norm(f_ref)
+        assert abs(x.energy(i) - energy) <= 1e-5 * abs(energy)
+
+    def same():
+        for a, b in zip((*e.get_particles(r), e.energy(r)), (*s.get_particles(q), s.energy(q))):
+            assert np.array_equal(a, b)
+        assert np.array_equal(e.get_forces(r)[0], s.get_forces(q)[0])
+        assert np.array_equal(e.reaction_totals(r), s.reaction_totals(q))
+
+    for rounds in range(3):
+        for x in (e, s):
+            x.run(L.HANDLER_UA, 2e-3, 2 + rounds)
+            x.react(L.HANDLER_UA, 2e-3)
+            x.update_neighbor_list()
+            x.calculate_forces()
+        same()
+        for x in (e, s):
+            x.integrate(1e-3)
+            x.update_neighbor_list()
+            x.react(L.HANDLER_GILLESPIE, 2e-3)
+            x.calculate_forces()
+        same()
+    assert e.reaction_totals(r).sum() > 0
+    e.close()
+    s.close()
