@@ -46,7 +46,9 @@ struct HostReplica {
     uint32_t tt_base = 0, n_tt = 0;  // topologies (their types) for spatial topology reactions
     bool has_particles = false;  // particles were uploaded since the replica was added
     uint64_t n_uploaded = 0;     // particles of the last upload
+    uint64_t n_live = 0;         // particles of the last upload or readback
     uint64_t handle_guess = 0;   // handles a readback makes room for (the last one read and some growth)
+    uint64_t handle_top = 0;     // and at least: past the highest handle that an earlier one found beyond its room
     ReplicaDev dev{};
 };
 
@@ -1633,6 +1635,8 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
                            (uint32_t)e->max_particles, e->err);
     }
     H.handle_guess = hn + (uint64_t)hn / 2 + 4096;
+    H.handle_top = 0;
+    H.n_live = n;
     e->wl_valid = false;
     e->version++;
     return check_errors(e);
@@ -1701,76 +1705,152 @@ static int copy_out(rdy_engine *e, const HostCopy (&c)[4]) {
     return drain(half ^ 1);
 }
 
+struct RowsOut {  // the caller's arrays (null: not asked for)
+    double *pos;
+    uint32_t *types, *handles;
+    double *forces;
+};
+
+// device rows in one piece of scratch, from byte offset `at` on
+struct RowsLayout {
+    size_t pos, forces, types, handles, end;
+    RowsLayout(const RowsOut &o, size_t at, uint64_t n) : pos(at) {
+        forces = pos + (o.pos ? 24 * n : 0);
+        types = forces + (o.forces ? 24 * n : 0);
+        handles = types + (o.types ? 4 * n : 0);
+        end = handles + (o.handles ? 4 * n : 0);
+    }
+    Rows rows(const RowsOut &o, char *base, const double *force_in) const {
+        return Rows{o.pos ? (double *)(base + pos) : nullptr, o.types ? (uint32_t *)(base + types) : nullptr,
+                    o.handles ? (uint32_t *)(base + handles) : nullptr, force_in,
+                    o.forces ? (double *)(base + forces) : nullptr};
+    }
+};
+
+// m rows from the device to the caller
+static int rows_out(rdy_engine *e, const RowsOut &o, const RowsLayout &l, const char *base, uint64_t m) {
+    const HostCopy all[4] = {{o.pos, base + l.pos, o.pos ? 24 * m : 0},
+                             {o.forces, base + l.forces, o.forces ? 24 * m : 0},
+                             {o.types, base + l.types, o.types ? 4 * m : 0},
+                             {o.handles, base + l.handles, o.handles ? 4 * m : 0}};
+    return copy_out(e, all);
+}
+
+// Whether a bitmap over `handles` handles places a replica's n particles (k_rank_mark).  Handles are never given out
+// again, so a long run's lie ever further apart, and a readback by the bitmap costs by the handles issued (0.1 ms per
+// 2^30), the host's sort 0.07 ms and 45 ns a particle whatever they are.  Measured readbacks, bitmap just below the
+// line and sort just above: 65 and 130 us at 500 particles (8.7e7 handles issued), 168 and 290 us at 5,000 (8.7e8);
+// at 30,000 the bitmap of all 2^32 takes 0.52 ms, the sort 1.3.
+static bool rank_by_bitmap(uint64_t handles, uint64_t n) {
+    return handles <= std::max<uint64_t>(1ull << 23, n << 18);
+}
+
+// The rows of replica r where a bitmap does not serve: the records are listed, the host sorts the list by handle
+// (records that share one, after the 32-bit counter has wrapped, come next to each other), the device writes the rows.
+static int gather_sorted(rdy_engine *e, uint32_t r, uint64_t ncap, const RowsOut &o, uint64_t *n) {
+    HostReplica &H = e->reps_h[r];
+    const Grid g = e->grid(e->cur);
+    const uint32_t blocks = std::min(blocks_for(H.n_cells, 256), RANK_BLOCKS);
+    std::vector<unsigned long long> list;
+    uint64_t room = H.n_live;
+    for (;;) {
+        if (int rc = ensure_scratch(e, 64 + 8 * room)) return rc;
+        uint32_t *count = (uint32_t *)e->scratch;
+        unsigned long long *d_list = (unsigned long long *)((char *)e->scratch + 64);
+        HIP_TRY(hipMemsetAsync(count, 0, 4, e->stream));
+        hipLaunchKernelGGL(k_list_live, dim3(blocks), dim3(256), 0, e->stream, g, r, e->cap, (uint32_t)H.cell_base,
+                           (uint32_t)H.n_cells, (uint32_t)room, count, d_list);
+        uint32_t live = 0;
+        HIP_TRY(hipMemcpyAsync(&live, count, 4, hipMemcpyDeviceToHost, e->stream));
+        HIP_TRY(hipStreamSynchronize(e->stream));
+        H.n_live = live;
+        if (live > room) {  // it has grown since
+            room = live;
+            continue;
+        }
+        list.resize(live);
+        if (live) HIP_TRY(hipMemcpyAsync(list.data(), d_list, 8ull * live, hipMemcpyDeviceToHost, e->stream));
+        HIP_TRY(hipStreamSynchronize(e->stream));
+        break;
+    }
+    std::sort(list.begin(), list.end());
+    *n = list.size();
+    if (list.empty()) return RDY_OK;
+    const uint64_t m = std::min<uint64_t>(list.size(), ncap);
+    const RowsLayout l(o, 8 * m, m);
+    if (int rc = ensure_scratch(e, l.end)) return rc;
+    char *base = (char *)e->scratch;
+    HIP_TRY(hipMemcpyAsync(base, list.data(), 8 * m, hipMemcpyHostToDevice, e->stream));
+    hipLaunchKernelGGL(k_list_write, dim3(blocks_for(m, 256)), dim3(256), 0, e->stream, g,
+                       (const unsigned long long *)base, (uint32_t)m, l.rows(o, base, (const double *)e->force_out));
+    return rows_out(e, o, l, base, m);
+}
+
 // the live particles of replica r in ascending handle order (cap 0: their number only)
-static int gather(rdy_engine *e, uint32_t r, uint64_t cap, double *pos, uint32_t *types, uint32_t *handles,
-                  double *forces, uint64_t *n) {
+static int gather(rdy_engine *e, uint32_t r, uint64_t cap, const RowsOut &o, uint64_t *n) {
     int rc = check_replica(e, r);
     if (rc) return rc;
     HostReplica &H = e->reps_h[r];
     const uint64_t ncap = std::min<uint64_t>(cap, e->max_particles);
     const Grid g = e->grid(e->cur);
     const uint32_t blocks = std::min(blocks_for(H.n_cells, 256), RANK_BLOCKS);
-    for (int attempt = 0;; ++attempt) {
-        // the bitmap covers the handles of the last read and half as many again; a replica that has grown
-        // past it says how many it has, and the readback is repeated
+    for (;;) {
+        // the bitmap covers the handles of the last read and half as many again; a replica that has grown past it
+        // says how far, and the readback is repeated
         const uint64_t hmax = std::min<uint64_t>(H.handle_guess, 1ull << 32), per = 32ull * RANK_GROUP_WORDS;
+        if (ncap && !rank_by_bitmap(hmax, H.n_live)) return gather_sorted(e, r, ncap, o, n);
         const uint32_t groups = ncap ? (uint32_t)((hmax + per - 1) / per) : 0u;
         const uint32_t tiles = (groups + RANK_TILE - 1) / RANK_TILE, words = groups * RANK_GROUP_WORDS;
         const size_t off_sum = 4ull * groups, off_bits = (off_sum + 4ull * tiles + 63) & ~(size_t)63;
-        const size_t off_info = off_bits + 4ull * words, off_pos = off_info + 64;
-        const size_t off_for = off_pos + (pos ? 24 * ncap : 0), off_ty = off_for + (forces ? 24 * ncap : 0);
-        const size_t off_h = off_ty + (types ? 4 * ncap : 0), end = off_h + (handles ? 4 * ncap : 0);
-        if ((rc = ensure_scratch(e, end))) return rc;
+        const size_t off_info = off_bits + 4ull * words;
+        const RowsLayout l(o, off_info + 64, ncap);
+        if ((rc = ensure_scratch(e, l.end))) return rc;
         char *base = (char *)e->scratch;
         uint32_t *pre = (uint32_t *)base, *sums = (uint32_t *)(base + off_sum), *bits = (uint32_t *)(base + off_bits);
-        HIP_TRY(hipMemsetAsync(base + off_bits, 0, off_pos - off_bits, e->stream));
+        RankInfo *d_info = (RankInfo *)(base + off_info);
+        HIP_TRY(hipMemsetAsync(base + off_bits, 0, l.pos - off_bits, e->stream));
         hipLaunchKernelGGL(k_rank_mark, dim3(blocks), dim3(256), 0, e->stream, g, (const ReplicaDev *)e->reps, r, e->cap,
-                           (uint32_t)H.cell_base, (uint32_t)H.n_cells, bits, words, (RankInfo *)(base + off_info));
+                           (uint32_t)H.cell_base, (uint32_t)H.n_cells, bits, words, d_info);
         if (ncap) {
             if (tiles > 1)
                 hipLaunchKernelGGL(k_rank_sums, dim3(tiles), dim3(SCAN_THREADS), 0, e->stream, (const uint32_t *)bits,
                                    groups, sums);
             hipLaunchKernelGGL(k_rank_prefix, dim3(tiles), dim3(SCAN_THREADS), 0, e->stream, (const uint32_t *)bits,
-                               groups, (const uint32_t *)sums, pre);
+                               groups, (const uint32_t *)sums, pre, d_info);
             hipLaunchKernelGGL(k_rank_write, dim3(blocks), dim3(256), 0, e->stream, g, r, e->cap, (uint32_t)H.cell_base,
                                (uint32_t)H.n_cells, (const uint32_t *)bits, words, (const uint32_t *)pre, (uint32_t)ncap,
-                               pos ? (double *)(base + off_pos) : nullptr, types ? (uint32_t *)(base + off_ty) : nullptr,
-                               handles ? (uint32_t *)(base + off_h) : nullptr, (const double *)e->force_out,
-                               forces ? (double *)(base + off_for) : nullptr);
+                               l.rows(o, base, (const double *)e->force_out));
         }
         // a small answer comes back whole with the count, in one copy and one wait
-        const bool small = end - off_info <= STAGING_SMALL;
-        const size_t first = small ? end - off_info : sizeof(RankInfo);
+        const bool small = l.end - off_info <= STAGING_SMALL;
+        const size_t first = small ? l.end - off_info : sizeof(RankInfo);
         if ((rc = ensure_staging(e, STAGING_SMALL))) return rc;
         HIP_TRY(hipMemcpyAsync(e->staging, base + off_info, first, hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
         RankInfo info;
         std::memcpy(&info, e->staging, sizeof info);
-        H.handle_guess = info.handle_next + (uint64_t)info.handle_next / 2 + 4096;
-        if (info.beyond && attempt == 0) continue;
+        H.n_live = info.live;
+        H.handle_top = std::max<uint64_t>(H.handle_top, info.beyond ? info.beyond + 1ull : 0ull);
+        H.handle_guess = std::max<uint64_t>(info.handle_next + (uint64_t)info.handle_next / 2 + 4096, H.handle_top);
+        if (info.beyond) continue;  // (the next attempt covers every handle, or sorts)
+        if (ncap && info.bits != info.live) return gather_sorted(e, r, ncap, o, n);
         *n = info.live;
         const uint64_t m = std::min<uint64_t>(info.live, ncap);
         if (m == 0) return RDY_OK;
-        if (small) {
-            const char *w = e->staging;
-            if (pos) std::memcpy(pos, w + (off_pos - off_info), 24 * m);
-            if (forces) std::memcpy(forces, w + (off_for - off_info), 24 * m);
-            if (types) std::memcpy(types, w + (off_ty - off_info), 4 * m);
-            if (handles) std::memcpy(handles, w + (off_h - off_info), 4 * m);
-            return RDY_OK;
-        }
-        const HostCopy all[4] = {{pos, base + off_pos, pos ? 24 * m : 0},
-                                 {forces, base + off_for, forces ? 24 * m : 0},
-                                 {types, base + off_ty, types ? 4 * m : 0},
-                                 {handles, base + off_h, handles ? 4 * m : 0}};
-        return copy_out(e, all);
+        if (!small) return rows_out(e, o, l, base, m);
+        const char *w = e->staging - off_info;
+        if (o.pos) std::memcpy(o.pos, w + l.pos, 24 * m);
+        if (o.forces) std::memcpy(o.forces, w + l.forces, 24 * m);
+        if (o.types) std::memcpy(o.types, w + l.types, 4 * m);
+        if (o.handles) std::memcpy(o.handles, w + l.handles, 4 * m);
+        return RDY_OK;
     }
 }
 
 int rdy_get_particles(rdy_engine *e, uint32_t r, uint64_t cap, double *pos, uint32_t *types, uint32_t *handles,
                       uint64_t *n) {
     uint64_t dummy;
-    return gather(e, r, cap, pos, types, handles, nullptr, n ? n : &dummy);
+    return gather(e, r, cap, {pos, types, handles, nullptr}, n ? n : &dummy);
 }
 
 int rdy_get_forces(rdy_engine *e, uint32_t r, uint64_t cap, double *forces, uint32_t *handles, uint64_t *n) {
@@ -1779,7 +1859,7 @@ int rdy_get_forces(rdy_engine *e, uint32_t r, uint64_t cap, double *forces, uint
     if (rc) return rc;
     if (!e->force_out) return set_err(RDY_ERR_STATE, "no forces have been calculated");
     uint64_t dummy;
-    return gather(e, r, cap, nullptr, nullptr, handles, forces, n ? n : &dummy);
+    return gather(e, r, cap, {nullptr, nullptr, handles, forces}, n ? n : &dummy);
 }
 
 static int set_terms(rdy_engine *e, uint32_t r, int kind, uint64_t n, const uint32_t *idx, int arity, const double *k,
@@ -2331,6 +2411,16 @@ int rdy_replica_set_handler(rdy_engine *e, uint32_t r, int handler) {
     if (handler < -1 || handler > RDY_HANDLER_NONE) return set_err(RDY_ERR_INVALID, "unknown reaction handler");
     const int32_t h = handler;
     return put_field(e, r, offsetof(ReplicaDev, handler), h);
+}
+
+int rdy_set_next_handle(rdy_engine *e, uint32_t r, uint32_t next) {
+    int rc = check_replica(e, r);
+    if (rc) return rc;
+    if (e->in_session) return set_err(RDY_ERR_STATE, "a run is open: finish it with rdy_run_end");
+    uint32_t now = 0;
+    if ((rc = get_field(e, r, offsetof(ReplicaDev, handle_next), &now))) return rc;
+    if (next < now) return set_err(RDY_ERR_INVALID, "handles are not given out again");
+    return put_field(e, r, offsetof(ReplicaDev, handle_next), next);
 }
 
 int rdy_synchronize(rdy_engine *e) {

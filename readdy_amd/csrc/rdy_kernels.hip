@@ -1452,13 +1452,17 @@ __global__ void k_upload(Grid g, ReplicaDev *reps, uint32_t r, uint32_t n, uint3
 // k_rank_sums / k_rank_prefix form the number of bits before every RANK_GROUP_WORDS words, and k_rank_write puts
 // each record at prefix + bits below its own.  Only the replica's own cells and the overflow region are read.
 // The order used to be the host's work: 300,000 particles' forces took 24 ms to read back, nearly all of it the
-// host's sort of the handles and the permuted copies, and now take 0.7 ms.
+// host's sort of the handles and the permuted copies, and now take 0.7 ms.  Where the handles are far apart
+// (rank_by_bitmap), or two records share one, the records are listed (k_list_live) and the host sorts the list.
 constexpr uint32_t RANK_GROUP_WORDS = 8;              // 256 handles, one 32 B sector of the bitmap
 constexpr uint32_t RANK_PER_THREAD = 4;               // groups of a thread of k_rank_sums / k_rank_prefix
 constexpr uint32_t RANK_TILE = 256 * RANK_PER_THREAD;  // groups of a block
 
-struct RankInfo {  // what k_rank_mark reports to the host
-    uint32_t live, beyond, handle_next, pad;
+struct RankInfo {  // what the kernels report to the host
+    uint32_t live;         // records
+    uint32_t beyond;       // the highest handle beyond the bitmap, if there is one (0: none)
+    uint32_t bits;         // set bits (fewer than records: two share a handle)
+    uint32_t handle_next;
 };
 
 // fn(slot) for the records of the replica's cells and of the overflow region, spread over the grid's threads
@@ -1477,8 +1481,8 @@ __device__ __forceinline__ void replica_records(const Grid &g, uint32_t cap, uin
     for (uint32_t o = i0; o < no; o += stride) fn(g.nbin + o);
 }
 
-// words = 0: count only.  A handle beyond the bitmap (its size is the host's estimate) is reported: the host
-// then repeats with the exact size.
+// words = 0: count only.  The highest handle beyond the bitmap (its size is the host's estimate) is reported: the
+// host then repeats with room for it.
 __global__ __launch_bounds__(256) void k_rank_mark(Grid cur, const ReplicaDev *reps, uint32_t r, uint32_t cap,
                                                    uint32_t cell_base, uint32_t n_cells, uint32_t *bits,
                                                    uint32_t words, RankInfo *info) {
@@ -1489,7 +1493,7 @@ __global__ __launch_bounds__(256) void k_rank_mark(Grid cur, const ReplicaDev *r
         ++live;
         if (words == 0) return;
         if ((th.y >> 5) < words) atomicOr(&bits[th.y >> 5], 1u << (th.y & 31u));
-        else info->beyond = 1u;
+        else atomicMax(&info->beyond, th.y);
     });
     uint32_t total;
     block_exclusive_scan(live, &total);
@@ -1517,7 +1521,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_rank_sums(const uint32_t *bits
 
 // bits before each group (a block adds up the tiles before its own: at most 2^14, for 2^32 handles)
 __global__ __launch_bounds__(SCAN_THREADS) void k_rank_prefix(const uint32_t *bits, uint32_t groups, const uint32_t *sums,
-                                                              uint32_t *prefix) {
+                                                              uint32_t *prefix, RankInfo *info) {
     uint32_t before = 0, base;
     for (uint32_t k = threadIdx.x; k < blockIdx.x; k += SCAN_THREADS) before += sums[k];
     block_exclusive_scan(before, &base);
@@ -1529,6 +1533,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_rank_prefix(const uint32_t *bi
         v += n[u];
     }
     uint32_t total, at = base + block_exclusive_scan(v, &total);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) info->bits = base + total;
 #pragma unroll
     for (uint32_t u = 0; u < RANK_PER_THREAD; ++u) {
         if (g0 + u < groups) prefix[g0 + u] = at;
@@ -1536,11 +1541,30 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_rank_prefix(const uint32_t *bi
     }
 }
 
+// row p of the readback from the record in slot s (null arrays are left out)
+struct Rows {
+    double *pos;
+    uint32_t *types, *handles;
+    const double *force_in;
+    double *forces;
+};
+
+__device__ __forceinline__ void write_row(const Grid &cur, const Rows &out, uint32_t p, uint32_t s, uint2 th) {
+    if (out.pos) {
+        const State &st = cur.bins[s];
+        out.pos[3ull * p] = st.x;
+        out.pos[3ull * p + 1] = st.y;
+        out.pos[3ull * p + 2] = st.z;
+    }
+    if (out.types) out.types[p] = tw_type(th.x);
+    if (out.handles) out.handles[p] = th.y;
+    if (out.forces)
+        for (int d = 0; d < 3; ++d) out.forces[3ull * p + d] = out.force_in ? out.force_in[3ull * s + d] : 0.0;
+}
+
 __global__ __launch_bounds__(256) void k_rank_write(Grid cur, uint32_t r, uint32_t cap, uint32_t cell_base,
                                                     uint32_t n_cells, const uint32_t *bits, uint32_t words,
-                                                    const uint32_t *prefix, uint32_t out_cap, double *pos,
-                                                    uint32_t *types, uint32_t *handles, const double *force_in,
-                                                    double *forces) {
+                                                    const uint32_t *prefix, uint32_t out_cap, Rows out) {
     replica_records(cur, cap, cell_base, n_cells, [&](uint32_t s) {
         const uint2 th = *reinterpret_cast<const uint2 *>(&cur.bins[s].tw);
         if ((th.x & TW_DEAD) || tw_replica(th.x) != r) return;
@@ -1548,18 +1572,28 @@ __global__ __launch_bounds__(256) void k_rank_write(Grid cur, uint32_t r, uint32
         if (w >= words) return;
         uint32_t p = prefix[g] + (uint32_t)__popc(bits[w] & ((1u << (th.y & 31u)) - 1u));
         for (uint32_t q = g * RANK_GROUP_WORDS; q < w; ++q) p += (uint32_t)__popc(bits[q]);
-        if (p >= out_cap) return;
-        if (pos) {
-            const State &st = cur.bins[s];
-            pos[3ull * p] = st.x;
-            pos[3ull * p + 1] = st.y;
-            pos[3ull * p + 2] = st.z;
-        }
-        if (types) types[p] = tw_type(th.x);
-        if (handles) handles[p] = th.y;
-        if (forces)
-            for (int d = 0; d < 3; ++d) forces[3ull * p + d] = force_in ? force_in[3ull * s + d] : 0.0;
+        if (p < out_cap) write_row(cur, out, p, s, th);
     });
+}
+
+// the live records in no order: handle in the high word, slot in the low one
+__global__ __launch_bounds__(256) void k_list_live(Grid cur, uint32_t r, uint32_t cap, uint32_t cell_base,
+                                                   uint32_t n_cells, uint32_t list_cap, uint32_t *count,
+                                                   unsigned long long *list) {
+    replica_records(cur, cap, cell_base, n_cells, [&](uint32_t s) {
+        const uint2 th = *reinterpret_cast<const uint2 *>(&cur.bins[s].tw);
+        if ((th.x & TW_DEAD) || tw_replica(th.x) != r) return;
+        const uint32_t p = atomicAdd(count, 1u);
+        if (p < list_cap) list[p] = (unsigned long long)th.y << 32 | s;
+    });
+}
+
+// the rows of the first n listed records
+__global__ __launch_bounds__(256) void k_list_write(Grid cur, const unsigned long long *list, uint32_t n, Rows out) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+    const uint32_t s = (uint32_t)list[p];
+    write_row(cur, out, p, s, *reinterpret_cast<const uint2 *>(&cur.bins[s].tw));
 }
 
 // Live records per replica and type, straight from the cell counters (no work list).  A block takes

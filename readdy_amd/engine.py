@@ -434,6 +434,10 @@ class Engine:
         L.check(self._lib.rdy_synchronize(self._h))
 
     # ---- parity exports ----
+    def set_next_handle(self, r, handle):
+        """The handle that replica r's next new particle takes (not below its counter)."""
+        L.check(self._lib.rdy_set_next_handle(self._h, r, int(handle)))
+
     def neighbor_pairs(self, r, cutoff):
         n = ctypes.c_uint64()
         L.check(self._lib.rdy_neighbor_pairs(self._h, r, cutoff, 0, None, ctypes.byref(n)))

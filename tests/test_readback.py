@@ -1,5 +1,7 @@
 """Counts and particles read back from the device: cells that overflow their bins, blocks of cells that hold one
 replica or many, empty replicas, removed replicas, and many types."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -83,3 +85,69 @@ def test_handles_past_the_expected_range_and_forces_in_step():
     ref = (np.where(dist < 1.0, 10.0 * (dist - 1.0) / dist, 0.0)[:, :, None] * d).sum(1)
     assert np.linalg.norm(f - ref) < 1e-5 * np.linalg.norm(ref)
     e.close()
+
+
+def _converting(n, inert, box, seed=3):
+    """the first `inert` particles stay (type 2), the others change their handle with every reaction (0 <-> 1)"""
+    rng = np.random.default_rng(seed)
+    e = Engine(3, [1.0] * 3, potentials=[(L.POT_HARMONIC_REPULSION, a, b, [10.0, 1.0]) for a in range(3) for b in range(a, 3)],
+               reactions=[dict(kind=L.RX_CONVERSION, educts=[a], products=[1 - a], rate=1e4) for a in (0, 1)],
+               events_per_replica=1024)
+    r = e.add_replica([box] * 3, seed=9, max_particles=n + 16)
+    pos = (rng.random((n, 3)) - 0.5) * box
+    e.set_particles(r, pos, np.where(np.arange(n) < inert, 2, 0).astype(np.uint32))
+    return e, r, pos
+
+
+@pytest.mark.parametrize("inert,shared", [(0, 0), (30, 15)])
+def test_readback_across_the_end_of_the_handle_counter(inert, shared):
+    """60 - inert particles take the last 2^32 handles and the first ones after the counter has wrapped; with inert
+    particles these are still in use, and every particle comes back all the same."""
+    e, r, pos = _converting(60, inert, 8.0)
+    new = 60 - inert
+    e.set_next_handle(r, 2 ** 32 - new // 2)
+    e.react(L.HANDLER_UA, 1.0)
+    want = sorted([*range(inert), *((2 ** 32 - new // 2 + k) % 2 ** 32 for k in range(new))])
+    assert len(want) - len(set(want)) == shared
+    for _ in range(2):
+        p, t, h = e.get_particles(r)
+        assert h.tolist() == want
+        assert np.array_equal(p[np.lexsort(p.T)], pos[np.lexsort(pos.T)])
+        assert np.bincount(t, minlength=3).tolist() == [0, new, inert]
+        e.calculate_forces()
+        f, hf = e.get_forces(r)
+        assert np.array_equal(hf, h) and np.abs(f).sum(1).astype(bool).any()
+    with pytest.raises(L.EngineError):
+        e.set_next_handle(r, 0)
+    e.close()
+
+
+@pytest.mark.parametrize("n,inert,start", [(500, 0, 2 ** 31), (500, 200, 87 * 10 ** 6), (500, 200, 88 * 10 ** 6),
+                                           (20, 0, 2 ** 22), (20, 0, 2 ** 23), (10000, 9500, 2 ** 32 - 10 ** 6),
+                                           (40000, 39500, 10 ** 8), (40000, 39500, 2 ** 32 - 10 ** 6)])
+def test_readback_of_handles_far_apart(n, inert, start):
+    """Both sides of the line between the bitmap and the sorted list, small answers and streamed ones; a shorter
+    array takes the first rows."""
+    e, r, pos = _converting(n, inert, 8.0 if n < 1000 else 40.0)
+    twin, q, _ = _converting(n, inert, 8.0 if n < 1000 else 40.0)  # the same system with its handles close together
+    e.set_next_handle(r, start)
+    for k in range(3):
+        for x in (e, twin):
+            x.react(L.HANDLER_UA, 1.0)
+            x.calculate_forces()
+        p, t, h = e.get_particles(r)
+        assert np.all(np.diff(h.astype(np.int64)) > 0)
+        assert h[inert:].tolist() == [start + k * (n - inert) + j for j in range(n - inert)]
+        # who takes which of the new handles depends on the draws, which follow the handles: compare by position
+        tp, tt, _ = twin.get_particles(q)
+        o, to = np.lexsort(p.T), np.lexsort(tp.T)
+        assert np.array_equal(p[o], tp[to]) and np.array_equal(t[o], tt[to])
+        f, hf = e.get_forces(r)
+        assert np.array_equal(hf, h) and np.array_equal(f[o], twin.get_forces(q)[0][to])
+    cap = min(33, n // 2)
+    some, m = np.zeros(cap, np.uint32), ctypes.c_uint64()
+    L.check(e._lib.rdy_get_particles(e._h, r, cap, None, None, some.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)),
+                                     ctypes.byref(m)))
+    assert m.value == n and np.array_equal(some, h[:cap])
+    e.close()
+    twin.close()
