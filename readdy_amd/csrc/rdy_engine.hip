@@ -47,7 +47,7 @@ struct HostReplica {
     bool has_particles = false;  // particles were uploaded since the replica was added
     uint64_t n_uploaded = 0;     // particles of the last upload
     uint64_t n_live = 0;         // particles of the last upload or readback
-    uint64_t handle_guess = 0;   // handles a readback makes room for (the last one read and some growth)
+    uint64_t handle_guess = 4096;  // handles a readback makes room for (the last one read and some growth; never none)
     uint64_t handle_top = 0;     // and at least: past the highest handle that an earlier one found beyond its room
     ReplicaDev dev{};
 };

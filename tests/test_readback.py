@@ -151,3 +151,23 @@ def test_readback_of_handles_far_apart(n, inert, start):
     assert m.value == n and np.array_equal(some, h[:cap])
     e.close()
     twin.close()
+
+
+def test_readback_of_a_replica_that_never_held_particles():
+    """with room for particles in the caller's arrays; the calls that follow are not affected"""
+    e, ((r, pos, _),) = _engine((50,))
+    e.remove_replica(r)
+    q = e.add_replica([12.0] * 3, seed=1, max_particles=50)
+    h, m = np.zeros(8, np.uint32), ctypes.c_uint64(7)
+    hp = h.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))
+    for _ in range(2):
+        L.check(e._lib.rdy_get_particles(e._h, q, 8, None, None, hp, ctypes.byref(m)))
+        assert m.value == 0
+        e.calculate_forces()
+        m.value = 7
+        L.check(e._lib.rdy_get_forces(e._h, q, 8, None, hp, ctypes.byref(m)))
+        assert m.value == 0
+        e.run(L.HANDLER_UA, 0.01, 2)
+    e.set_particles(q, pos, np.zeros(50, np.uint32))
+    assert np.array_equal(e.get_particles(q)[0], pos)
+    e.close()
