@@ -1195,8 +1195,13 @@ void advance_state(rdy_engine *e) {
     e->cur = e->next();
 }
 
+// Without bricks (every replica has been removed) nothing is stepped, and the state stays: a walk clears the counters
+// of the state after next, so the states must not advance without one.
+bool nothing_to_step(const rdy_engine *e) { return e->bricks_h.empty(); }
+
 // the first walk of a run: the forces of the current state and step 1's move (bonded terms first)
 void launch_prologue(rdy_engine *e, double dt) {
+    if (nothing_to_step(e)) return;
     launch_bonded(e, false);
     launch_walk(e, WALK_PROLOGUE, (int)RDY_HANDLER_NONE, dt);
     advance_state(e);
@@ -1209,6 +1214,7 @@ void launch_epilogue(rdy_engine *e) { launch_topo_begin(e, 0); }
 // yields step t's candidates and, optimistically, step t+1's move; the reactions, the exact
 // corrections and the redone moves follow.  last: the launch's final step copies instead of moving.
 void launch_step(rdy_engine *e, int handler, double dt, int last) {
+    if (nothing_to_step(e)) return;
     const uint32_t nr = std::max<uint32_t>(e->n_reps_used, 1);
     const Grid cur = e->grid(e->cur), nxt = e->grid(e->next());
     const bool topo_rx = topo_reactions_on(e);
@@ -1919,7 +1925,7 @@ int rdy_update_neighbor_list(rdy_engine *e) {
     if (int rb = ensure_bricks(e)) return rb;
     int rc = upload_tables(e, e->tables_dt > 0 ? e->tables_dt : 1.0);
     if (rc) return rc;
-    if (e->bricks_h.empty()) return RDY_OK;  // every replica has been removed
+    if (nothing_to_step(e)) return RDY_OK;
     hipLaunchKernelGGL((k_brick<MODE_REBIN, false>), dim3(n_bricks(e)), dim3(BRICK_THREADS), 0, e->stream,
                        e->grid(e->cur), e->grid(e->next()), e->grid(e->after_next()), e->reps, e->T, e->topo(),
                        (const BrickDev *)e->d_bricks, 0u, e->cap, e->radius, 0.0, (const double *)nullptr,
@@ -2284,7 +2290,7 @@ int rdy_run(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
     if (handler < 0 || handler > RDY_HANDLER_NONE) return set_err(RDY_ERR_INVALID, "unknown reaction handler");
     int rc = upload_tables(e, dt);
     if (rc) return rc;
-    if (n_steps == 0 || e->bricks_h.empty()) return RDY_OK;  // nothing to step
+    if (n_steps == 0 || nothing_to_step(e)) return RDY_OK;
     if ((rc = ensure_step_pools(e))) return rc;
     e->export_valid = false;
     launch_prologue(e, dt);
@@ -2345,7 +2351,7 @@ int rdy_run_graph(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
     if (e->in_session) return set_err(RDY_ERR_STATE, "a run is open: finish it with rdy_run_end");
     int rc = upload_tables(e, dt);
     if (rc) return rc;
-    if (n_steps == 0 || e->bricks_h.empty()) return RDY_OK;  // nothing to step
+    if (n_steps == 0 || nothing_to_step(e)) return RDY_OK;
     if ((rc = ensure_step_pools(e))) return rc;
     e->export_valid = false;
     launch_prologue(e, dt);

@@ -84,3 +84,25 @@ def test_no_replicas_left():
     e.run(L.HANDLER_UA, 0.005, 40, graph=True)
     assert 75 <= e.n_particles(q) <= 300
     e.close()
+
+
+@pytest.mark.parametrize("steps", [1, 2, 3])
+def test_an_open_run_without_replicas(steps):
+    """It steps nothing and leaves every state's counters as they are: the replica admitted next, under the removed
+    one's id and with crowded cells, is as in an engine of its own."""
+    e, (r,) = _engine((700,), bin_capacity=1)
+    e.run(L.HANDLER_UA, 0.005, 5)  # overflow records in both buffers
+    e.remove_replica(r)
+    e.run_begin(L.HANDLER_UA, 0.005, steps)
+    e.run_enqueue(steps)
+    e.run_end()
+    one, _ = _engine((), bin_capacity=1)
+    for x in (e, one):
+        assert _admit(x, 400, 7) == r
+    _same(e, one, [r])
+    for n in (1, 2, 3, 4):
+        for x in (e, one):
+            x.run(L.HANDLER_UA, 0.005, n)
+        _same(e, one, [r])
+    for x in (e, one):
+        x.close()
