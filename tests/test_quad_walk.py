@@ -125,3 +125,34 @@ def test_the_brick_shape_follows_growth_within_a_run(steps):
     assert len(out[0][0]) > 1000
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(lds_states=1), dict(n_types=20)],
+                         ids=["staged", "bin-reading", "more types than are staged"])
+@pytest.mark.parametrize("graph", [False, True])
+def test_a_replica_without_a_handler_reacts_in_no_launch(kw, graph):
+    """Its own handler NONE holds in a launch with reactions, on the bin-reading path too: no reactions, and the
+    trajectory of a launch without any; its neighbour in the launch reacts."""
+    rng = np.random.default_rng(5)
+    rxs = [dict(kind=L.RX_FUSION, educts=[0, 1], products=[2], rate=40.0, educt_distance=0.9),
+           dict(kind=L.RX_CONVERSION, educts=[1], products=[0], rate=40.0)]
+    nt = kw.get("n_types", 3)
+    kw = {k: v for k, v in kw.items() if k != "n_types"}
+    n, steps = 400, 41
+    e, quiet = (Engine(nt, np.ones(nt), potentials=POTS, reactions=rxs, nl_cutoff=1.0, max_replicas=2, **kw)
+                for _ in range(2))
+    ids = []
+    for k in range(2):
+        pos, types = rng.uniform(-4.0, 4.0, (n, 3)), rng.integers(0, 3, n).astype(np.uint32)
+        for x in (e, quiet):
+            r = x.add_replica([8.0] * 3, seed=k, max_particles=2 * n)
+            x.set_particles(r, pos, types)
+        ids.append(r)
+    e.set_handler(ids[0], L.HANDLER_NONE)
+    e.run(L.HANDLER_UA, 1e-3, steps, graph=graph)
+    quiet.run(L.HANDLER_NONE, 1e-3, steps)
+    assert e.reaction_totals(ids[0]).sum() == 0 and e.reaction_totals(ids[1]).sum() > 0
+    for a, b in zip(e.get_particles(ids[0]), quiet.get_particles(ids[0])):
+        assert np.array_equal(a, b)
+    for x in (e, quiet):
+        x.close()
