@@ -780,9 +780,10 @@ struct SearchTables {
     uint32_t *o1;   // [nt] order-1 reactions of the type: first entry of the list | number << 16 (the fused walk)
 };
 
-// reach of a type from the FP32 squared cutoffs of its row, widened like the prefilter
+// reach of a type from the FP32 squared cutoffs of its row, widened like the prefilter; beyond every box, but short
+// of the place of the records that are no neighbours
 __device__ __forceinline__ float reach_of(float max_cut2_f, bool any, float margin) {
-    return any ? sqrtf(max_cut2_f) * (1.0f + 1.0e-6f) + 2.0f * margin : -1.0f;
+    return any ? fminf(sqrtf(max_cut2_f) * (1.0f + 1.0e-6f) + 2.0f * margin, 0.1f * FAR_POS) : -1.0f;
 }
 
 __device__ __forceinline__ ForceTables load_force_tables(char *base, const Tables &T, float margin) {

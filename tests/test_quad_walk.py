@@ -156,3 +156,32 @@ def test_a_replica_without_a_handler_reacts_in_no_launch(kw, graph):
         assert np.array_equal(a, b)
     for x in (e, quiet):
         x.close()
+
+
+@pytest.mark.parametrize("cutoff", [1e9, 3e18, 1e20])
+def test_a_cutoff_far_beyond_the_box(cutoff):
+    """Every pair of an open box interacts; records outside it, and the padding of a quad's last step, stay out."""
+    rng = np.random.default_rng(2)
+    box = 9.0
+    g = np.stack(np.meshgrid(*[np.arange(-3, 3) * 1.4 + 0.7] * 3, indexing="ij"), -1).reshape(-1, 3)
+    pos = g + rng.uniform(-0.15, 0.15, g.shape)
+    pos[::17, 0] += box  # beyond the wall
+    lj = [12, 6, cutoff, 0.0, 1.0, 1.0]
+    e = Engine(1, [1.0], potentials=[(L.POT_LENNARD_JONES, 0, 0, lj)])
+    r = e.add_replica([box] * 3, (0, 0, 0), max_particles=len(pos))
+    e.set_particles(r, pos, np.zeros(len(pos), np.uint32))
+    e.calculate_forces()
+    f, _ = e.get_forces(r)
+    o = po.System(1, [box] * 3, [0, 0, 0], diffusion=[1.0])
+    o.add_pair_potential(po.POT_LENNARD_JONES, 0, 0, lj)
+    o.add_particles(pos, np.zeros(len(pos), np.int32), ids=np.arange(len(pos)))
+    o.nl_setup(cutoff)
+    energy = o.calculate_forces()
+    f_ref = o.particles()[3][np.argsort(o.particles()[2])]
+    assert np.linalg.norm(f - f_ref) <= 1e-5 * np.linalg.norm(f_ref)
+    assert abs(e.energy(r) - energy) <= 1e-5 * abs(energy)
+    assert not f[::17].any()
+    for _ in range(2):
+        e.run(L.HANDLER_NONE, 1e-5, 3)
+    assert np.isfinite(e.get_particles(r)[0]).all()
+    e.close()
