@@ -1507,19 +1507,20 @@ int rdy_replica_add(rdy_engine *e, const rdy_replica_desc *d, uint32_t *replica_
     return RDY_OK;
 }
 
+// empties a replica's cells in the buffer of state s
+static void release_cells(rdy_engine *e, const HostReplica &H, int s) {
+    hipLaunchKernelGGL(k_release_cells, dim3(blocks_for(H.n_cells, 256)), dim3(256), 0, e->stream, e->grid(s),
+                       (uint32_t)H.cell_base, (uint32_t)H.n_cells);
+}
+
 int rdy_replica_remove(rdy_engine *e, uint32_t r) {
     int rc = check_replica(e, r);
     if (rc) return rc;
-    ensure_wl(e);
-    hipLaunchKernelGGL(k_kill_replica, dim3(wl_blocks(e)), dim3(e->block), 0, e->stream, e->grid(e->cur), r,
-                       (uint32_t)e->max_particles);
     uint32_t zero = 0;
     if ((rc = put_field(e, r, offsetof(ReplicaDev, in_use), zero))) return rc;
     if ((rc = put_field(e, r, offsetof(ReplicaDev, active), zero))) return rc;
     HostReplica &H = e->reps_h[r];
-    for (int b = 0; b < N_STATES; ++b)
-        hipLaunchKernelGGL(k_release_cells, dim3(blocks_for(H.n_cells, 256)), dim3(256), 0, e->stream, e->grid(b),
-                           (uint32_t)H.cell_base, (uint32_t)H.n_cells);
+    for (int b = 0; b < N_STATES; ++b) release_cells(e, H, b);
     release_range(e->free_cells, H.cell_base, H.n_cells);
     // the replica's bonded terms and topology slots go with it (a later replica may reuse slot r)
     if ((rc = drop_terms(e, r))) return rc;
@@ -1547,14 +1548,10 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
             seen_free = true;
         }
     }
-    // replace: drop the replica's current particles (a replica that never held any has none to drop,
-    // which keeps filling many fresh replicas linear in their particles)
+    // replace: drop the replica's current particles (a replica that never held any has none to drop).  Their cells are
+    // emptied, so that they take no room in the bins and are not counted where the bricks are fitted.
     HostReplica &H = e->reps_h[r];
-    if (H.has_particles) {
-        ensure_wl(e);
-        hipLaunchKernelGGL(k_kill_replica, dim3(wl_blocks(e)), dim3(e->block), 0, e->stream, e->grid(e->cur), r,
-                           (uint32_t)e->max_particles);
-    }
+    if (H.has_particles) release_cells(e, H, e->cur);
     H.has_particles = true;
     e->fit_dirty = true;
     H.n_uploaded = n;

@@ -1401,18 +1401,7 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_detailed_balance(Grid cur, 
                           (uint32_t *)nullptr, 0u, recs, rec_count, err, D);
 }
 
-// marks every particle of replica r dead in the current buffer
-__global__ void k_kill_replica(Grid cur, uint32_t r, uint32_t max_wl) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t n = *cur.wl_count;
-    n = n < max_wl ? n : max_wl;
-    if (i >= n) return;
-    uint32_t s = cur.wl[i];
-    State st = cur.bins[s];
-    if (tw_replica(st.tw) == r) cur.bins[s].tw = st.tw | TW_DEAD;
-}
-
-// frees the cells of a removed replica in one buffer: counters to zero, overflow records detached
+// frees a replica's cells in one buffer: counters to zero, overflow records dead and detached
 __global__ void k_release_cells(Grid g, uint32_t base, uint32_t n) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) g.counts[base + i] = 0u;
@@ -1420,7 +1409,10 @@ __global__ void k_release_cells(Grid g, uint32_t base, uint32_t n) {
     no = no < g.ovf_cap ? no : g.ovf_cap;
     for (uint32_t o = i; o < no; o += gridDim.x * blockDim.x) {
         uint32_t c = g.ovf_cell[o];
-        if (c >= base && c < base + n) g.ovf_cell[o] = 0xFFFFFFFFu;
+        if (c >= base && c < base + n) {
+            g.ovf_cell[o] = 0xFFFFFFFFu;
+            g.bins[g.nbin + o].tw |= TW_DEAD;
+        }
     }
 }
 

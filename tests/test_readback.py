@@ -171,3 +171,27 @@ def test_readback_of_a_replica_that_never_held_particles():
     e.set_particles(q, pos, np.zeros(50, np.uint32))
     assert np.array_equal(e.get_particles(q)[0], pos)
     e.close()
+
+
+@pytest.mark.parametrize("kw", [{}, dict(bin_capacity=2)])
+def test_an_upload_takes_the_room_of_the_one_it_replaces(kw):
+    """Uploads one after another without a step between them, more than the engine holds at once: each is as the first
+    one of an engine of its own, and the other replica is untouched."""
+    rng = np.random.default_rng(8)
+    e, data = _engine((700, 700), **kw)
+    (r, _, _), (other, opos, _) = data
+    for k in range(16):
+        n = 700 if k % 2 else 100 + k
+        pos, types = (rng.random((n, 3)) - 0.5) * 12.0, rng.integers(0, 3, n).astype(np.uint32)
+        e.set_particles(r, pos, types)
+        p, t, h = e.get_particles(r)
+        assert np.array_equal(p, pos) and np.array_equal(t, types) and np.array_equal(h, np.arange(n))
+        assert np.array_equal(e.count_types(2)[r], np.bincount(types, minlength=3))
+        assert np.array_equal(e.get_particles(other)[0], opos)
+        one, ((q, _, _),) = _engine((700,), **kw)
+        one.set_particles(q, pos, types)
+        for x, i in ((e, r), (one, q)):
+            x.calculate_forces()
+        assert np.array_equal(e.get_forces(r)[0], one.get_forces(q)[0]) and e.energy(r) == one.energy(q)
+        one.close()
+    e.close()
