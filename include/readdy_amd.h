@@ -343,9 +343,11 @@ int rdy_replica_steps_done(rdy_engine *e, uint32_t replica, uint64_t *steps);
 int rdy_replica_set_handler(rdy_engine *e, uint32_t replica, int handler);
 int rdy_synchronize(rdy_engine *e);
 
-/* ---- test exports (parity): the handle counter, the pair set of the cell list, the candidate list ---- */
+/* ---- test exports (parity): the handle counter, the brick shape, the pair set of the cell list, the candidate list ---- */
 /* the handle that the replica's next new particle takes (not below its counter): readback at and past 2^32 */
 int rdy_set_next_handle(rdy_engine *e, uint32_t replica, uint32_t next);
+/* the bricks of the last launch: cells along x, y, z and the records one may stage */
+int rdy_brick_shape(const rdy_engine *e, uint32_t shape[4]);
 /* ordered pairs (handle_i, handle_j) with d2 < cutoff^2 seen by the cell-list traversal */
 int rdy_neighbor_pairs(rdy_engine *e, uint32_t replica, double cutoff, uint64_t cap, uint32_t *pairs,
                        uint64_t *n);

@@ -245,19 +245,6 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
     return v;
 }
 
-// err[STAT_FULL_BRICKS]: the bricks whose halo holds more than max_states records (a wave each)
-__global__ void __launch_bounds__(BRICK_THREADS) k_brick_fill(const uint32_t *counts, const BrickDev *bricks, uint32_t nb,
-                                                              uint32_t max_states, uint32_t *err) {
-    const uint32_t b = blockIdx.x * BRICK_WAVES + threadIdx.x / 64;
-    if (b >= nb) return;
-    const BrickDev &B = bricks[b];
-    const Halo Hs = make_halo(B);
-    uint32_t sum = 0;
-    for (uint32_t c = __lane_id(); c < Hs.nh; c += 64) sum += load_halo_cells(counts, nullptr, B, Hs, c, 1).n[0];
-    sum = wave_inclusive_sum(sum);
-    if (__lane_id() == 63 && sum > max_states) atomicAdd(&err[STAT_FULL_BRICKS], 1u);
-}
-
 // stages buffer g around brick B into LDS; returns the number of staged records, or UINT32_MAX if
 // they do not fit (the caller then takes the slow path).  h: load_halo_cells of the thread's cells
 // (only used when a thread has at most STAGE_CELLS).
@@ -968,6 +955,27 @@ template <class Fn>
 __device__ __forceinline__ void for_each_own_cell(const BrickDev &B, Fn &&fn) {
     const uint32_t ncell = (uint32_t)(B.e[0] * B.e[1] * B.e[2]);
     for (uint32_t ci = threadIdx.x; ci < ncell; ci += BRICK_THREADS) fn(own_cell(B, ci));
+}
+
+// What a staging capacity of max_states records leaves to the bin-reading path, a wave a brick: full[0] bricks, and
+// full[1 + r] records of replica r in them.
+__global__ void __launch_bounds__(BRICK_THREADS) k_brick_fill(const uint32_t *counts, const BrickDev *bricks, uint32_t nb,
+                                                              uint32_t max_states, uint32_t *full) {
+    const uint32_t b = blockIdx.x * BRICK_WAVES + threadIdx.x / 64;
+    if (b >= nb) return;
+    const BrickDev &B = bricks[b];
+    const Halo Hs = make_halo(B);
+    uint32_t sum = 0, own = 0;
+    for (uint32_t c = __lane_id(); c < Hs.nh; c += 64) sum += load_halo_cells(counts, nullptr, B, Hs, c, 1).n[0];
+    sum = (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum(sum), 63);
+    if (sum <= max_states) return;  // wave-uniform
+    const uint32_t n_cells = (uint32_t)(B.e[0] * B.e[1] * B.e[2]);
+    for (uint32_t ci = __lane_id(); ci < n_cells; ci += 64) own += counts[own_cell(B, ci)];
+    own = wave_inclusive_sum(own);
+    if (__lane_id() == 63) {
+        atomicAdd(&full[0], 1u);
+        atomicAdd(&full[1 + B.r], own);
+    }
 }
 
 // visits the records of the brick's own cells straight from the bins: fn(slot, state), a slot a thread (a cell a

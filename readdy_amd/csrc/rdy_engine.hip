@@ -47,6 +47,7 @@ struct HostReplica {
     bool has_particles = false;  // particles were uploaded since the replica was added
     uint64_t n_uploaded = 0;     // particles of the last upload
     uint64_t n_live = 0;         // particles of the last upload or readback
+    double boost = 1.0;          // occupancy that its particles need bricks for, in means: how they have gathered
     uint64_t handle_guess = 4096;  // handles a readback makes room for (the last one read and some growth; never none)
     uint64_t handle_top = 0;     // and at least: past the highest handle that an earlier one found beyond its room
     ReplicaDev dev{};
@@ -136,7 +137,6 @@ struct rdy_engine {
     uint32_t brick[3] = {0, 0, 0};
     uint32_t max_states = 0, max_halo = 0;
     double brick_lam = 0, brick_cells = 0;  // what the shape was chosen for
-    double lam_boost = 1.0;                                  // raised until few bricks outgrow their staging capacity
     uint32_t max_states_cfg = 0, brick_cfg[3] = {0, 0, 0};  // as the caller set them (0: chosen here)
     size_t brick_smem = 0;
     size_t brick_static_lds = 0;
@@ -145,6 +145,7 @@ struct rdy_engine {
     std::vector<BrickDev> bricks_h;
     BrickDev *d_bricks = nullptr;
     size_t d_bricks_cap = 0;
+    uint32_t *d_full = nullptr;  // k_brick_fill's counts
     uint32_t *d_slow = nullptr;  // two lists of bricks left to the bin-reading kernels (forces, search)
     uint32_t n_bricks_ah = 0;    // leading bricks of bricks_h in halo mode on every axis
     bool bricks_dirty = false;   // replicas changed since the last brick upload
@@ -834,24 +835,43 @@ uint32_t n_bricks(const rdy_engine *e) { return (uint32_t)std::max<size_t>(e->br
 
 int configure_bricks(rdy_engine *e, double lam, const int32_t *dims, double scale);
 
+// what the present shape leaves to the bin-reading path (k_brick_fill)
+int count_full(rdy_engine *e, std::vector<uint32_t> &full) {
+    if (!e->d_full) HIP_TRY(dalloc(&e->d_full, 1 + (size_t)e->max_reps));
+    full.resize(1 + (size_t)e->n_reps_used);
+    const uint32_t nb = (uint32_t)e->bricks_h.size();
+    HIP_TRY(hipMemsetAsync(e->d_full, 0, full.size() * sizeof(uint32_t), e->stream));
+    hipLaunchKernelGGL(k_brick_fill, dim3(blocks_for(nb, BRICK_WAVES)), dim3(BRICK_THREADS), 0, e->stream,
+                       (const uint32_t *)e->grid(e->cur).counts, (const BrickDev *)e->d_bricks, nb, e->max_states,
+                       e->d_full);
+    HIP_TRY(hipMemcpyAsync(full.data(), e->d_full, full.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    return RDY_OK;
+}
+
 // The shape follows the particles that were uploaded, not the budget that they may grow to (a budget of four times
 // the particles quartered the bricks: 21.7 us a walk of 2,000 particles, now 19): their mean occupancy, raised until
 // few bricks hold more than their staging capacity (chains gather by their length: a Poisson fill is too narrow).
+// How far it was raised stays with the replicas that needed it: they start from there as long as they keep their
+// particles, and an engine that held a clump is no different from any other.
 int fit_bricks(rdy_engine *e) {
-    double n = 0, cells = 0, largest = 0;
+    double n = 0, cells = 0, largest = 0, boost = 1.0;
     const int32_t *dims = nullptr;
     for (const HostReplica &H : e->reps_h)
         if (H.in_use && H.has_particles && H.n_uploaded) {
             n += (double)H.n_uploaded;
             cells += (double)H.n_cells;
+            boost = std::max(boost, H.boost);
             if ((double)H.n_cells > largest) {
                 largest = (double)H.n_cells;
                 dims = H.dev.dims;
             }
         }
+    std::vector<uint32_t> full;
+    std::vector<char> needed(e->n_reps_used, 0);
     for (;;) {
         // a change of 15% in occupancy, or of two in size, is inside the flat part of the choice
-        const double lam = dims ? n / cells * e->lam_boost : e->brick_lam;
+        const double lam = dims ? n / cells * boost : e->brick_lam;
         if (std::abs(lam / e->brick_lam - 1.0) >= 0.15 || (dims && (cells >= 2.0 * e->brick_cells || cells <= 0.5 * e->brick_cells))) {
             e->brick_cells = cells;
             e->bricks_dirty = true;
@@ -862,20 +882,17 @@ int fit_bricks(rdy_engine *e) {
             if (int rc = upload_bricks(e)) return rc;
             e->bricks_dirty = false;
         }
-        if (!dims || e->max_states_cfg || e->lam_boost > 64.0) return RDY_OK;
-        uint32_t full = 0;
-        HIP_TRY(hipMemsetAsync(e->err + STAT_FULL_BRICKS, 0, sizeof(uint32_t), e->stream));
-        const uint32_t nb = (uint32_t)e->bricks_h.size();
-        hipLaunchKernelGGL(k_brick_fill, dim3(blocks_for(nb, BRICK_WAVES)), dim3(BRICK_THREADS), 0, e->stream,
-                           (const uint32_t *)e->grid(e->cur).counts, (const BrickDev *)e->d_bricks, nb, e->max_states,
-                           e->err);
-        HIP_TRY(hipMemcpyAsync(&full, e->err + STAT_FULL_BRICKS, sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(hipStreamSynchronize(e->stream));
+        if (!dims || e->max_states_cfg || boost > 64.0) break;
+        if (int rc = count_full(e, full)) return rc;
         // a brick left to the bin-reading path costs up to a thousand staged ones (one workgroup a replica takes them:
         // 31 of 2,000 bricks of chains took 20 ms a step), until the others would have to shrink to nothing for it
-        if (full == 0 || (e->lam_boost > 4.0 && full <= nb / 64)) return RDY_OK;
-        e->lam_boost *= 1.25;
+        if (full[0] == 0 || (boost > 4.0 && full[0] <= e->bricks_h.size() / 64)) break;
+        for (size_t r = 0; r < needed.size(); ++r) needed[r] |= full[1 + r] != 0;
+        boost *= 1.25;
     }
+    for (size_t r = 0; r < needed.size(); ++r)
+        if (needed[r]) e->reps_h[r].boost = boost;
+    return RDY_OK;
 }
 
 // brick tables of the current replicas on the device (before any brick launch or graph capture)
@@ -1409,7 +1426,7 @@ int rdy_engine_destroy(rdy_engine *e) {
         if (e->gexec[s]) (void)hipGraphExecDestroy(e->gexec[s]);
         (void)hipFree(e->counts[s]);
     }
-    void *ptrs[] = {e->wl_count, e->ovf_count, e->tile_sums, e->d_bricks, e->d_slow, e->reps, e->events, e->ev_count, e->recs, e->rec_count, e->rx_step, e->rx_total, e->e_bonded, e->virial, e->err,
+    void *ptrs[] = {e->wl_count, e->ovf_count, e->tile_sums, e->d_bricks, e->d_slow, e->d_full, e->reps, e->events, e->ev_count, e->recs, e->rec_count, e->rx_step, e->rx_total, e->e_bonded, e->virial, e->err,
                     e->force_out, e->edits, e->edit_count, e->aff_bits, e->aff_list, e->d_pots, e->d_pidx, e->d_rx, e->d_o1idx, e->d_o1list, e->d_o2list, e->d_o2idx,
                     e->d_rowmax, e->d_dbpots, e->d_dbpidx, e->d_dbtable, e->d_dbkind, e->d_dbpref, e->d_dbradii, e->d_dbcdf, e->d_D, e->d_bd_scale, e->d_flavor, e->topo_of, e->topo_owner, e->treact, e->loc_cur, e->d_sr, e->ttype, e->tev, e->tev_count, e->tfus, e->tfus_count, e->tmrg, e->tmrg_count, e->adj_off, e->adj, e->str_step, e->str_total, e->fb, e->loc, e->scratch, e->d_noise, e->d_terms[0], e->d_terms[1],
                     e->d_terms[2]};
@@ -1526,6 +1543,7 @@ int rdy_replica_remove(rdy_engine *e, uint32_t r) {
     if ((rc = drop_terms(e, r))) return rc;
     release_topo(e, H);
     H.in_use = false;
+    if (H.boost > 1.0) e->fit_dirty = true;  // the others no longer share their bricks with its clumps
     e->version++;
     e->wl_valid = false;
     HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1555,6 +1573,7 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
     H.has_particles = true;
     e->fit_dirty = true;
     H.n_uploaded = n;
+    H.boost = 1.0;
     // the bonded terms name the replaced particles' handles: the caller sets them again
     if ((rc = drop_terms(e, r))) return rc;
     release_topo(e, H);
@@ -2426,6 +2445,13 @@ int rdy_set_next_handle(rdy_engine *e, uint32_t r, uint32_t next) {
     return put_field(e, r, offsetof(ReplicaDev, handle_next), next);
 }
 
+int rdy_brick_shape(const rdy_engine *e, uint32_t shape[4]) {
+    if (!e || !shape) return set_err(RDY_ERR_INVALID, "null argument");
+    for (int a = 0; a < 3; ++a) shape[a] = e->brick[a];
+    shape[3] = e->max_states;
+    return RDY_OK;
+}
+
 int rdy_synchronize(rdy_engine *e) {
     if (!e) return set_err(RDY_ERR_INVALID, "null engine");
     HIP_TRY(hipStreamSynchronize(e->stream));
@@ -2560,7 +2586,7 @@ bool plan_rdf(const rdy_engine *e, uint32_t r, double rmax, const int *rad, uint
     if (!(rmax > 0.0) || !(rmax < 1.0e30) || H.n_cells == 0) return false;
     for (int a = 0; a < 3; ++a)
         if (R.pbc[a] && R.dims[a] < 2 * rad[a] + 2) return false;
-    const double lam = (double)H.n_uploaded / (double)H.n_cells * e->lam_boost;
+    const double lam = (double)H.n_uploaded / (double)H.n_cells * H.boost;
     for (uint32_t edge = 8; edge >= 1; --edge) {
         uint64_t halo = 1, own = 1, bricks = 1;
         for (int a = 0; a < 3; ++a) {

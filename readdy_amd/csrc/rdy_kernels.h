@@ -106,8 +106,8 @@ struct DbTables {
 enum : int { ERR_BIN_OVERFLOW = 0, ERR_EVENT_OVERFLOW = 1, ERR_WL_OVERFLOW = 2, ERR_NONFINITE = 3, ERR_EVENT_LDS = 4,
              ERR_LDS_SEARCH = 5, ERR_LDS_LAYOUT = 6, ERR_EDIT_OVERFLOW = 7, ERR_FORCE_RANGE = 8, ERR_TOPO_RESERVE = 9,
              N_ERR = 10,
-             // no errors: bricks left to the bin-reading path, and those that would be (k_brick_fill)
-             STAT_SLOW_BRICKS = N_ERR, STAT_FULL_BRICKS, N_STAT };
+             // no error: bricks left to the bin-reading path
+             STAT_SLOW_BRICKS = N_ERR, N_STAT };
 
 constexpr int MODE_FORCES = 0;  // forces + energy of the current buffer
 constexpr int MODE_STEP = 1;    // forces, Euler-Maruyama step, re-bin into the other buffer

@@ -434,6 +434,12 @@ class Engine:
         L.check(self._lib.rdy_synchronize(self._h))
 
     # ---- parity exports ----
+    def brick_shape(self):
+        """(cells along x, y, z, staged records) of the bricks of the last launch."""
+        s = np.zeros(4, np.uint32)
+        L.check(self._lib.rdy_brick_shape(self._h, _ptr(s, _u32p)))
+        return tuple(int(v) for v in s)
+
     def set_next_handle(self, r, handle):
         """The handle that replica r's next new particle takes (not below its counter)."""
         L.check(self._lib.rdy_set_next_handle(self._h, r, int(handle)))

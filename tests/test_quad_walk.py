@@ -185,3 +185,44 @@ def test_a_cutoff_far_beyond_the_box(cutoff):
         e.run(L.HANDLER_NONE, 1e-5, 3)
     assert np.isfinite(e.get_particles(r)[0]).all()
     e.close()
+
+
+def _gas_engine(replicas=1):
+    e = Engine(1, [0.5], potentials=POTS[:1], nl_cutoff=1.0, max_replicas=replicas)
+    return e, [e.add_replica([20.0] * 3, seed=k, max_particles=4000) for k in range(replicas)]
+
+
+def _fill(e, r, clump):
+    rng = np.random.default_rng(7)
+    pos = rng.uniform(-9.9, 9.9, (2000, 3))
+    if clump:
+        pos[:1500] = rng.normal(scale=1.2, size=(1500, 3))
+    e.set_particles(r, pos, np.zeros(2000, np.uint32))
+    e.calculate_forces()
+
+
+def test_the_brick_shape_does_not_depend_on_what_the_engine_held():
+    """A clump raises the occupancy that the bricks are made for; a gas uploaded over it, or left alone with the
+    engine, has the bricks of an engine that never held a clump."""
+    e, (r,) = _gas_engine()
+    _fill(e, r, False)
+    gas = e.brick_shape()
+    _fill(e, r, True)
+    clump = e.brick_shape()
+    assert clump != gas
+    _fill(e, r, False)
+    assert e.brick_shape() == gas
+    e.close()
+
+    e, (a, b) = _gas_engine(2)
+    _fill(e, a, False)
+    one = e.brick_shape()
+    _fill(e, b, True)
+    both = e.brick_shape()
+    assert both != one
+    _fill(e, a, False)  # the clump stays, and so do its bricks
+    assert e.brick_shape() == both
+    e.remove_replica(b)
+    e.calculate_forces()
+    assert e.brick_shape() == one
+    e.close()
