@@ -1011,11 +1011,12 @@ struct StepWave : ForceWave {  // per-wave LDS of k_brick_step
 constexpr uint32_t NO_PARTNER = 0xFFFFu;  // an order-1 candidate's entry
 
 // Bricks whose halo does not fit in LDS are listed for a second kernel that reads neighbours
-// straight from the bins.  list: [0] count, [1] blocks of the second kernel done, [2..] bricks.
+// straight from the bins.  list: [0] count, [1] blocks of the second kernel done, [2..] bricks.  err: null where no
+// shape would stage the brick.
 __device__ __forceinline__ void list_slow_brick(uint32_t *list, uint32_t b, uint32_t *err) {
     if (threadIdx.x == 0) {
         list[2 + atomicAdd(&list[0], 1u)] = b;
-        atomicAdd(&err[STAT_SLOW_BRICKS], 1u);
+        if (err) atomicAdd(&err[STAT_SLOW_BRICKS], 1u);
     }
 }
 
@@ -1178,7 +1179,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
         block_add_energy(reps, B.r, e_blk);
         if (virial) block_add_virial(virial, B.r, vir);
     } else {
-        list_slow_brick(slow, bidx, err);
+        list_slow_brick(slow, bidx, nt <= MAX_STAGED_TYPES ? err : nullptr);
     }
 }
 
@@ -1252,7 +1253,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
                                             min(cells_per_thread(Hs), STAGE_CELLS)));
     }
     if (total == 0xFFFFFFFFu) {
-        list_slow_brick(slow, bidx, err);
+        list_slow_brick(slow, bidx, nt <= MAX_STAGED_TYPES ? err : nullptr);
         return;
     }
     const uint32_t r = B.r, step = R.step;

@@ -48,6 +48,7 @@ struct HostReplica {
     uint64_t n_uploaded = 0;     // particles of the last upload
     uint64_t n_live = 0;         // particles of the last upload or readback
     double boost = 1.0;          // occupancy that its particles need bricks for, in means: how they have gathered
+    uint64_t unfit = 0;          // its records that those bricks still leave to the bin-reading path
     uint64_t handle_guess = 4096;  // handles a readback makes room for (the last one read and some growth; never none)
     uint64_t handle_top = 0;     // and at least: past the highest handle that an earlier one found beyond its room
     ReplicaDev dev{};
@@ -149,7 +150,11 @@ struct rdy_engine {
     uint32_t *d_slow = nullptr;  // two lists of bricks left to the bin-reading kernels (forces, search)
     uint32_t n_bricks_ah = 0;    // leading bricks of bricks_h in halo mode on every axis
     bool bricks_dirty = false;   // replicas changed since the last brick upload
-    bool fit_dirty = false;      // particles were uploaded since the shape was last fitted to them
+    bool fit_dirty = false;      // the shape is fitted anew before the next brick launch
+    // looks at the errors that found slow bricks and are let pass before the next fit, and as many as the last time:
+    // a fit that changed nothing is not repeated at every call
+    uint32_t fit_wait = 0, fit_pause = 0;
+    bool fit_slow = false;       // the fit is due to slow bricks
     bool wl_valid = true;  // the current buffer has a work list
     uint64_t cells_hwm = 0;  // end of the highest cell range handed out (the scan covers [0, hwm))
     Event *events = nullptr;
@@ -292,8 +297,10 @@ int check_errors(rdy_engine *e) {
     for (int i = 0; i < N_ERR; ++i) any = any || h[i];
     if (!any && !h[STAT_SLOW_BRICKS]) return RDY_OK;
     HIP_TRY(hipMemsetAsync(e->err, 0, sizeof h, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    if (h[STAT_SLOW_BRICKS]) e->fit_dirty = true;  // the particles have gathered or multiplied
+    if (h[STAT_SLOW_BRICKS] && !e->max_states_cfg) {  // the particles have gathered or multiplied
+        if (e->fit_wait) --e->fit_wait;
+        else e->fit_dirty = e->fit_slow = true;
+    }
     if (!any) return RDY_OK;
     if (h[ERR_FORCE_RANGE])
         return set_err(RDY_ERR_NUMERIC, "a force beyond the fixed-point range (|F| >= 1.68e7 per pair or particle, " +
@@ -856,42 +863,66 @@ int count_full(rdy_engine *e, std::vector<uint32_t> &full) {
 // particles, and an engine that held a clump is no different from any other.
 int fit_bricks(rdy_engine *e) {
     double n = 0, cells = 0, largest = 0, boost = 1.0;
+    uint64_t unfit = 0;
     const int32_t *dims = nullptr;
     for (const HostReplica &H : e->reps_h)
         if (H.in_use && H.has_particles && H.n_uploaded) {
             n += (double)H.n_uploaded;
             cells += (double)H.n_cells;
             boost = std::max(boost, H.boost);
+            unfit += H.unfit;
             if ((double)H.n_cells > largest) {
                 largest = (double)H.n_cells;
                 dims = H.dev.dims;
             }
         }
-    std::vector<uint32_t> full;
-    std::vector<char> needed(e->n_reps_used, 0);
-    for (;;) {
+    auto shape = [&](double raised) -> int {
         // a change of 15% in occupancy, or of two in size, is inside the flat part of the choice
-        const double lam = dims ? n / cells * boost : e->brick_lam;
+        const double lam = dims ? n / cells * raised : e->brick_lam;
         if (std::abs(lam / e->brick_lam - 1.0) >= 0.15 || (dims && (cells >= 2.0 * e->brick_cells || cells <= 0.5 * e->brick_cells))) {
             e->brick_cells = cells;
             e->bricks_dirty = true;
             e->version++;
             if (int rc = configure_bricks(e, lam, dims, cells / largest)) return rc;
         }
-        if (e->bricks_dirty) {
-            if (int rc = upload_bricks(e)) return rc;
-            e->bricks_dirty = false;
-        }
-        if (!dims || e->max_states_cfg || boost > 64.0) break;
+        if (!e->bricks_dirty) return RDY_OK;
+        if (int rc = upload_bricks(e)) return rc;
+        e->bricks_dirty = false;
+        return RDY_OK;
+    };
+    // (with more species than are staged every brick is left to the bin-reading path, whatever its shape)
+    if (!dims || e->max_states_cfg || e->n_types > MAX_STAGED_TYPES) return shape(boost);
+    // A record left to the bin-reading path costs up to a thousand staged ones (one workgroup a replica takes its
+    // bricks: 31 of 2,000 bricks of chains took 20 ms a step), so none is left where a higher occupancy can help, a
+    // 64th of the records from fourfold on, and not much more than an earlier fit had to leave.  Where nothing helps,
+    // the lowest occupancy that leaves about the fewest wins, not the smallest bricks.
+    std::vector<uint32_t> full, least;
+    std::vector<char> needed(e->n_reps_used, 0);
+    double best = boost, now = boost;
+    uint64_t best_left = ~0ull;
+    for (;; now *= 1.25) {
+        if (int rc = shape(now)) return rc;
         if (int rc = count_full(e, full)) return rc;
-        // a brick left to the bin-reading path costs up to a thousand staged ones (one workgroup a replica takes them:
-        // 31 of 2,000 bricks of chains took 20 ms a step), until the others would have to shrink to nothing for it
-        if (full[0] == 0 || (boost > 4.0 && full[0] <= e->bricks_h.size() / 64)) break;
-        for (size_t r = 0; r < needed.size(); ++r) needed[r] |= full[1 + r] != 0;
-        boost *= 1.25;
+        uint64_t left = 0;
+        for (size_t r = 0; r < needed.size(); ++r) {
+            left += full[1 + r];
+            needed[r] |= full[1 + r] != 0;
+        }
+        if (left < best_left - best_left / 8) {
+            best = now;
+            best_left = left;
+            least = full;
+        }
+        if (left <= unfit + unfit / 4 || (now > 4.0 && 64.0 * (double)left <= n) || now > 64.0) break;
+    }
+    if (best != now) {
+        if (int rc = shape(best)) return rc;
     }
     for (size_t r = 0; r < needed.size(); ++r)
-        if (needed[r]) e->reps_h[r].boost = boost;
+        if (needed[r]) {
+            e->reps_h[r].boost = best;
+            e->reps_h[r].unfit = least[1 + r];
+        }
     return RDY_OK;
 }
 
@@ -899,8 +930,11 @@ int fit_bricks(rdy_engine *e) {
 int ensure_bricks(rdy_engine *e) {
     int rc = RDY_OK;
     if (e->fit_dirty) {
+        const uint64_t before = e->version;
         if ((rc = fit_bricks(e))) return rc;
-        e->fit_dirty = false;
+        e->fit_pause = e->fit_slow && e->version == before ? std::min(2 * e->fit_pause + 1, 63u) : 0u;
+        e->fit_wait = e->fit_pause;
+        e->fit_dirty = e->fit_slow = false;
     }
     if (!e->bricks_dirty) return RDY_OK;
     rc = upload_bricks(e);
@@ -1572,8 +1606,11 @@ int rdy_set_particles(rdy_engine *e, uint32_t r, uint64_t n, const double *pos, 
     if (H.has_particles) release_cells(e, H, e->cur);
     H.has_particles = true;
     e->fit_dirty = true;
+    e->fit_slow = false;
+    e->fit_wait = e->fit_pause = 0;
     H.n_uploaded = n;
     H.boost = 1.0;
+    H.unfit = 0;
     // the bonded terms name the replaced particles' handles: the caller sets them again
     if ((rc = drop_terms(e, r))) return rc;
     release_topo(e, H);

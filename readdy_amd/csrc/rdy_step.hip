@@ -278,7 +278,7 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(5
             total = stage_brick(a.cur, B, geo, F, a.cap, m, a.max_states, Hs, hcn);
         }
         if (total == 0xFFFFFFFFu) {
-            list_slow_brick(a.slow, bidx, a.err);
+            list_slow_brick(a.slow, bidx, staged_types ? a.err : nullptr);
             return;
         }
         wc = make_walk(B, geo, Hs, a.radius);

@@ -226,3 +226,21 @@ def test_the_brick_shape_does_not_depend_on_what_the_engine_held():
     e.calculate_forces()
     assert e.brick_shape() == one
     e.close()
+
+
+def test_records_that_no_bricks_stage_do_not_shrink_the_others():
+    """8000 of 24000 particles in 27 cells, more than a block's LDS holds around any of them: the rest keeps the bricks
+    of a gas of as many particles, in every later call too."""
+    rng = np.random.default_rng(4)
+    shapes = []
+    for clump in (0, 8000):
+        e = Engine(1, [0.0], potentials=[(L.POT_HARMONIC_REPULSION, 0, 0, [1e-3, 1.0])], nl_cutoff=1.0, bin_capacity=480)
+        r = e.add_replica([40.0] * 3, max_particles=24000)
+        pos = rng.uniform(-20.0, 20.0, (24000, 3))
+        pos[:clump] = rng.uniform(0.0, 3.0, (clump, 3))
+        e.set_particles(r, pos, np.zeros(24000, np.uint32))
+        for _ in range(3):
+            e.calculate_forces()
+            shapes.append(e.brick_shape())
+        e.close()
+    assert len(set(shapes)) == 1
