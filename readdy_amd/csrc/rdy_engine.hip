@@ -1184,6 +1184,9 @@ void ensure_wl(rdy_engine *e) {
 }
 
 constexpr uint64_t GRAPH_MIN_STEPS = 32;
+// A longer run looks after its errors, and its bricks, every so many steps: about 20 us, where a step takes 30 and
+// more, and some 15 ms once its bricks have been outgrown (3,000 particles that multiplied in 125 cells).
+constexpr uint64_t LOOK_STEPS = 256;
 
 // workgroups of the fix-up kernels (their waves stride over the change lists): 1024 waves, one per changed record
 // of every step measured (about 230 at 1,000,000 particles), since a launch of 1024 workgroups takes longer to
@@ -2351,8 +2354,10 @@ int rdy_run(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
         launch_step(e, handler, dt, s + 1 == n_steps);
         if (e->prof && e->prof_used == e->prof_ev.size())
             if ((rc = flush_prof(e))) return rc;
-        if ((s & 1023) == 1023)
+        if (s % LOOK_STEPS == LOOK_STEPS - 1 && s + 1 < n_steps) {
             if ((rc = check_errors(e))) return rc;
+            if ((rc = ensure_bricks(e))) return rc;
+        }
     }
     launch_epilogue(e);
     if ((rc = flush_prof(e))) return rc;
@@ -2413,7 +2418,6 @@ int rdy_run_graph(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
     // every step but the last from the graph of N_STATES steps, which starts and ends in the same state (the last
     // step copies instead of moving).  A capture costs about as much host time as GRAPH_MIN_STEPS launched steps.
     uint64_t generic = n_steps - 1;
-    uint32_t stretch = 64;  // launches between two looks at the errors
     while (generic >= N_STATES) {
         if (e->g_version != e->version || e->g_handler != handler || e->g_dt != dt) {
             for (hipGraphExec_t &g : e->gexec) {
@@ -2437,12 +2441,11 @@ int rdy_run_graph(rdy_engine *e, int handler, double dt, uint64_t n_steps) {
             (void)hipGraphDestroy(g);
             HIP_TRY(ge);
         }
-        for (uint32_t p = 0; p < stretch && generic >= N_STATES; ++p, generic -= N_STATES)
+        for (uint64_t p = 0; p < LOOK_STEPS / N_STATES && generic >= N_STATES; ++p, generic -= N_STATES)
             HIP_TRY(hipGraphLaunch(exec, e->stream));
-        if (generic >= N_STATES) {  // a longer run looks after its errors, and its bricks, on the way
+        if (generic >= N_STATES) {
             if ((rc = check_errors(e))) return rc;
             if ((rc = ensure_bricks(e))) return rc;
-            stretch = 256;
         }
     }
     for (uint64_t k = 0; k < generic; ++k) launch_step(e, handler, dt, 0);

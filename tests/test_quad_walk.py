@@ -109,20 +109,26 @@ def test_the_brick_shape_follows_the_particles():
     e.close()
 
 
-@pytest.mark.parametrize("steps", [1500, 2600])
-def test_the_brick_shape_follows_growth_within_a_run(steps):
-    """30 particles that multiply to thousands in the middle of the box in one run: the bricks are fitted on the way."""
+@pytest.mark.parametrize("steps", [300, 600])
+@pytest.mark.parametrize("graph", [False, True])
+def test_the_brick_shape_follows_growth_within_a_run(steps, graph):
+    """125 particles that multiply to thousands in one run: the bricks are fitted on the way (after 256 steps or 512),
+    and the run goes on in them as in bricks of a given shape."""
     out = []
     for kw in (dict(), dict(brick=(3, 3, 3))):
-        rxs = [dict(kind=L.RX_FISSION, educts=[0], products=[0, 0], rate=1.9, product_distance=0.5)]
-        e = Engine(1, [0.5], potentials=POTS[:1], reactions=rxs, nl_cutoff=1.0, bin_capacity=128, **kw)
-        r = e.add_replica([12.0] * 3, (1, 1, 1), seed=2, max_particles=20000)
-        pos = np.random.default_rng(1).uniform(-2.0, 2.0, (30, 3))
-        e.set_particles(r, pos, np.zeros(30, np.uint32))
-        e.run(L.HANDLER_UA, 1.6e-3 * 1500 / steps, steps)
+        rxs = [dict(kind=L.RX_FISSION, educts=[0], products=[0, 0], rate=5.5, product_distance=0.5)]
+        e = Engine(1, [0.5], potentials=[(L.POT_HARMONIC_REPULSION, 0, 0, [0.1, 1.0])], reactions=rxs, nl_cutoff=1.0,
+                   bin_capacity=64, **kw)
+        r = e.add_replica([5.0] * 3, (1, 1, 1), seed=2, max_particles=20000)
+        pos = np.random.default_rng(1).uniform(-2.5, 2.5, (125, 3))
+        e.set_particles(r, pos, np.zeros(125, np.uint32))
+        e.calculate_forces()
+        before = e.brick_shape()
+        e.run(L.HANDLER_UA, 2e-3 * 300 / steps, steps, graph=graph)
+        assert kw or e.brick_shape() != before  # (a fit that is due at the end of a run waits for the next launch)
         out.append((*e.get_particles(r), e.energy(r), e.reaction_totals(r)))
         e.close()
-    assert len(out[0][0]) > 1000
+    assert len(out[0][0]) > 2000
     for a, b in zip(*out):
         assert np.array_equal(a, b)
 
