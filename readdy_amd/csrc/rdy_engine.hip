@@ -2626,7 +2626,8 @@ bool plan_rdf(const rdy_engine *e, uint32_t r, double rmax, const int *rad, uint
     if (!(rmax > 0.0) || !(rmax < 1.0e30) || H.n_cells == 0) return false;
     for (int a = 0; a < 3; ++a)
         if (R.pbc[a] && R.dims[a] < 2 * rad[a] + 2) return false;
-    const double lam = (double)H.n_uploaded / (double)H.n_cells * H.boost;
+    // (as the walk's bricks had to be raised for gathered particles, and no less than the particles last counted)
+    const double lam = std::max((double)H.n_uploaded * H.boost, (double)H.n_live) / (double)H.n_cells;
     for (uint32_t edge = 8; edge >= 1; --edge) {
         uint64_t halo = 1, own = 1, bricks = 1;
         for (int a = 0; a < 3; ++a) {
@@ -2745,6 +2746,10 @@ int rdy_rdf_counts(rdy_engine *e, uint32_t r, const double *borders, uint32_t n_
     HIP_TRY(hipMemcpyAsync(counts, d_c, 8 * nbins, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipMemcpyAsync(n_from, d_n, 8, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
+    if (left[1]) {  // bricks too full: the next call's are made for as many particles as there are now
+        uint64_t live = 0;
+        if ((rc = gather(e, r, 0, {}, &live))) return rc;
+    }
     return check_errors(e);
 }
 
