@@ -1487,7 +1487,7 @@ int rdy_replica_footprint(const rdy_engine *e, const rdy_replica_desc *d, uint64
     double cs[3];
     cell_dims(e, d->box, dims, cs);
     uint64_t cells = (uint64_t)dims[0] * dims[1] * dims[2];
-    *bytes = cells * (2ull * e->cap * sizeof(State) + 2ull * sizeof(uint32_t)) + d->max_particles * 2ull * 4ull +
+    *bytes = cells * (2ull * e->cap * sizeof(State) + N_STATES * sizeof(uint32_t)) + d->max_particles * 2ull * 4ull +
              (uint64_t)e->ev_per_rep * sizeof(Event);
     return RDY_OK;
 }

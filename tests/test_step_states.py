@@ -106,3 +106,10 @@ def test_an_open_run_without_replicas(steps):
         _same(e, one, [r])
     for x in (e, one):
         x.close()
+
+
+def test_a_replicas_footprint_counts_every_state():
+    """A cell takes its records in two buffers and a counter in each of the four states."""
+    e, _ = _engine((100,), bin_capacity=8)
+    assert e.footprint([20.0] * 3, 50) - e.footprint([10.0] * 3, 50) == (8000 - 1000) * (2 * 8 * 32 + 4 * 4)
+    e.close()
