@@ -402,7 +402,6 @@ struct WalkCtx {
     uint32_t whole;
     int32_t dims[3];
     int radius;
-    uint32_t n;         // 2r + 1
     int32_t h[3];       // halo widths
     float cs[3], inv_cs[3];
 };
@@ -415,7 +414,6 @@ __device__ __forceinline__ WalkCtx make_walk(const BrickDev &B, const RepGeom &g
     c.dims[1] = geo.dims[1];
     c.dims[2] = geo.dims[2];
     c.radius = radius;
-    c.n = 2u * (uint32_t)radius + 1u;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         c.h[a] = B.h[a];
@@ -425,81 +423,38 @@ __device__ __forceinline__ WalkCtx make_walk(const BrickDev &B, const RepGeom &g
     return c;
 }
 
-// general case: per axis halo mode (offsets -r..r), whole-axis mode with all cells (dims <= 2r) or
-// whole-axis mode with wrapped offsets; z as one run unless wrapped
+// general case: per axis the offsets -r..r (halo mode) or all cells (whole-axis mode); z is one run
 struct Walk {
-    int nx, ny, nzr;
-    int bx, by, bz;  // base coordinates
-    int mx, my, mz;  // axis modes: 0 halo, 1 whole (all cells), 2 whole (wrapped offsets)
-    int Dz;
-    int ia, ib, iz;
+    int nx, ny, nz;  // cells an axis
+    int bx, by, bz;  // the first ones
+    int ia, ib;
     uint32_t q, qe;
 
-    __device__ __forceinline__ static void axis_mode(bool whole, int D, int radius, int hcoord, int &n, int &base,
-                                                     int &mode) {
-        if (!whole) {
-            n = 2 * radius + 1;
-            base = hcoord - radius;
-            mode = 0;
-        } else if (D <= 2 * radius) {
-            n = D;
-            base = 0;
-            mode = 1;
-        } else {
-            n = 2 * radius + 1;
-            base = hcoord - radius;
-            mode = 2;
-        }
-    }
-    __device__ __forceinline__ static int elem(int k, int base, int mode, int D) {
-        if (mode != 2) return base + k;
-        int v = base + k;  // |overhang| <= r < D
-        return v < 0 ? v + D : (v >= D ? v - D : v);
+    __device__ __forceinline__ static void axis(const WalkCtx &c, int a, uint32_t hcoord, int &n, int &base) {
+        const bool whole = c.whole >> a & 1u;
+        n = whole ? c.dims[a] : 2 * c.radius + 1;
+        base = whole ? 0 : (int)hcoord - c.radius;
     }
     __device__ __forceinline__ void range(const WalkCtx &c, const uint16_t *hs) {
-        const int x = elem(ia, bx, mx, c.dims[0]);
-        const int y = elem(ib, by, my, c.dims[1]);
-        const uint32_t row = ((uint32_t)x * c.Hs.H1 + (uint32_t)y) * c.Hs.H2;
-        int z0, z1;
-        if (mz == 2) {
-            z0 = elem(iz, bz, 2, c.dims[2]);
-            z1 = z0 + 1;
-        } else {
-            z0 = bz;
-            z1 = bz + Dz;
-        }
-        q = hs[row + (uint32_t)z0];
-        qe = hs[row + (uint32_t)z1];
+        const uint32_t z0 = ((uint32_t)(bx + ia) * c.Hs.H1 + (uint32_t)(by + ib)) * c.Hs.H2 + (uint32_t)bz;
+        q = hs[z0];
+        qe = hs[z0 + (uint32_t)nz];
     }
     __device__ __forceinline__ bool begin(const WalkCtx &c, uint32_t hc, const uint16_t *hs) {
         uint32_t hx, hy, hz;
         c.Hs.decode(hc, hx, hy, hz);
-        axis_mode(c.whole & 1u, c.dims[0], c.radius, (int)hx, nx, bx, mx);
-        axis_mode(c.whole & 2u, c.dims[1], c.radius, (int)hy, ny, by, my);
-        int nz;
-        axis_mode(c.whole & 4u, c.dims[2], c.radius, (int)hz, nz, bz, mz);
-        if (mz == 0) {  // one contiguous z-run of 2r+1 cells
-            nzr = 1;
-            Dz = 2 * c.radius + 1;
-        } else if (mz == 1) {  // the whole axis
-            nzr = 1;
-            Dz = c.dims[2];
-        } else {
-            nzr = nz;
-            Dz = 1;
-        }
-        ia = ib = iz = 0;
+        axis(c, 0, hx, nx, bx);
+        axis(c, 1, hy, ny, by);
+        axis(c, 2, hz, nz, bz);
+        ia = ib = 0;
         range(c, hs);
         return q < qe || advance(c, hs);
     }
     __device__ __forceinline__ bool advance(const WalkCtx &c, const uint16_t *hs) {
         do {
-            if (++iz >= nzr) {
-                iz = 0;
-                if (++ib >= ny) {
-                    ib = 0;
-                    if (++ia >= nx) return false;
-                }
+            if (++ib >= ny) {
+                ib = 0;
+                if (++ia >= nx) return false;
             }
             range(c, hs);
         } while (q >= qe);
