@@ -722,10 +722,9 @@ struct SearchTables {
     uint32_t *o1;   // [nt] order-1 reactions of the type: first entry of the list | number << 16 (the fused walk)
 };
 
-// reach of a type from the FP32 squared cutoffs of its row, widened like the prefilter; beyond every box, but short
-// of the place of the records that are no neighbours
+// reach of a type from the FP32 squared cutoffs of its row, widened like the prefilter
 __device__ __forceinline__ float reach_of(float max_cut2_f, bool any, float margin) {
-    return any ? fminf(sqrtf(max_cut2_f) * (1.0f + 1.0e-6f) + 2.0f * margin, 0.1f * FAR_POS) : -1.0f;
+    return any ? sqrtf(max_cut2_f) * (1.0f + 1.0e-6f) + 2.0f * margin : -1.0f;
 }
 
 __device__ __forceinline__ ForceTables load_force_tables(char *base, const Tables &T, float margin) {
@@ -966,12 +965,11 @@ struct StepWave : ForceWave {  // per-wave LDS of k_brick_step
 constexpr uint32_t NO_PARTNER = 0xFFFFu;  // an order-1 candidate's entry
 
 // Bricks whose halo does not fit in LDS are listed for a second kernel that reads neighbours
-// straight from the bins.  list: [0] count, [1] blocks of the second kernel done, [2..] bricks.  err: null where no
-// shape would stage the brick.
+// straight from the bins.  list: [0] count, [1] blocks of the second kernel done, [2..] bricks.
 __device__ __forceinline__ void list_slow_brick(uint32_t *list, uint32_t b, uint32_t *err) {
     if (threadIdx.x == 0) {
         list[2 + atomicAdd(&list[0], 1u)] = b;
-        if (err) atomicAdd(&err[STAT_SLOW_BRICKS], 1u);
+        atomicAdd(&err[STAT_SLOW_BRICKS], 1u);
     }
 }
 
@@ -1134,7 +1132,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick(Grid cur, Grid nxt, Gri
         block_add_energy(reps, B.r, e_blk);
         if (virial) block_add_virial(virial, B.r, vir);
     } else {
-        list_slow_brick(slow, bidx, nt <= MAX_STAGED_TYPES ? err : nullptr);
+        list_slow_brick(slow, bidx, err);
     }
 }
 
@@ -1208,7 +1206,7 @@ __global__ __launch_bounds__(BRICK_THREADS) void k_brick_search(Grid cur, Replic
                                             min(cells_per_thread(Hs), STAGE_CELLS)));
     }
     if (total == 0xFFFFFFFFu) {
-        list_slow_brick(slow, bidx, nt <= MAX_STAGED_TYPES ? err : nullptr);
+        list_slow_brick(slow, bidx, err);
         return;
     }
     const uint32_t r = B.r, step = R.step;

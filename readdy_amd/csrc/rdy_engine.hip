@@ -295,12 +295,13 @@ int check_errors(rdy_engine *e) {
     HIP_TRY(hipStreamSynchronize(e->stream));
     bool any = false;
     for (int i = 0; i < N_ERR; ++i) any = any || h[i];
-    if (!any && !h[STAT_SLOW_BRICKS]) return RDY_OK;
+    // slow bricks (the particles have gathered or multiplied) ask for a fit, where another shape can help: with more
+    // species than are staged, or a given staging capacity, none can
+    const bool slow = h[STAT_SLOW_BRICKS] && !e->max_states_cfg && e->n_types <= MAX_STAGED_TYPES;
+    if (!any && !slow) return RDY_OK;
     HIP_TRY(hipMemsetAsync(e->err, 0, sizeof h, e->stream));
-    if (h[STAT_SLOW_BRICKS] && !e->max_states_cfg) {  // the particles have gathered or multiplied
-        if (e->fit_wait) --e->fit_wait;
-        else e->fit_dirty = e->fit_slow = true;
-    }
+    if (slow && e->fit_wait) --e->fit_wait;
+    else if (slow) e->fit_dirty = e->fit_slow = true;
     if (!any) return RDY_OK;
     if (h[ERR_FORCE_RANGE])
         return set_err(RDY_ERR_NUMERIC, "a force beyond the fixed-point range (|F| >= 1.68e7 per pair or particle, " +
@@ -332,6 +333,9 @@ int upload_tables(rdy_engine *e, double dt) {
     if (e->tables_dt == dt && e->d_rx) return RDY_OK;
     HIP_TRY(hipStreamSynchronize(e->stream));  // old tables may still be read by queued kernels
     const uint32_t nt = e->n_types;
+    // squared cutoffs for the FP32 prefilters: beyond every box, but short of where the records that are no neighbours
+    // lie (the exact gates use the cutoffs themselves)
+    auto square_f = [](double c2) { return (float)std::min(c2, 0.01 * (double)FAR_SQ); };
     // pair potentials: symmetric type-pair lists in registration order (PotentialRegistry.h:65-70)
     std::vector<std::vector<uint32_t>> lists((size_t)nt * nt);
     std::vector<PotDev> pots;
@@ -395,7 +399,7 @@ int upload_tables(rdy_engine *e, double dt) {
             flat.push_back(pots[id]);
             pidx[k].maxcut2 = std::max(pidx[k].maxcut2, pots[id].cut2);
         }
-        pidx[k].maxcut2_f = (float)pidx[k].maxcut2;
+        pidx[k].maxcut2_f = square_f(pidx[k].maxcut2);
     }
     if (flat.size() > 65535) return set_err(RDY_ERR_INVALID, "too many pair potentials");
     // reactions
@@ -441,7 +445,7 @@ int upload_tables(rdy_engine *e, double dt) {
         o2idx[k].count = (uint16_t)o2[k].size();
         double m2 = 0.0;
         for (uint32_t rx : o2[k]) m2 = std::max(m2, e->rx_h[rx].educt_dist2);
-        o2idx[k].maxr2_f = (float)m2;
+        o2idx[k].maxr2_f = square_f(m2);
         has_o2 = has_o2 || !o2[k].empty();
         o2list.insert(o2list.end(), o2[k].begin(), o2[k].end());
     }

@@ -278,7 +278,7 @@ __global__ __launch_bounds__(BRICK_THREADS) __attribute__((amdgpu_waves_per_eu(5
             total = stage_brick(a.cur, B, geo, F, a.cap, m, a.max_states, Hs, hcn);
         }
         if (total == 0xFFFFFFFFu) {
-            list_slow_brick(a.slow, bidx, staged_types ? a.err : nullptr);
+            list_slow_brick(a.slow, bidx, a.err);
             return;
         }
         wc = make_walk(B, geo, Hs, a.radius);
@@ -524,13 +524,12 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
         const ReplicaDev &R = reps[B.r];
         const RepGeom geo = load_geom(R);
         const bool integ = R.integ != 0u;
-        const bool search = R.active && replica_handler(R, handler) <= 1;  // as the staged walk's rx_on
         const uint32_t step_next = R.step + 1u;
         for_each_own_record(cur, B, cap, [&](uint32_t s, const State &me) {
             if (me.tw & TW_DEAD) return;
             long long fx = 0, fy = 0, fz = 0, e = 0;
             if (!(me.tw & TW_OUTSIDE)) global_forces(cur, geo, cap, radius, T, s, me, fx, fy, fz, e);
-            if (search) search_one(cur, reps, T, cap, radius, 0, events, ev_count, nullptr, 0, s, me, err);
+            if (R.active && replica_handler(R, handler) <= 1) search_one(cur, reps, T, cap, radius, 0, events, ev_count, nullptr, 0, s, me, err);
             advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, integ, me, fx, fy, fz, err);
         });
     }
