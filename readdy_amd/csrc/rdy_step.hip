@@ -529,7 +529,8 @@ __global__ __launch_bounds__(RESOLVE_THREADS) void k_resolve_step(Grid cur, Grid
             if (me.tw & TW_DEAD) return;
             long long fx = 0, fy = 0, fz = 0, e = 0;
             if (!(me.tw & TW_OUTSIDE)) global_forces(cur, geo, cap, radius, T, s, me, fx, fy, fz, e);
-            if (R.active && replica_handler(R, handler) <= 1) search_one(cur, reps, T, cap, radius, 0, events, ev_count, nullptr, 0, s, me, err);
+            if (R.active && replica_handler(R, handler) <= 1)  // as the staged walk's rx_on
+                search_one(cur, reps, T, cap, radius, 0, events, ev_count, nullptr, 0, s, me, err);
             advance_particle(nxt, R, geo, T, topo, cap, dt, step_next, integ, me, fx, fy, fz, err);
         });
     }

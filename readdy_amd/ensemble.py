@@ -179,9 +179,8 @@ class Plain:
 
 
 def half_round_brick(cell):
-    """A cube of cells whose expected particles fill about half of a brick's 256 lanes (two waves): the
-    engine's own choice fills one round of lanes, and with many small replicas the smaller brick can
-    win (fewer waves per block, so a block's slowest wave holds its LDS for less time)."""
+    """A cube of cells whose expected particles fill about half of a brick's 256 lanes (two waves): with many small
+    replicas it can beat the engine's own choice (a block's slowest wave holds its LDS for less time)."""
     lam = DENSITY * cell ** 3
     e = int(round((128.0 / lam) ** (1.0 / 3.0)))
     e = max(2, min(16, e))
@@ -189,7 +188,7 @@ def half_round_brick(cell):
 
 
 def brick_candidates(cell):
-    """The engine's one-round choice, the half-round cube and the two shapes next to it: how bricks tile
+    """The engine's own choice, the half-round cube and the two shapes next to it: how bricks tile
     the uneven replica grids (the last brick of an axis is clipped) changes the best shape by a cell."""
     e = half_round_brick(cell)[0]
     return [(0, 0, 0), (e, e, e), (e, e, e + 1), (e + 1, e + 1, e + 1)]

@@ -1,8 +1,7 @@
 """Autotuning of one system's launch geometry.
 
-The engine's own brick chooser is a cost model (`choose_brick`: the expected own particles of a brick fill
-one round of a workgroup's lanes, among those shapes the fewest staged cells).  `autotune_system` checks it
-on the system itself: it times short graph-replayed runs of candidate configurations (cell size as
+The engine's own brick chooser is a cost model (`choose_brick`: the shape of least modelled time for the mean
+occupancy, fitted to measured walks).  `autotune_system` checks it on the system itself: it times short graph-replayed runs of candidate configurations (cell size as
 cutoff / cell_radius, brick shape in cells) and returns the fastest.  Every candidate gives the same
 trajectory bit for bit (fixed-point force sums, draws keyed by handle and step), so a choice changes the
 speed only; `test_autotune_candidates_give_one_trajectory` checks that.
@@ -13,9 +12,9 @@ import numpy as np
 
 
 def brick_candidates(density, cutoff, lanes=256):
-    """Cubes around the one-round brick (about `lanes` expected own particles) and the two-round cube, at
-    cells of the cutoff; the engine's own choice ((0, 0, 0)); and cells of half the cutoff with the engine's
-    brick (the 125-cell stencil of cell_radius 2)."""
+    """Cubes of about `lanes` and 2 `lanes` expected own particles and their neighbours, at cells of the cutoff; the
+    engine's own choice ((0, 0, 0)); and cells of half the cutoff with the engine's brick (the 125-cell stencil of
+    cell_radius 2)."""
     lam = density * cutoff ** 3  # expected particles per cell
     e1 = max(2, int(round((lanes / lam) ** (1.0 / 3.0))))
     e2 = max(2, int(round((2 * lanes / lam) ** (1.0 / 3.0))))
